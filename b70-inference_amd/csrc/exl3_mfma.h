@@ -166,4 +166,54 @@ __device__ __forceinline__ h8_t frag_decode_k(const uint32_t* __restrict__ tw, i
     }
 }
 
+// sum over b < n of q[b] (n >= 1), in order, with the loads issued 16 at a time (unconditionally: indices clamped to
+// n - 1, so no branch splits a batch into separate round trips)
+__device__ __forceinline__ float sum_ordered(const float* q, int n) {
+    float v = 0.f;
+    for (int b0 = 0; b0 < n; b0 += 16) {
+        float t[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t[i] = ldg(q + (b0 + i < n ? b0 + i : n - 1));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v += b0 + i < n ? t[i] : 0.f;
+    }
+    return v;
+}
+
+// ------------------------------------------------------------------------------------------------ dense linear
+// A of a block of cnt rows (cnt * k / 8 units of 16 bytes, where the block's rows would lie): the unit holding k unit h
+// (half of a 16-k block, see exl3_wide.h) of 16-k block kk of its row r.
+__host__ __device__ __forceinline__ constexpr int64_t block_unit(int cnt, int kk, int h, int r) {
+    return (int64_t)(2 * kk + h) * cnt + r;
+}
+
+struct LinArgs {
+    const _Float16* xh;                              // [S][m][k]
+    const float* xsum;                               // [S][m][k / 128]
+    const int32_t* sonb;                             // shard of each 128-column block (S > 1), else null
+    int S;
+    const uint32_t* tr;
+    const uint16_t* svh;
+    void* out;
+    int64_t out_ld;
+    float* part;                                     // [P][m][n] when P > 1
+    int m, k, n, nblk;
+    int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits, 128-blocks per split
+    int f32;
+};
+
+typedef void (*lin_fn)(LinArgs);
+
+__device__ __forceinline__ void linear_store(const LinArgs& a, int row, int col, float v0, float v1) {
+    if (a.f32) {
+        float* o = reinterpret_cast<float*>(a.out) + (int64_t)row * a.out_ld + col;
+        o[0] = v0;
+        o[64] = v1;
+    } else {
+        uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + (int64_t)row * a.out_ld + col;
+        o[0] = f2h(v0);
+        o[64] = f2h(v1);
+    }
+}
+
 }  // namespace exl3

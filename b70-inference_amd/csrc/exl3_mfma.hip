@@ -520,20 +520,6 @@ __device__ __forceinline__ void gateup_epilogue(const MoeArgs& a, const ItemDesc
     }
 }
 
-// sum over b < n of q[b] (n >= 1), in order, with the loads issued 16 at a time (unconditionally: indices clamped to
-// n - 1, so no branch splits a batch into separate round trips)
-__device__ __forceinline__ float sum_ordered(const float* q, int n) {
-    float v = 0.f;
-    for (int b0 = 0; b0 < n; b0 += 16) {
-        float t[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) t[i] = ldg(q + (b0 + i < n ? b0 + i : n - 1));
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v += b0 + i < n ? t[i] : 0.f;
-    }
-    return v;
-}
-
 // One instance per row class (RGA row groups of 16): workgroup (list index, column block); indices past the class's
 // block count exit at once.
 template <int K, int RGA, bool PL = false>
@@ -1075,32 +1061,20 @@ __global__ __launch_bounds__(256, EXL3_MIX_OCC(RGA)) void down_mix_kernel(MoeArg
 
 // ------------------------------------------------------------------------------------------------ dense linear
 // exl3_gemm for more rows than the GEMV takes per pass: y = Hn(Hk(x * suh) @ W_hat) * svh with the trellis decoded
-// straight into MFMA B fragments once per row block (up to 64 rows), as in the reference's large-M linear
+// straight into MFMA B fragments once per row block, as in the reference's large-M linear
 // (glm/xpu/csrc/exl3_ops.sycl:643-757), which reconstructs 16384-column fp16 slices and runs a GEMM instead.
 //   linear_had   xh[s][m][k] = fp16(H128(fp16(x * suh[s])) / sqrt(128)) and the 128-blocks' sums xsum[s][m][k / 128]
 //                (the Hadamard on MFMA, as in the MoE input transform; 16 rows per wave)
 //                for every shard s (a fused multi-projection linear: output column blocks of S projections that share
 //                the input, each with its own input signs suh[s]; shard_of_nb maps 128-column blocks to shards)
-//   linear_mfma  workgroup per (row block, k-split, 256-column block); a wave owns four tile columns. With one split
-//                the epilogue writes y; otherwise it writes fp32 partials (affine applied)
+//   linear_wide  (exl3_wide.hip) workgroup per (row block of 32 .. 256 rows, k-split, 256-column block); a wave owns four
+//                tile columns. With one split the epilogue writes y; otherwise it writes fp32 partials (affine applied)
 //   linear_reduce (k-split only) wave per (row, 128 columns): partials in split order, Hadamard, * svh -> y
-struct LinArgs {
-    const _Float16* xh;                              // [S][m][k]
-    const float* xsum;                               // [S][m][k / 128]
-    const int32_t* sonb;                             // shard of each 128-column block (S > 1), else null
-    int S;
-    const uint32_t* tr;
-    const uint16_t* svh;
-    void* out;
-    int64_t out_ld;
-    float* part;                                     // [P][m][n] when P > 1
-    int m, k, n, nblk;
-    int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits, 128-blocks per split
-    int f32;
-};
-
+// xh in blocks of R rows (a multiple of 32) in block_unit order, the units' k as they are or (kperm) as the two 4-k runs
+// of a k-permuted fragment
 __global__ __launch_bounds__(256) void linear_had_kernel(const uint16_t* __restrict__ x, int64_t x_ld, int m, int k,
-                                                         const uint16_t* __restrict__ suh, _Float16* xh, float* xsum) {
+                                                         const uint16_t* __restrict__ suh, _Float16* xh, float* xsum,
+                                                         int R, bool kperm) {
     __shared__ __attribute__((aligned(16))) _Float16 s_out[4][16][136];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kb = blockIdx.y, nblk = k / 128;
@@ -1120,123 +1094,21 @@ __global__ __launch_bounds__(256) void linear_had_kernel(const uint16_t* __restr
     const uint16_t* sv = suh + kb * 128 + 8 * g;
     float part[4];
     had16_rows(xv, sv, ((uintptr_t)sv & 15) == 0, F, lane, s_out[wave], part);
+    const int b0 = r0 / R * R, cnt = m - b0 < R ? m - b0 : R;    // the block that holds the wave's rows
+    u32x4_t* dst = reinterpret_cast<u32x4_t*>(xh + (size_t)b0 * k);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const int u = lane + 64 * c, rr = u >> 4, ch = u & 15;
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&s_out[wave][rr][8 * ch]);
-        if (r0 + rr < m) *reinterpret_cast<u32x4_t*>(xh + (size_t)(r0 + rr) * k + kb * 128 + 8 * ch) = v;
+        const int u = lane + 64 * c, rr = u & 15, h = (u >> 4) & 1, kk = u >> 5;
+        const _Float16* t = &s_out[wave][rr][16 * kk];
+        typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+        const u2_t lo = *reinterpret_cast<const u2_t*>(t + (kperm ? 4 * h : 8 * h));
+        const u2_t hi = *reinterpret_cast<const u2_t*>(t + (kperm ? 4 * h + 8 : 8 * h + 4));
+        if (r0 + rr < m) dst[block_unit(cnt, kb * 8 + kk, h, r0 + rr - b0)] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float v = row16_sum(part[i]);
         if (mm == 0 && r0 + 4 * g + i < m) xsum[(size_t)(r0 + 4 * g + i) * nblk + kb] = v;
-    }
-}
-
-__device__ __forceinline__ void linear_store(const LinArgs& a, int row, int col, float v0, float v1) {
-    if (a.f32) {
-        float* o = reinterpret_cast<float*>(a.out) + (int64_t)row * a.out_ld + col;
-        o[0] = v0;
-        o[64] = v1;
-    } else {
-        uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + (int64_t)row * a.out_ld + col;
-        o[0] = f2h(v0);
-        o[64] = f2h(v1);
-    }
-}
-
-// NPS = 2 for several shards: the two 128-column halves of the block may read different shards' inputs, so both
-// are staged and waves 0, 1 (first half) read plane 0, waves 2, 3 plane 1.
-template <int K, int RGA, int NPS>
-__global__ __launch_bounds__(256, RGA == 1 ? 4 : RGA == 2 ? 3 : 2) void linear_mfma_kernel(LinArgs a) {
-    __shared__ u32x4_t stage[4 * (RGA == 1 ? 4 : NPS * RGA) * 64];   // [4 stages][planes][16 RGA rows x 4 units]
-                                                                    // (per wave at one row group)
-    __shared__ uint32_t wlds[4 * 8 * (8 * K + 4)];       // per wave: 8 staged tiles
-    __shared__ float C[16 * 256];
-    __shared__ float rsum[NPS][16 * RGA];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int blk, nb;
-    xcd_map(a.ncb, blk, nb);
-    if (blk >= a.nrb * a.P) return;
-    const int rb = blk / a.P, p = blk - rb * a.P;
-    const int r0 = rb * 16 * RGA;
-    const int cnt = a.m - r0 < 16 * RGA ? a.m - r0 : 16 * RGA;
-    const int kb0 = p * a.bps, nkb = a.nblk - kb0 < a.bps ? a.nblk - kb0 : a.bps;
-    const int tn = a.n / 16;
-    const int nhalf = 2 * nb + 1 < a.n / 128 ? 2 : 1;
-    // output scales of the two 128-column halves (unconditional loads, unused past nhalf)
-    const uint16_t* sv = a.svh + nb * 256;
-    float sd[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int hh = h < nhalf ? h : 0;
-        sd[h][0] = h2f(ldg(sv + 128 * hh + lane)) * kRsqrt128;
-        sd[h][1] = h2f(ldg(sv + 128 * hh + lane + 64)) * kRsqrt128;
-    }
-    // shard of each staged plane (plane p: the block's 128-column half p; clamped into [0, S))
-    int shard[NPS];
-#pragma unroll
-    for (int q = 0; q < NPS; ++q) {
-        int v = 0;
-        if (NPS > 1) {
-            v = a.sonb[2 * nb + (q < nhalf ? q : 0)];
-            v = v < 0 ? 0 : (v >= a.S ? a.S - 1 : v);
-        }
-        shard[q] = v;
-    }
-    if (threadIdx.x < NPS * 16 * RGA) {                // the rows' sums over this split's 128-blocks, per plane
-        const int q = threadIdx.x / (16 * RGA), r = threadIdx.x - q * 16 * RGA;
-        rsum[q][r] = sum_ordered(a.xsum + ((size_t)shard[q] * a.m + r0 + (r < cnt ? r : cnt - 1)) * a.nblk + kb0, nkb);
-    }
-    __syncthreads();
-    MfmaPipe<K, 1, RGA, NPS> L;
-    L.nsteps = nkb * 4;
-    L.lds = stage;
-    L.lane = lane;
-    L.apl = NPS > 1 ? (wave >> 1) : 0;
-    const uint32_t* trk = a.tr + (size_t)kb0 * 8 * tn * (8 * K);
-    L.setup_w(tn, wlds + wave * 8 * (8 * K + 4), trk, [&](int pair) {
-        const int ct = nb * 16 + 4 * wave + 2 * pair;
-        return ct < tn ? ct : tn - 2;                  // a last half block: in-bounds loads, results unused
-    });
-    L.setup_a(cnt, [&](int q, int row) {                 // a select, not an index: shard[] stays in registers
-        const int sq = (NPS > 1 && q != 0) ? shard[NPS - 1] : shard[0];
-        return a.xh + ((size_t)sq * a.m + r0 + row) * a.k + kb0 * 128;
-    });
-    f4_t acc[kMfT][RGA];
-#pragma unroll
-    for (int t = 0; t < kMfT; ++t)
-#pragma unroll
-        for (int rg = 0; rg < RGA; ++rg) acc[t][rg] = f4_t{0.f, 0.f, 0.f, 0.f};
-    L.run(acc);
-    const bool single = a.P == 1;
-    float* part = a.part + (size_t)p * a.m * a.n;
-#pragma unroll
-    for (int rg = 0; rg < RGA; ++rg) {
-#pragma unroll
-        for (int t = 0; t < kMfT; ++t) {
-            const int col = (4 * wave + t) * 16 + (lane & 15);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) C[(4 * (lane >> 4) + i) * 256 + col] = acc[t][rg][i];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {                 // (row, half) pairs of this wave
-            const int ml = 4 * wave + (j >> 1), h = j & 1, m = 16 * rg + ml;
-            if (m >= cnt || h >= nhalf) continue;
-            const float sx = kMul1C2 * rsum[NPS > 1 ? h : 0][m];
-            float v0 = kMul1C1 * C[ml * 256 + 128 * h + lane] + sx, v1 = kMul1C1 * C[ml * 256 + 128 * h + lane + 64] + sx;
-            const int col = nb * 256 + 128 * h + lane;
-            if (single) {
-                fwht128_wave(v0, v1, lane);
-                linear_store(a, r0 + m, col, v0 * sd[h][0], v1 * sd[h][1]);
-            } else {
-                float* dst = part + (size_t)(r0 + m) * a.n + col;
-                dst[0] = v0;
-                dst[64] = v1;
-            }
-        }
-        __syncthreads();
     }
 }
 
@@ -1377,37 +1249,77 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
     linear_store(a, row, col, v0 * s0, v1 * s1);
 }
 
-typedef void (*lin_fn)(LinArgs);
 
-template <int RGA, int NPS>
-static lin_fn pick_lin(int K) {
-    switch (K) {
-        case 1: return linear_mfma_kernel<1, RGA, NPS>;
-        case 2: return linear_mfma_kernel<2, RGA, NPS>;
-        case 3: return linear_mfma_kernel<3, RGA, NPS>;
-        case 4: return linear_mfma_kernel<4, RGA, NPS>;
-        case 5: return linear_mfma_kernel<5, RGA, NPS>;
-        case 6: return linear_mfma_kernel<6, RGA, NPS>;
-        case 7: return linear_mfma_kernel<7, RGA, NPS>;
-        default: return linear_mfma_kernel<8, RGA, NPS>;
+
+lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
+
+// Row block (RG groups of 32 rows) and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
+// each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
+// workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
+// and that kernel's launch. Fitted to 878 measured points at K = 4 (1024 x 4096 .. 5376 x 21504, 16 .. 1024 rows, 1 .. 16
+// splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
+// blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
+// the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
+struct LinPlan {
+    int RG, P, bps;
+};
+static LinPlan linear_plan(int64_t m, int64_t n, int nblk, const int (&occ)[4], int cus) {
+    static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
+                                        {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
+    static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
+    const int64_t ncb = (n + 255) / 256;
+    // at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the scratch of the partials)
+    const int r0 = m <= 16 ? 16 : m <= 32 ? 32 : 64;
+    const int64_t t0 = (m + r0 - 1) / r0 * ncb, cap = ((m <= 32 ? 3 : 2) * (int64_t)cus + t0 - 1) / t0;
+    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
+    LinPlan best = {1, 1, nblk};
+    float tb = 1e30f;
+    for (int g = 0; g < 4; ++g) {
+        const int64_t tiles = (m + (32 << g) - 1) / (32 << g) * ncb;
+        for (int p = 1; p <= pmax && p <= cap; ++p) {
+            const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
+            if (P != p) continue;
+            const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
+            const float mb = (float)P * (float)m * (float)n * 4e-6f;
+            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
+                      kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
+            if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
+            if (t < tb) {
+                tb = t;
+                best = {1 << g, P, bps};
+            }
+        }
     }
+    return best;
 }
 
-template <int NPS>
-static lin_fn pick_lin_rga(int RGA, int K) {
-    return RGA == 4 ? pick_lin<4, NPS>(K) : RGA == 2 ? pick_lin<2, NPS>(K) : pick_lin<1, NPS>(K);
-}
-
-// Dense linear on MFMA (m > the GEMV's rows per pass). Row blocks of 16, 32 or 64 rows (by m); k-splits so that the
-// grid covers about the workgroups the device holds at once, each split at least two 128-blocks of k.
+// Dense linear on MFMA (m > the GEMV's rows per pass): input transform, blocks of 32 .. 256 rows x 256 columns and, with
+// k-splits, the reduction.
 int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n, int K,
                        void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
                        const uint16_t* svh, hipStream_t st) {
-    const int RGA = m <= 16 ? 1 : m <= 32 ? 2 : 4;
-    const int R = 16 * RGA;
     const int nblk = (int)(k / 128);
     if (m > 0x7FFFFFFF / 64 || k > 0x7FFFFFFF || n > 0x7FFFFFFF || nblk > 65535)
         return fail(EXL3_ERR_INVALID, "exl3_gemm: shape too large");
+    int dev = 0, cus = 0, occ[4];
+    EXL3_CHECK_HIP(hipGetDevice(&dev));
+    EXL3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    for (int g = 0; g < 4; ++g) {
+        int resident = 0;
+        const int rc = resident_blocks((const void*)linear_wide_pick(1 << g, S, K), 256, &resident);
+        if (rc) return rc;
+        occ[g] = resident / cus < 1 ? 1 : resident / cus > 4 ? 4 : resident / cus;
+    }
+    LinPlan pl = linear_plan(m, n, nblk, occ, cus);
+    const int force = env_int("EXL3MI_LINEAR_BLOCK", 0);           // row groups of 32 per block: 1, 2, 4 or 8
+    if (force == 1 || force == 2 || force == 4 || force == 8) pl.RG = force;
+    const int R = 32 * pl.RG;
+    if (const int jobs = env_int("EXL3MI_LINEAR_JOBS", 0)) {       // forced workgroup target
+        const int64_t tiles = (m + R - 1) / R * ((n + 255) / 256), want = (jobs + tiles - 1) / tiles;
+        const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
+        pl.bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
+        pl.P = (nblk + pl.bps - 1) / pl.bps;
+    }
     LinArgs a;
     a.m = (int)m;
     a.k = (int)k;
@@ -1415,21 +1327,12 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     a.nblk = nblk;
     a.nrb = (int)((m + R - 1) / R);
     a.ncb = (int)((n + 255) / 256);
-    lin_fn fn = S > 1 ? pick_lin_rga<2>(RGA, K) : pick_lin_rga<1>(RGA, K);
-    int resident = 0;
-    int rc = resident_blocks((const void*)fn, 256, &resident);
-    if (rc) return rc;
-    const int target = env_int("EXL3MI_LINEAR_JOBS", resident);
-    const int64_t tiles = (int64_t)a.nrb * a.ncb;
-    int P = (int)((target + tiles - 1) / tiles);
-    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
-    P = P < 1 ? 1 : (P > pmax ? pmax : P);
-    a.bps = (nblk + P - 1) / P;
-    a.P = (nblk + a.bps - 1) / a.bps;
+    a.bps = pl.bps;
+    a.P = pl.P;
     const size_t xh_b = carve_size((size_t)S * m * k, 2), xs_b = carve_size((size_t)S * m * nblk, 4);
     const size_t part_b = a.P > 1 ? carve_size((size_t)a.P * m * n, 4) : 0;
     Workspace ws;
-    rc = workspace(xh_b + xs_b + part_b, 0, st, &ws);
+    int rc = workspace(xh_b + xs_b + part_b, 0, st, &ws);
     if (rc) return rc;
     Carve cv{ws.scratch, ws.scratch_bytes};
     _Float16* xh = cv.take<_Float16>((size_t)S * m * k);
@@ -1446,10 +1349,11 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     a.out_ld = c_ld;
     a.f32 = f32 ? 1 : 0;
     const dim3 hgrid((unsigned)((m + 63) / 64), (unsigned)nblk, (unsigned)S);
-    EXL3_LAUNCH("linear_had", linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum);
-    const int64_t nx = ((int64_t)a.nrb * a.P + 7) / 8 * 8 * a.ncb;
+    EXL3_LAUNCH("linear_had", linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum, R,
+                K <= 5);
+    const int64_t nx = ((int64_t)a.nrb * a.ncb * a.P + 7) / 8 * 8;
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_gemm: grid too large");
-    EXL3_LAUNCH("linear_mfma", fn, dim3((unsigned)nx), dim3(256), 0, st, a);
+    EXL3_LAUNCH("linear_wide", linear_wide_pick(pl.RG, S, K), dim3((unsigned)nx), dim3(256), 0, st, a);
     if (a.P > 1)
         EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, dim3((unsigned)((m + 3) / 4), (unsigned)(n / 128)),
                     dim3(256), 0, st, a);

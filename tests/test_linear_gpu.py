@@ -208,6 +208,43 @@ def test_gemm_mfma_splits(exl3, oracle, monkeypatch, jobs, M, out_dtype):
     assert max_rel(y, ref) <= MAX_REL
 
 
+@pytest.mark.parametrize("block", [1, 2, 4, 8])
+@pytest.mark.parametrize("k,n,K,M,out_dtype", [
+    (256, 128, 1, 9, torch.float32), (512, 384, 4, 33, torch.float16), (1152, 640, 5, 257, torch.float32),
+    (640, 256, 6, 31, torch.float16), (1024, 128, 8, 130, torch.float32), (384, 512, 7, 300, torch.float16)])
+def test_gemm_mfma_row_blocks(exl3, oracle, monkeypatch, block, k, n, K, M, out_dtype):
+    """Every row block size (32, 64, 128, 256 rows) over ragged row counts, half column blocks and both fragment orders
+    (K <= 5 and K >= 6), one k-split and several."""
+    monkeypatch.setenv("EXL3MI_LINEAR_BLOCK", str(block))
+    for jobs in ("1", "512"):
+        monkeypatch.setenv("EXL3MI_LINEAR_JOBS", jobs)
+        y, ref = _linear_case(exl3, oracle, k, n, K, M, out_dtype, 7000 + 10 * K + M)
+        assert max_rel(y, ref) <= MAX_REL, jobs
+
+
+@pytest.mark.parametrize("block", [1, 4, 8])
+def test_linear_sharded_row_blocks(exl3, oracle, monkeypatch, block):
+    """Shards under every way a block reads its input planes (straight from memory, two staged planes), into rows
+    that no wide store fits (one element past an aligned address)."""
+    monkeypatch.setenv("EXL3MI_LINEAR_BLOCK", str(block))
+    monkeypatch.setenv("EXL3MI_LINEAR_JOBS", "1")
+    S_ = synth()
+    k, widths, K, M = 512, (128, 384), 3, 140
+    shards = [S_.linear(k, n, K, 7400 + i) for i, n in enumerate(widths)]
+    lins = [exl3.BC_LinearEXL3(tr.cuda(), su.cuda(), sv.cuda(), K, None, False, True, None) for tr, su, sv in shards]
+    tr, suh, svh, sonb, bounds, Kf = exl3.fuse_linears(lins)
+    x = S_.activations(M, k, 7410)
+    n = sum(widths)
+    for dt in (torch.float16, torch.float32):
+        buf = torch.zeros(M * n + 2, dtype=dt, device="cuda")
+        exl3.linear(x.cuda(), tr, suh, svh, sonb, bounds, Kf, out=buf[1:-1].view(M, n))
+        assert buf[0] == 0 and buf[-1] == 0
+        y = buf[1:-1].view(M, n).float().cpu().numpy()
+        for i, (t, su, sv) in enumerate(shards):
+            ref = oracle.exl3_linear(x.numpy(), t.numpy(), su.numpy(), sv.numpy(), K, np.float32)
+            assert max_rel(y[:, bounds[i]:bounds[i + 1]], ref) <= MAX_REL, i
+
+
 @pytest.mark.parametrize("M", [64, 300])
 def test_gemm_mfma_c1_full_size(exl3, oracle, M):
     """4096 -> 4096, K=4 with a prefill-sized batch."""
