@@ -187,6 +187,12 @@ __host__ __device__ __forceinline__ constexpr int64_t block_unit(int cnt, int kk
     return (int64_t)(2 * kk + h) * cnt + r;
 }
 
+// Element of column k in row r of such a block (kperm: the units of k-permuted fragments, K <= 5).
+__host__ __device__ __forceinline__ constexpr int64_t unit_elem(int cnt, int k, int r, bool kperm) {
+    const int q = (k >> 2) & 3, h = kperm ? q & 1 : q >> 1, hi = kperm ? q >> 1 : q & 1;
+    return 8 * block_unit(cnt, k >> 4, h, r) + 4 * hi + (k & 3);
+}
+
 struct LinArgs {
     const _Float16* xh;                              // [S][m][k]
     const float* xsum;                               // [S][m][k / 128]

@@ -1,17 +1,17 @@
 // Expert-sorted ragged grouped GEMM on fp16 MFMA for prefill-sized calls.
 //
-// Rows (token, expert pairs) are grouped by expert and cut into blocks of up to kMfmaRows rows; in a prefill call
-// every expert with rows gets blocks (no GEMV items). Per layer call:
-//   pairs_had   transformed gate / up inputs of every block row, xh[pair][proj] = fp16(H128(fp16(x * suh)) / sqrt(128)),
-//               and their 128-blocks' sums (the codebook affine term)
-//   gateup      workgroup per (block, 128-column block of I), full H; each wave owns two gate and two up tile columns
-//               and decodes them straight into MFMA B fragments once per 32-k step (B holds h = 1024 + bytesum; the
-//               affine is applied as c1 * acc + c2 * rowsum(A) in the epilogue), then the fused activation / down-input
-//               epilogue (Hadamard * svh, act, * suh_d, Hadamard) per 16-row group
+// Rows (token, expert pairs) are grouped by expert and cut into row blocks; in a prefill call every expert with rows gets
+// blocks (no GEMV items). Per layer call:
+//   pairs_had   transformed gate / up inputs of every block row, fp16(H128(fp16(x * suh)) / sqrt(128)), in the order the
+//               gate|up kernel reads them, and their 128-blocks' sums (the codebook affine term)
+//   gateup      workgroup per (block, 128-column block of I), full H: decode straight into MFMA B fragments (B holds
+//               h = 1024 + bytesum; the affine is applied as c1 * acc + c2 * rowsum(A) in the epilogue), then the fused
+//               activation / down-input epilogue (Hadamard * svh, act, * suh_d, Hadamard)
 //   down        workgroup per (block, 256-column block of H), full I, epilogue Hadamard * svh_d * w, then the combine
-// The A rows of the active row groups are staged through a four-stage LDS ring (loaded into registers four steps
-// ahead, stored two steps ahead), weight words three steps ahead; one barrier every second step. Workgroup ids are laid out so that the column blocks
-// of one row block run on one XCD (shared L2 for its A rows).
+// Uniform K runs in exl3_moe_wide.hip (blocks of up to 128 rows), per-tile K here (blocks of up to 64 rows: A staged
+// through a four-stage LDS ring, weight words three steps ahead, one barrier every second step). Workgroup ids are laid
+// out so that the column blocks of one row block run on one XCD (shared L2 for its A rows). The dense linear's input
+// transform, plan and reduction are here too (its kernel: exl3_wide.hip).
 // Semantics: the reference's GateUpDpasKernel / DownDpasKernel / moe_prefill (glm/xpu/csrc/exl3_moe.n128.sycl:
 // 472-689, 868-916) and exllamav3's exl3_moe (ext-op-inventory.md:1060-1093).
 #include "exl3_device.h"
@@ -121,11 +121,11 @@ __global__ __launch_bounds__(256) void pairs_had_kernel(MoeArgs a) {
     if (r0 >= np) return;                                    // past the last row group (uniform)
     const int m = lane & 15, g = lane >> 4;
     const int p = r0 + m < np ? r0 + m : np - 1;
-    const int tok = a.pair_tok[p], e = a.pair_e[p];
-    const bool valid = r0 + m < np && e >= 0;
+    const int tok = a.pair_tok[p], pw = a.pair_e[p];
+    const bool valid = r0 + m < np && pw >= 0;
     const uint32_t vmask = (uint32_t)__builtin_amdgcn_ballot_w64(valid) & 0xFFFFu;   // rows of this job to store
     if (vmask == 0) return;
-    const int ec = valid ? e : 0;
+    const int ec = valid ? pair_expert(pw) : 0;
     const uint16_t* sgn[2];
     if (a.uniform) {
         sgn[0] = reinterpret_cast<const uint16_t*>(a.tb[1] + (int64_t)ec * a.ts[1]);
@@ -152,6 +152,20 @@ __global__ __launch_bounds__(256) void pairs_had_kernel(MoeArgs a) {
     for (int proj = 0; proj < 2; ++proj) {
         float part[4];
         had16_rows(xv, sg[proj], F, lane, s_out[wave], part);
+        if (a.Kg > 0) {                                 // per block in block_unit order: lane = row, 16-byte units
+            const int row = pair_row(pw), cnt = pair_block_rows(pw);
+            u32x4_t* dst = reinterpret_cast<u32x4_t*>(a.xh + ((size_t)(r0 + m - row) * 2 + (size_t)proj * cnt) * a.H);
+            const bool kp = a.Kg <= 5;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int u = lane + 64 * c, h = (u >> 4) & 1, kk = u >> 5;
+                const _Float16* t = &s_out[wave][m][16 * kk];
+                typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+                const u2_t lo = *reinterpret_cast<const u2_t*>(t + (kp ? 4 * h : 8 * h));
+                const u2_t hi = *reinterpret_cast<const u2_t*>(t + (kp ? 4 * h + 8 : 8 * h + 4));
+                if (valid) dst[block_unit(cnt, kb * 8 + kk, h, row)] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+            }
+        } else
 #pragma unroll
         for (int c = 0; c < 4; ++c) {                   // 16-byte row stores from the tile
             const int u = lane + 64 * c, rr = u >> 4, ch = u & 15;
@@ -178,31 +192,11 @@ __device__ __forceinline__ void xcd_map(int nbc, int& blk, int& nb) {
     nb = j - q * nbc;
 }
 
-// ------------------------------------------------------------------------------------------------ pipelined K loop
+// ------------------------------------------------------------------------------------------------ per-tile-K loop
 constexpr int kMfT = 4;                              // tile columns per wave
 
-// Workgroups per CU (= waves per SIMD) the grouped GEMM kernels are compiled for, by row class (1, 2 or 4 row
-// groups). The 4-row-group uniform kernels take one more where their registers allow it without spills (168 VGPRs:
-// gate|up at K = 1, 2 and 4, down at K <= 4); the 1-row-group kernels run five (96 VGPRs; uniform K up to 4, above
-// which they would spill), their epilogue buffer aliasing the pipeline's LDS so that five fit.
-#ifndef EXL3_MFMA_OCC1
-#define EXL3_MFMA_OCC1 4
-#endif
-#ifndef EXL3_MFMA_OCC2
-#define EXL3_MFMA_OCC2 3
-#endif
-#ifndef EXL3_MFMA_OCC4
-#define EXL3_MFMA_OCC4 2
-#endif
-#ifndef EXL3_MFMA_OCC1_KMAX
-#define EXL3_MFMA_OCC1_KMAX 4
-#endif
-#define EXL3_MFMA_OCC(RGA) ((RGA) == 1 ? EXL3_MFMA_OCC1 : (RGA) == 2 ? EXL3_MFMA_OCC2 : EXL3_MFMA_OCC4)
-#define EXL3_MFMA_GU_OCC(RGA, K) \
-    ((RGA) == 4 && ((K) <= 2 || (K) == 4) ? EXL3_MFMA_OCC4 + 1 : (RGA) == 1 && (K) <= EXL3_MFMA_OCC1_KMAX ? 5 \
-                                                                   : EXL3_MFMA_OCC(RGA))
-#define EXL3_MFMA_DOWN_OCC(RGA, K) \
-    ((RGA) == 4 && (K) <= 4 ? EXL3_MFMA_OCC4 + 1 : (RGA) == 1 && (K) <= EXL3_MFMA_OCC1_KMAX ? 5 : EXL3_MFMA_OCC(RGA))
+// Workgroups per CU (= waves per SIMD) the per-tile-K kernels are compiled for, by row class (1, 2 or 4 row groups of 16);
+// the 1-row-group kernels run five (96 VGPRs), their epilogue buffer aliasing the pipeline's LDS so that five fit.
 #ifndef EXL3_MIX_OCC1
 #define EXL3_MIX_OCC1 5
 #endif
@@ -222,218 +216,6 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 
-// One wave accumulates kMfT tile columns over all 32-k steps for RGA row groups. Tile column t of the wave belongs to
-// column pair t >> 1 (gate|up: the projection; down: columns c0, c0 + 1 or c0 + 2, c0 + 3), whose two adjacent tiles of
-// one tile-row are contiguous in memory.
-//   weights: per step the wave's 8 tiles (2 pairs x 2 tile-rows x 2 tiles) come in with ONE coalesced load of K words
-//            per lane (16 lanes per 2-tile segment), loaded DW - 1 steps ahead into a register ring, and are staged in a
-//            wave-private LDS slot per tile laid out as [w(8K-1), w(0) .. w(8K-1), w(0), w(1), w(2)], so that every
-//            lane's fragment window (first word -1 .. 8K - 1, at most 8K + 2 past) is contiguous: no wrap logic, and
-//            per-lane scattered loads (64-bit addresses per lane into the texture unit) become LDS reads. For K <= 5
-//            the fragments are k-permuted (two funnels of four windows per lane, fragp_finish); K >= 6 keeps the
-//            natural k order (frag_finish).
-//   A:       staged per step by the whole workgroup: loaded into register slot s % 2 three steps ahead, stored to
-//            LDS stage s % 4 two steps ahead, with a barrier after the even steps only (a stage is rewritten two steps
-//            after its last read, with a barrier in between, and read at least one barrier after its write); memory-
-//            counter waits complete in issue order, so each step issues its A load before its weight load. With
-//            k-permuted fragments a row's 4-k units are staged in the order 0 2 1 3 4 6 5 7 (two 8-byte stores per
-//            16-byte unit), so that a lane's 16-byte read holds the k of its B fragment. With one row group and one
-//            plane read per wave, each wave stages its own plane in a private ring instead (one unit per lane, the
-//            loads and LDS writes of the shared ring, whose threads stage its units twice or more) and the loop has no
-//            barrier.
-template <int K, int NP, int RGA, int NPS = NP, bool PL = false>
-struct MfmaPipe {
-    static constexpr bool KP = K <= 5;                      // k-permuted fragments
-    static constexpr int NW = FragCfg<K>::NW;
-    static constexpr int DW = 4;
-    static constexpr int TPP = kMfT / NP;
-    static constexpr int TS = 8 * K + 4;                     // LDS words per staged tile
-    static constexpr int UNITS = NPS * RGA * 64;             // 16-byte A units per stage (NPS staged planes)
-    static constexpr bool PRIV = RGA == 1 && NP == 1;        // wave-private A ring
-    static constexpr int SU = PRIV ? 64 : UNITS;             // units per stage (of the wave's ring if PRIV)
-    static constexpr int CPT = PRIV ? 1 : (UNITS + 255) / 256;   // A units a thread stages per step
-    const uint32_t* wsrc;                                    // this lane's K words at step 0
-    uint32_t wstep;                                          // words between consecutive steps (two tile-rows)
-    int nsteps;
-    uint32_t* wl;                                            // the wave's LDS slots [8][TS]
-    int wdst, wslot;                                         // this lane's staged words: slot wslot, word wdst
-    int w0;                                                  // fragment window origin (ring word, -1 .. 8K - 1)
-    uint32_t sh;
-    uint32_t fa[2], fsh[2];                                  // k-permuted: LDS byte address of each run's funnel
-                                                             // words in slot 0, and its shift
-    __amdgpu_buffer_rsrc_t abuf[CPT];                        // this thread's staged A units at step 0: a buffer
-    uint32_t aoff[CPT];                                      // the wave shares, and the lane's byte offset in it
-    int adst[CPT];                                           // k-permuted: 8-byte units of the low and high halves
-    int adst2[CPT];
-    u32x4_t* lds;                                            // [4][SU] (per wave if PRIV)
-    int lane;
-    int apl = 0;                                             // first staged plane this wave reads (NPS > NP)
-
-    __device__ __forceinline__ void load_w(uint32_t (&D)[K], int s) const {
-        const uint32_t* p = wsrc + (uint32_t)(s < nsteps ? s : nsteps - 1) * wstep;
-#pragma unroll
-        for (int i = 0; i < K; ++i) D[i] = ldg_nt(p + WordOrder<K, PL>::word_off(i));
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    __device__ __forceinline__ void stage_w(const uint32_t (&D)[K]) const {
-        uint32_t* t = wl + wslot * TS;
-#pragma unroll
-        for (int i = 0; i < K; ++i) t[1 + wdst + i] = D[i];
-        const int q = lane & 7;                              // this lane's eighth of the tile
-        if (q == 7) t[0] = D[K - 1];                          // w(8K - 1) in front
-#pragma unroll
-        for (int u = 0; u < 3; ++u)                          // w(0..2) behind
-            if (q == u / K) t[8 * K + 1 + u] = D[u % K];
-    }
-    __device__ __forceinline__ void compute(int stage, f4_t (&acc)[kMfT][RGA]) const {
-        h8_t bf[kMfT];
-        if constexpr (KP) {
-            uint32_t fw[kMfT][4];
-#pragma unroll
-            for (int t = 0; t < kMfT; ++t) {
-                const int slot = 2 * (2 * (t >> 1) + (lane >> 5)) + (t & 1);
-#pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const lds_cu32_t o = (lds_cu32_t)fa[g];
-                    fw[t][2 * g] = o[slot * TS];
-                    fw[t][2 * g + 1] = o[slot * TS + 1];
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < kMfT; ++t) bf[t] = fragp_finish<K>(fw[t], fsh);
-        } else {
-#pragma unroll
-            for (int t = 0; t < kMfT; ++t) {
-                const int slot = 2 * (2 * (t >> 1) + (lane >> 5)) + (t & 1);
-                const uint32_t* r = wl + slot * TS + 1 + w0;
-                uint32_t R[NW];
-#pragma unroll
-                for (int i = 0; i < NW; ++i) R[i] = r[i];
-                bf[t] = frag_finish<K>(R, sh);
-            }
-        }
-        // A fragments per plane, after the B decode (fewer live registers: three waves per SIMD at four row groups)
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            h8_t af[RGA];
-#pragma unroll
-            for (int rg = 0; rg < RGA; ++rg)
-                af[rg] = __builtin_bit_cast(
-                    h8_t, lds[stage * SU + (PRIV ? 0 : (p + apl) * RGA * 64) + a_unit(16 * rg + (lane & 15), lane >> 4)]);
-#pragma unroll
-            for (int t = p * TPP; t < (p + 1) * TPP; ++t)
-#pragma unroll
-                for (int rg = 0; rg < RGA; ++rg)
-                    acc[t][rg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[rg], bf[t], acc[t][rg], 0, 0, 0);
-        }
-    }
-    // step s, with every ring slot known at compile time (R = s mod 4)
-    template <int R>
-    __device__ __forceinline__ void step(int s, uint32_t (&W)[DW][K], u32x4_t (&RA)[2][CPT],
-                                         f4_t (&acc)[kMfT][RGA]) const {
-        load_a(RA[R % 2], s + 3);
-        load_w(W[(R + DW - 1) % DW], s + DW - 1);
-        stage_w(W[R % DW]);
-        compute(R, acc);
-        store_a(RA[(R + 1) % 2], (R + 2) % 4);
-        if constexpr (!PRIV) {
-            if (R % 2 == 0) __syncthreads();
-        }
-    }
-    __device__ __forceinline__ void load_a(u32x4_t (&Ra)[CPT], int s) const {
-        const int ss = (s < nsteps ? s : nsteps - 1) * 32;
-#pragma unroll
-        for (int j = 0; j < CPT; ++j)
-            Ra[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(abuf[j], aoff[j], 2 * ss, 0));
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    __device__ __forceinline__ void store_a(const u32x4_t (&Ra)[CPT], int stage) const {
-        if constexpr (KP) {
-            typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
-            u2_t* l2 = reinterpret_cast<u2_t*>(lds) + 2 * stage * SU;
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                const u2_t lo = {Ra[j][0], Ra[j][1]}, hi = {Ra[j][2], Ra[j][3]};
-                l2[adst[j]] = lo;
-                l2[adst2[j]] = hi;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) lds[stage * SU + adst[j]] = Ra[j];
-        }
-    }
-    __device__ __forceinline__ void run(f4_t (&acc)[kMfT][RGA]) const {
-        uint32_t W[DW][K];
-        u32x4_t RA[2][CPT];
-        load_a(RA[0], 0);
-        load_a(RA[1], 1);
-#pragma unroll
-        for (int i = 0; i < DW - 1; ++i) load_w(W[i], i);
-        store_a(RA[0], 0);
-        store_a(RA[1], 1);
-        load_a(RA[1], 2);
-        __syncthreads();
-        int s = 0;
-        for (; s + 4 <= nsteps; s += 4) {
-            step<0>(s, W, RA, acc);
-            step<1>(s + 1, W, RA, acc);
-            step<2>(s + 2, W, RA, acc);
-            step<3>(s + 3, W, RA, acc);
-        }
-        if (s < nsteps) step<0>(s, W, RA, acc);
-        if (s + 1 < nsteps) step<1>(s + 1, W, RA, acc);
-        if (s + 2 < nsteps) step<2>(s + 2, W, RA, acc);
-        __syncthreads();                                 // every wave's last LDS read done: callers may reuse it
-    }
-    // weight set-up: tr = tile-row 0 of the projection, pair_col(pair) = the pair's first tile column (even); tile-rows
-    // are tn * 8K words apart. Lane (lane & 15) of a pair segment takes chunk lane & 7 of the pair's tile
-    // (lane & 15) >> 3, in the word order PL (WordOrder).
-    template <typename F>
-    __device__ __forceinline__ void setup_w(int tn, uint32_t* wave_lds, const uint32_t* tr, F pair_col) {
-        const int g = lane >> 4, pair = g >> 1, hr = g & 1;
-        wsrc = tr + (size_t)hr * tn * (8 * K) +
-               WordOrder<K, PL>::chunk_base(pair_col(pair) + ((lane & 15) >> 3), lane & 7);
-        wstep = (uint32_t)(2 * tn * 8 * K);
-        wl = wave_lds;
-        wslot = 2 * g + ((lane & 15) >> 3);
-        wdst = (lane & 7) * K;
-        if constexpr (KP) {
-            int off[2];
-            fragp_origin<K>(lane, off, fsh);
-#pragma unroll
-            for (int g = 0; g < 2; ++g) fa[g] = lds_addr(wl) + 4u * (uint32_t)off[g];
-        } else {
-            frag_origin<K>(lane, w0, sh);
-        }
-    }
-    // staging set-up: unit u = (tid + 256 j) mod UNITS (UNITS < 256: several threads stage the same unit, writing
-    // the same value, so that the loads and stores stay unconditional: a branch around them would make the compiler
-    // drain every outstanding load, the weight prefetch included) of plane p = u / (RGA * 64): row (u % (RGA * 64)) / 4
-    // (clamped to the block's last row), chunk u % 4, from row pointer rowptr(p, row) (k offset 0). A wave's 64 units
-    // lie in one plane (UNITS and RGA * 64 are multiples of 64), so the loads are buffer loads from the plane's row 0
-    // (a wave-uniform resource) at a 32-bit lane offset plus the step's scalar offset: no address arithmetic per step.
-    template <typename F>
-    __device__ __forceinline__ void setup_a(int cnt, F rowptr) {
-        const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        if constexpr (PRIV) lds += wv * 4 * SU;
-#pragma unroll
-        for (int j = 0; j < CPT; ++j) {
-            const int u0 = PRIV ? apl * 64 : (64 * wv + 256 * j) % UNITS, u = u0 + (threadIdx.x & 63);
-            const int p = u0 / (RGA * 64), rem = u - p * RGA * 64, row = rem >> 2, ch = rem & 3;
-            const int pd = PRIV ? 0 : p;                     // the unit's plane in the stage
-            const _Float16* b = rowptr(p, 0);
-            abuf[j] = buffer_rsrc(b);
-            aoff[j] = (uint32_t)(2 * (rowptr(p, row < cnt ? row : cnt - 1) + 8 * ch - b));
-            if constexpr (KP) {                              // 4-k units 2 ch, 2 ch + 1 -> 16-byte units
-                adst[j] = 2 * (pd * RGA * 64 + a_unit(row, ch & 2)) + (ch & 1);       // (ch & 2) and (ch & 2) + 1,
-                adst2[j] = 2 * (pd * RGA * 64 + a_unit(row, (ch & 2) + 1)) + (ch & 1); // half ch & 1
-            } else {
-                adst[j] = pd * RGA * 64 + a_unit(row, ch);
-            }
-        }
-    }
-};
-
 // ------------------------------------------------------------------------------------------------ gate | up
 template <int RGA>
 __device__ __forceinline__ void gateup_epilogue(const MoeArgs& a, const ItemDesc* d, int nb, int cnt,
@@ -441,31 +223,6 @@ __device__ __forceinline__ void gateup_epilogue(const MoeArgs& a, const ItemDesc
 template <int RGA>
 __device__ __forceinline__ void down_epilogue(const MoeArgs& a, const ItemDesc* d, int nb, int cnt,
                                               const f4_t (&acc)[kMfT][RGA], float* C, const float* rsum, int* s_comb);
-
-template <int K, int RGA, bool PL>
-__device__ __forceinline__ void gateup_mfma_body(const MoeArgs& a, const ItemDesc* d, int nb, int cnt, u32x4_t* stage,
-                                                 uint32_t* wlds, float* C, float* rsum) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int p0 = d->p0;
-    const int tn = a.gu_tn;
-    const int pw = wave >> 1;                              // this wave's projection (gate, up), its 4 tile columns
-    const uint32_t* trp = reinterpret_cast<const uint32_t*>(d->tab[3 * pw]);
-    const int ct0 = nb * 8 + 4 * (wave & 1);
-    MfmaPipe<K, 1, RGA, 2, PL> L;
-    L.nsteps = a.H / 32;
-    L.lds = stage;
-    L.lane = lane;
-    L.apl = pw;
-    L.setup_w(tn, wlds + wave * 8 * (8 * K + 4), trp, [&](int pair) { return ct0 + 2 * pair; });
-    L.setup_a(cnt, [&](int p, int row) { return a.xh + ((size_t)(p0 + row) * 2 + p) * a.H; });
-    f4_t acc[kMfT][RGA];
-#pragma unroll
-    for (int t = 0; t < kMfT; ++t)
-#pragma unroll
-        for (int rg = 0; rg < RGA; ++rg) acc[t][rg] = f4_t{0.f, 0.f, 0.f, 0.f};
-    L.run(acc);
-    gateup_epilogue<RGA>(a, d, nb, cnt, acc, C, rsum);
-}
 
 // Affine, Hadamard * svh, act(g, u) * suh_d, Hadamard of the workgroup's 128 columns per 16-row group -> abuf (fp16)
 // and its block sums (the down GEMM's affine term).
@@ -510,9 +267,15 @@ __device__ __forceinline__ void gateup_epilogue(const MoeArgs& a, const ItemDesc
             a1 = (float)(_Float16)(a1 * sd1);
             fwht128_wave(a0, a1, lane);
             const _Float16 h0 = (_Float16)(a0 * kRsqrt128), h1 = (_Float16)(a1 * kRsqrt128);
-            uint16_t* dst = a.abuf + (size_t)(p0 + m) * a.I + nb * 128;
-            dst[lane] = __builtin_bit_cast(uint16_t, h0);
-            dst[lane + 64] = __builtin_bit_cast(uint16_t, h1);
+            if (a.Kd > 0) {                           // uniform down K: the block in block_unit order
+                uint16_t* dst = a.abuf + (size_t)p0 * a.I + unit_elem(cnt, nb * 128 + lane, m, a.Kd <= 5);
+                dst[0] = __builtin_bit_cast(uint16_t, h0);
+                dst[8 * block_unit(cnt, 4, 0, 0)] = __builtin_bit_cast(uint16_t, h1);   // 64 columns on
+            } else {
+                uint16_t* dst = a.abuf + (size_t)(p0 + m) * a.I + nb * 128;
+                dst[lane] = __builtin_bit_cast(uint16_t, h0);
+                dst[lane + 64] = __builtin_bit_cast(uint16_t, h1);
+            }
             const float bs = wave_sum_f32((float)h0 + (float)h1);
             if (lane == 0) a.asum[(size_t)(p0 + m) * nbI + nb] = bs;
         }
@@ -520,62 +283,8 @@ __device__ __forceinline__ void gateup_epilogue(const MoeArgs& a, const ItemDesc
     }
 }
 
-// One instance per row class (RGA row groups of 16): workgroup (list index, column block); indices past the class's
-// block count exit at once.
-template <int K, int RGA, bool PL = false>
-__global__ __launch_bounds__(256, EXL3_MFMA_GU_OCC(RGA, K)) void gateup_mfma_kernel(MoeArgs a) {
-    constexpr int CL = RGA == 1 ? 0 : RGA == 2 ? 1 : 2;
-    // A stages [4][2 planes][16 RGA rows x 4 units] (or per wave [4][16 rows x 4 units]) and per wave 8 staged tiles;
-    // the epilogue's C reuses them (dead once the pipeline has drained)
-    constexpr int kStage = 4 * (RGA == 1 ? 4 : 2 * RGA) * 64 * 16, kW = 4 * 8 * (8 * K + 4) * 4, kC = 2 * 16 * 128 * 4;
-    __shared__ __attribute__((aligned(16))) char smem[kStage + kW > kC ? kStage + kW : kC];
-    u32x4_t* stage = reinterpret_cast<u32x4_t*>(smem);
-    uint32_t* wlds = reinterpret_cast<uint32_t*>(smem + kStage);
-    float* C = reinterpret_cast<float*>(smem);
-    __shared__ float rsum[2 * 64];
-    const int nbI = a.I / 128;
-    int idx, nb;
-    xcd_map(nbI, idx, nb);
-    if (idx >= a.cls_cnt[CL]) return;
-    const ItemDesc* d = a.blocks + a.cls_list[CL * a.max_blocks + idx];
-    const int cnt = d->cnt;
-    // row sums of the block's A rows (block sums in order)
-    const int nblk = a.H / 128;
-    for (int i = threadIdx.x; i < 2 * 64; i += 256) {
-        const int p = i >> 6, m = i & 63;
-        rsum[i] = m < cnt ? sum_ordered(a.xsum + ((size_t)(d->p0 + m) * 2 + p) * nblk, nblk) : 0.f;
-    }
-    __syncthreads();
-    gateup_mfma_body<K, RGA, PL>(a, d, nb, cnt, stage, wlds, C, rsum);
-}
-
 // ------------------------------------------------------------------------------------------------ down
 // 256 output columns per workgroup (two Hadamard blocks): wave w owns tile columns 4w .. 4w + 3.
-template <int K, int RGA, bool PL>
-__device__ __forceinline__ void down_mfma_body(const MoeArgs& a, const ItemDesc* d, int nb, int cnt, u32x4_t* stage,
-                                               uint32_t* wlds, float* C, float* rsum, int* s_comb) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int p0 = d->p0;
-    const int tn = a.H / 16;
-    const uint32_t* trd = reinterpret_cast<const uint32_t*>(d->tab[6]);
-    MfmaPipe<K, 1, RGA, 1, PL> L;
-    L.nsteps = a.I / 32;
-    L.lds = stage;
-    L.lane = lane;
-    L.setup_w(tn, wlds + wave * 8 * (8 * K + 4), trd, [&](int pair) {
-        const int ct = nb * 16 + 4 * wave + 2 * pair;
-        return ct < tn ? ct : tn - 2;                  // a last half block: in-bounds loads, results unused
-    });
-    L.setup_a(cnt, [&](int, int row) { return reinterpret_cast<const _Float16*>(a.abuf) + (size_t)(p0 + row) * a.I; });
-    f4_t acc[kMfT][RGA];
-#pragma unroll
-    for (int t = 0; t < kMfT; ++t)
-#pragma unroll
-        for (int rg = 0; rg < RGA; ++rg) acc[t][rg] = f4_t{0.f, 0.f, 0.f, 0.f};
-    L.run(acc);
-    down_epilogue<RGA>(a, d, nb, cnt, acc, C, rsum, s_comb);
-}
-
 // Affine, Hadamard * svh_d * w of the workgroup's 256 columns per 16-row group -> y rows, then the combine.
 template <int RGA>
 __device__ __forceinline__ void down_epilogue(const MoeArgs& a, const ItemDesc* d, int nb, int cnt,
@@ -641,30 +350,6 @@ __device__ __forceinline__ void down_epilogue(const MoeArgs& a, const ItemDesc* 
     __syncthreads();
     for (int i = wave; i < 2 * cnt; i += 4)
         if (s_comb[i] >= 0) combine_token(a, s_comb[i], 2 * nb + (i & 1), lane);
-}
-
-template <int K, int RGA, bool PL = false>
-__global__ __launch_bounds__(256, EXL3_MFMA_DOWN_OCC(RGA, K)) void down_mfma_kernel(MoeArgs a) {
-    constexpr int CL = RGA == 1 ? 0 : RGA == 2 ? 1 : 2;
-    // A stages [4][16 RGA rows x 4 units] (per wave at one row group) and per wave 8 staged tiles; C aliases, as above
-    constexpr int kStage = 4 * (RGA == 1 ? 4 : RGA) * 64 * 16, kW = 4 * 8 * (8 * K + 4) * 4, kC = 16 * 256 * 4;
-    __shared__ __attribute__((aligned(16))) char smem[kStage + kW > kC ? kStage + kW : kC];
-    u32x4_t* stage = reinterpret_cast<u32x4_t*>(smem);
-    uint32_t* wlds = reinterpret_cast<uint32_t*>(smem + kStage);
-    float* C = reinterpret_cast<float*>(smem);
-    __shared__ float rsum[64];
-    __shared__ int s_comb[2 * 64];
-    const int nbH2 = (a.H / 128 + 1) / 2;
-    int idx, nb;
-    xcd_map(nbH2, idx, nb);
-    if (idx >= a.cls_cnt[CL]) return;
-    const ItemDesc* d = a.blocks + a.cls_list[CL * a.max_blocks + idx];
-    const int cnt = d->cnt;
-    const int nbI = a.I / 128;
-    for (int m = threadIdx.x; m < 64; m += 256)
-        rsum[m] = m < cnt ? sum_ordered(a.asum + (size_t)(d->p0 + m) * nbI, nbI) : 0.f;
-    __syncthreads();
-    down_mfma_body<K, RGA, PL>(a, d, nb, cnt, stage, wlds, C, rsum, s_comb);
 }
 
 // ------------------------------------------------------------------------------------------------ per-tile K
@@ -1115,64 +800,6 @@ __global__ __launch_bounds__(256) void linear_had_kernel(const uint16_t* __restr
 // ------------------------------------------------------------------------------------------------ host
 typedef void (*mfma_fn)(MoeArgs);
 
-// Raise a kernel's dynamic-LDS limit once (the attribute is per function).
-static hipError_t set_max_lds(const void* fn, int bytes) {
-    static const void* done[64];
-    static int ndone = 0;
-    for (int i = 0; i < ndone; ++i)
-        if (done[i] == fn) return hipSuccess;
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess && ndone < 64) done[ndone++] = fn;
-    return e;
-}
-
-// PLANAR4 instantiations where that order differs from tile order (K = 3, 5, 6, 7)
-template <int RGA>
-static mfma_fn pick_gu(int K, bool pl) {
-    if (pl) {
-        switch (K) {
-            case 3: return gateup_mfma_kernel<3, RGA, true>;
-            case 5: return gateup_mfma_kernel<5, RGA, true>;
-            case 6: return gateup_mfma_kernel<6, RGA, true>;
-            case 7: return gateup_mfma_kernel<7, RGA, true>;
-            default: break;
-        }
-    }
-    switch (K) {
-        case 1: return gateup_mfma_kernel<1, RGA>;
-        case 2: return gateup_mfma_kernel<2, RGA>;
-        case 3: return gateup_mfma_kernel<3, RGA>;
-        case 4: return gateup_mfma_kernel<4, RGA>;
-        case 5: return gateup_mfma_kernel<5, RGA>;
-        case 6: return gateup_mfma_kernel<6, RGA>;
-        case 7: return gateup_mfma_kernel<7, RGA>;
-        default: return gateup_mfma_kernel<8, RGA>;
-    }
-}
-
-template <int RGA>
-static mfma_fn pick_dn(int K, bool pl) {
-    if (pl) {
-        switch (K) {
-            case 3: return down_mfma_kernel<3, RGA, true>;
-            case 5: return down_mfma_kernel<5, RGA, true>;
-            case 6: return down_mfma_kernel<6, RGA, true>;
-            case 7: return down_mfma_kernel<7, RGA, true>;
-            default: break;
-        }
-    }
-    switch (K) {
-        case 1: return down_mfma_kernel<1, RGA>;
-        case 2: return down_mfma_kernel<2, RGA>;
-        case 3: return down_mfma_kernel<3, RGA>;
-        case 4: return down_mfma_kernel<4, RGA>;
-        case 5: return down_mfma_kernel<5, RGA>;
-        case 6: return down_mfma_kernel<6, RGA>;
-        case 7: return down_mfma_kernel<7, RGA>;
-        default: return down_mfma_kernel<8, RGA>;
-    }
-}
-
 template <typename F>
 static int fork3(hipStream_t st, F launch) {
     // the three row classes run concurrently: 4 row groups on the caller's stream, 2 and 1 on the side streams
@@ -1195,6 +822,10 @@ static int fork3(hipStream_t st, F launch) {
     return EXL3_OK;
 }
 
+int launch_gateup_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);     // exl3_moe_wide.hip (uniform K)
+int launch_down_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);
+int launch_moe_combine(const MoeArgs& a, hipStream_t st);
+
 // The grouped GEMM of one layer call: the input transform, then per row class gate|up followed by down on that class's
 // stream (a class's down blocks read only the down inputs its own gate|up blocks wrote; tokens whose slots span
 // classes are combined by the last slot to finish), so one class's down pass overlaps the others' gate|up.
@@ -1204,19 +835,22 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
     EXL3_CHECK_ARG(had_jobs / 4 < 0x7FFFFFFF, "exl3_moe_forward: too many rows");
     EXL3_LAUNCH("moe_pairs_had", pairs_had_kernel, dim3((unsigned)((had_jobs + 3) / 4)), dim3(256), 0, st, a);
     const dim3 grid_gu(nxb * (a.I / 128)), grid_dn(nxb * ((a.H / 128 + 1) / 2));
-    return fork3(st, [&](int rga, hipStream_t s) -> int {
-        mfma_fn gu = a.Kg == 0 ? (rga == 4 ? gateup_mix_kernel<4> : rga == 2 ? gateup_mix_kernel<2> : gateup_mix_kernel<1>)
-                               : (rga == 4 ? pick_gu<4>(a.Kg, a.planar) : rga == 2 ? pick_gu<2>(a.Kg, a.planar)
-                                            : pick_gu<1>(a.Kg, a.planar));
-        mfma_fn dn = a.Kd == 0 ? (rga == 4 ? down_mix_kernel<4> : rga == 2 ? down_mix_kernel<2> : down_mix_kernel<1>)
-                               : (rga == 4 ? pick_dn<4>(a.Kd, a.planar) : rga == 2 ? pick_dn<2>(a.Kd, a.planar)
-                                            : pick_dn<1>(a.Kd, a.planar));
-        EXL3_LAUNCH(rga == 4 ? "moe_gateup_mfma_r4" : rga == 2 ? "moe_gateup_mfma_r2" : "moe_gateup_mfma_r1", gu,
-                    grid_gu, dim3(256), 0, s, a);
+    const int rc = fork3(st, [&](int rga, hipStream_t s) -> int {
+        const int cl = rga == 4 ? 2 : rga == 2 ? 1 : 0;
+        if (a.Kg == 0) {
+            mfma_fn gu = rga == 4 ? gateup_mix_kernel<4> : rga == 2 ? gateup_mix_kernel<2> : gateup_mix_kernel<1>;
+            EXL3_LAUNCH(rga == 4 ? "moe_gateup_mfma_r4" : rga == 2 ? "moe_gateup_mfma_r2" : "moe_gateup_mfma_r1", gu,
+                        grid_gu, dim3(256), 0, s, a);
+        } else if (const int e = launch_gateup_wide(a, cl, grid_gu, s)) {
+            return e;
+        }
+        if (a.Kd > 0) return launch_down_wide(a, cl, grid_dn, s);
+        mfma_fn dn = rga == 4 ? down_mix_kernel<4> : rga == 2 ? down_mix_kernel<2> : down_mix_kernel<1>;
         EXL3_LAUNCH(rga == 4 ? "moe_down_mfma_r4" : rga == 2 ? "moe_down_mfma_r2" : "moe_down_mfma_r1", dn, grid_dn,
                     dim3(256), 0, s, a);
         return EXL3_OK;
     });
+    return rc || a.Kd == 0 ? rc : launch_moe_combine(a, st);
 }
 
 // Split-K finish: wave per (row, 128-column block): the split partials summed in split order (eight splits' loads in

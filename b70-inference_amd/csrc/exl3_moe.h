@@ -8,10 +8,19 @@ namespace exl3 {
 constexpr int kMoeMaxExperts = 2048;   // expert tables per layer (routed + shared); the align kernel keeps 5 ints each in LDS
 constexpr int kMoeSmallRows = 8;       // experts with at most this many rows in a call take the GEMV kernels
 constexpr int kMfmaRows = 64;          // row block of the MFMA grouped GEMM
+constexpr int kWideRows = 128;         // the same with uniform K <= 5 (gate|up and down; above, 128 rows would spill)
 
-// Row class of an MFMA block (0: <= 16 rows, 1: <= 32, 2: <= 64): each class runs its own kernel instance sized for
-// its row groups, so that small blocks get the register budget (and occupancy) of a small block.
-__host__ __device__ constexpr int mfma_row_class(int cnt) { return cnt <= 16 ? 0 : cnt <= 32 ? 1 : 2; }
+// Row class of an MFMA block by the call's row block MB (class 0: <= MB / 4 rows, 1: <= MB / 2, 2: <= MB): each class runs
+// its own kernel instance sized for its rows, so that small blocks get the register budget (and occupancy) of a small
+// block.
+__host__ __device__ constexpr int mfma_row_class(int cnt, int MB) { return 4 * cnt <= MB ? 0 : 2 * cnt <= MB ? 1 : 2; }
+
+// A sorted pair's expert, its row in its MFMA block and the block's rows, in one word.
+static_assert(kMoeMaxExperts <= 1 << 11 && kWideRows <= 1 << 7 && kMfmaRows <= 1 << 7, "pair word");
+__host__ __device__ constexpr int pair_word(int e, int row, int cnt) { return e | row << 11 | (cnt - 1) << 18; }
+__host__ __device__ constexpr int pair_expert(int w) { return w & 0x7FF; }
+__host__ __device__ constexpr int pair_row(int w) { return w >> 11 & 0x7F; }
+__host__ __device__ constexpr int pair_block_rows(int w) { return (w >> 18 & 0x7F) + 1; }
 
 // One work unit of the GEMV kernels: up to 8 rows (pairs) of one expert, with everything a workgroup needs so that a
 // single uniform load replaces the table lookups. Items past the last real one have cnt == 0.
@@ -37,13 +46,13 @@ struct RouteArgs {
     int use_mfma, MB;                  // experts with more than MR rows -> blocks of MB rows for the MFMA kernels
     ItemDesc* blocks;                  // [max_blocks]
     int max_blocks;
-    int* cls_list;                     // optional [3][max_blocks]: block indices by row class (<= 16, 32, 64 rows)
+    int* cls_list;                     // optional [3][max_blocks]: block indices by row class
     int* cls_cnt;                      // [3]
     int* pair_tok;
     float* pair_w;
     int* pair_of;
-    int* pair_e;                       // optional [M * slots]: expert of each pair in sorted order, -1 past the valid
-                                       // pairs
+    int* pair_e;                       // optional [M * slots]: pair_word of each pair in sorted order, -1 past the
+                                       // valid pairs
     int* tok_nvalid;                   // optional [M]: valid slots per token; tokens with none get a zero output row
     void* out;
     int64_t out_ld;
@@ -90,20 +99,23 @@ struct MoeArgs {
     const ItemDesc* items;
     const ItemDesc* blocks;            // MFMA row blocks (cnt == 0 past the last)
     int max_blocks;
-    const int* cls_list;               // [3][max_blocks] block indices by row class (<= 16, <= 32, <= 64 rows)
+    const int* cls_list;               // [3][max_blocks] block indices by row class
     const int* cls_cnt;                // [3] blocks per class
-    _Float16* xh;                      // [pairs][2][H] transformed gate / up inputs of MFMA rows
+    _Float16* xh;                      // [pairs][2][H] transformed gate / up inputs of MFMA rows; uniform gate|up K:
+                                       // per block [2][cnt * H] in block_unit order (exl3_mfma.h)
     float* xsum;                       // [pairs][2][H / 128] block sums of xh (the MFMA rows' affine term)
     float* asum;                       // [pairs][I / 128] block sums of abuf (MFMA rows)
     int* pair_tok;
     float* pair_w;
     int* pair_of;
-    int* pair_e;                       // [pairs] expert of each pair in sorted order, -1 past the valid pairs (MFMA
-                                       // path)
+    int* pair_e;                       // [pairs] pair_word of each pair in sorted order, -1 past the valid pairs
+                                       // (MFMA path)
+    int block_rows;                    // row block of the call's MFMA blocks (kMfmaRows or kWideRows)
     int* tok_nvalid;                   // [M] valid slots per token
     int* cnt_tok;                      // [M][H/128] combine arrival counters
     // intermediates (workspace)
-    uint16_t* abuf;                    // [pairs][I] fp16, Hadamard-domain down input
+    uint16_t* abuf;                    // [pairs][I] fp16, Hadamard-domain down input (MFMA rows at uniform down K: per
+                                       // block in block_unit order)
     float* y;                          // [pairs][H] fp32, weighted expert outputs
     float* part_gu;
     int* cnt_gu;

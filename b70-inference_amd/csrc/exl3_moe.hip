@@ -290,7 +290,7 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
             const int dc = min(r.MB, c - q * r.MB);
             write_desc(d, e, start[e] + q * r.MB, dc, tb, km);
             if (r.cls_list) {
-                const int cl = mfma_row_class(dc);
+                const int cl = mfma_row_class(dc, r.MB);
                 r.cls_list[cl * r.max_blocks + atomicAdd(&s_cls[cl], 1)] = b;
             }
         }
@@ -349,16 +349,17 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
             const int tok = tk[k], e = ev[k];
             if (e >= 0) {
                 const int f = r.held ? hrk[k] : atomicAdd(&fill[e], 1);
-                const int pos = start[e] + f;
+                const int pos = start[e] + f, row = r.MB ? f % r.MB : 0;
+                const int pw = r.MB ? pair_word(e, row, min(r.MB, cnt[e] - f + row)) : e;
                 const float wt = wv[k];
                 if (r.staged) {
                     stok[pos] = tok;
                     sw[pos] = wt;
-                    se[pos] = e;
+                    se[pos] = pw;
                 } else {
                     r.pair_tok[pos] = tok;
                     r.pair_w[pos] = wt;
-                    if (r.pair_e) r.pair_e[pos] = e;
+                    if (r.pair_e) r.pair_e[pos] = pw;
                 }
                 r.pair_of[i] = pos;
                 if (r.items && !(r.use_mfma && cnt[e] > r.MR)) {
@@ -441,7 +442,10 @@ __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
             r.pair_tok[pos] = tok;
             r.pair_w[pos] = wt;
             r.pair_of[t] = pos;
-            if (r.pair_e) r.pair_e[pos] = e;
+            if (r.pair_e) {
+                const int row = before % r.MB;
+                r.pair_e[pos] = pair_word(e, row, min(r.MB, cnt - before + row));
+            }
         } else {
             r.pair_of[t] = -1;
         }
@@ -473,7 +477,7 @@ __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
             for (int i = 0; i < 9; ++i) d.tab[i] = ldg(r.tables + (int64_t)i * r.E + e);
             for (int i = 0; i < 6; ++i) d.km[i] = r.kmaps ? ldg(r.kmaps + (int64_t)i * r.E + e) : 0;
             if (r.cls_list) {
-                const int cl = mfma_row_class(d.cnt);
+                const int cl = mfma_row_class(d.cnt, r.MB);
                 r.cls_list[cl * r.max_blocks + atomicAdd(&s_cls[cl], 1)] = block;
             }
         }
@@ -1171,7 +1175,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     r.tables = a.tables;
     r.kmaps = a.kmaps;
     r.use_mfma = use_mfma;
-    r.MB = kMfmaRows;
+    r.MB = a.block_rows;
     r.blocks = blocks;
     r.max_blocks = a.max_blocks;
     r.cls_list = cls;
@@ -1312,7 +1316,7 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     // an expert takes one or two rows) and, with uniform K, batches of up to 16 tokens, up to 32 when the experts
     // are small (H * I <= 2^22), and up to 128 when the MFMA grid would be thin (active experts * I / 128 < 160
     // gate|up workgroups: 8 experts top-2, 128 tokens 116 -> 74 us; 32 experts top-4, 96 tokens 101 -> 87). Other prefill batches: every expert with rows goes to the MFMA kernels in blocks of up to
-    // kMfmaRows rows (MR = 0: no GEMV items). Measured against the MFMA path: 512 experts of 2048 -> 512, top-10,
+    // kWideRows or kMfmaRows rows (MR = 0: no GEMV items). Measured against the MFMA path: 512 experts of 2048 -> 512, top-10,
     // 16 / 20 / 25 tokens 141.5 -> 100.6, 153.5 -> 118.8, 165.6 -> 141.6 us; 16 experts top-9, 16 tokens 90.9 ->
     // 56.0; 8 experts top-8, 32 tokens 117.6 -> 72.5; 129 experts of 4096 -> 1408 with a shared one, 16 tokens
     // 254.6 -> 223.6; one expert of 4096 -> 4096, 32 / 64 tokens 176 -> 77, 210 -> 125; 8 experts top-2, 64 tokens
@@ -1363,6 +1367,7 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     int64_t mi = mfma ? 0 : E + npairs / a.MR;
     if (mi > npairs) mi = npairs;
     a.max_items = (int)mi;
+    a.block_rows = a.Kg > 0 && a.Kd > 0 && a.Kg <= 5 && a.Kd <= 5 ? kWideRows : kMfmaRows;
     a.max_blocks = mfma ? (int)(npairs / kMfmaRows + (E < npairs ? E : npairs) + 1) : 0;
     EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= 65535,
                    "exl3_moe_forward: grid too large");

@@ -336,4 +336,75 @@ struct DirectPipe : TileWords<K, PL> {
     }
 };
 
+// ------------------------------------------------------------------------------------------------ epilogue
+// The 128-point transform of a row spread over four lanes of a quad: lane sub = lane & 3 holds columns
+// 16 i + 4 sub + j of v[i][j]. Bits 0, 1, 4, 5, 6 of the column are registers, bits 2 and 3 the lanes.
+__device__ __forceinline__ void fwht128_quad(f4_t (&v)[8], int lane) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
+        v[i] = f4_t{a + c, b + d, a - c, b - d};
+    }
+#pragma unroll
+    for (int st = 1; st < 8; st *= 2)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (!(i & st)) {
+                const f4_t a = v[i], b = v[i + st];
+                v[i] = a + b;
+                v[i + st] = a - b;
+            }
+    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float x = v[i][j];
+            x = x * s1 + lane_xor<1>(x, lane);
+            x = x * s2 + lane_xor<2>(x, lane);
+            v[i][j] = x;
+        }
+}
+
+// The same over eight lanes: lane sub = lane & 7 holds columns 32 i + 4 sub + j of v[i][j]; bits 0, 1, 5, 6 of the column are
+// registers, bits 2 to 4 the lanes.
+__device__ __forceinline__ void fwht128_oct(f4_t (&v)[4], int lane) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
+        v[i] = f4_t{a + c, b + d, a - c, b - d};
+    }
+    const f4_t a = v[0] + v[1], b = v[0] - v[1], c = v[2] + v[3], d = v[2] - v[3];
+    v[0] = a + c;
+    v[1] = b + d;
+    v[2] = a - c;
+    v[3] = b - d;
+    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f, s4 = lane & 4 ? -1.f : 1.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float x = v[i][j];
+            x = x * s1 + lane_xor<1>(x, lane);
+            x = x * s2 + lane_xor<2>(x, lane);
+            x = x * s4 + lane_xor<4>(x, lane);
+            v[i][j] = x;
+        }
+}
+
+// Floats per row of a 32 x 256 output tile in LDS, column c at c + 16 (c >> 7): the 16-byte reads of the lanes of a row and
+// of the next row hit distinct banks.
+constexpr int kWideCS = 288;
+
+// One row group's accumulators of the workgroup (wave w: columns 64 w .. 64 w + 63) into the tile.
+__device__ __forceinline__ void store_tile(float* C, const f16_t (&acc)[2], int wave, int lane) {
+    const int cl = 64 * wave + (lane & 31) + 16 * (wave >> 1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int r = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        C[r * kWideCS + cl] = acc[0][i];
+        C[r * kWideCS + cl + 32] = acc[1][i];
+    }
+}
+
 }  // namespace exl3

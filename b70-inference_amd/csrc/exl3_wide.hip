@@ -20,38 +20,6 @@ __device__ __forceinline__ bool wide_tile(const LinArgs& a, int& rb, int& nb, in
     return true;
 }
 
-// The 128-point transform of a row spread over four lanes of a quad: lane sub = lane & 3 holds columns
-// 16 i + 4 sub + j of v[i][j]. Bits 0, 1, 4, 5, 6 of the column are registers, bits 2 and 3 the lanes.
-__device__ __forceinline__ void fwht128_quad(f4_t (&v)[8], int lane) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
-        v[i] = f4_t{a + c, b + d, a - c, b - d};
-    }
-#pragma unroll
-    for (int st = 1; st < 8; st *= 2)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (!(i & st)) {
-                const f4_t a = v[i], b = v[i + st];
-                v[i] = a + b;
-                v[i + st] = a - b;
-            }
-    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float x = v[i][j];
-            x = x * s1 + lane_xor<1>(x, lane);
-            x = x * s2 + lane_xor<2>(x, lane);
-            v[i][j] = x;
-        }
-}
-
-constexpr int kWideCS = 288;                         // floats per row of the output tile in LDS: column c at
-                                                     // c + 16 (c >> 7) (a quad's 16-byte reads hit distinct banks)
-
 template <int K, int RG, int NPL>
 __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 ? 3 : 2) : (K <= 5 ? 4 : 3)) void linear_wide_kernel(LinArgs a) {
     constexpr bool kDirect = RG <= 2;
@@ -145,13 +113,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
         if (rg > 0) __syncthreads();
-        const int c0 = 64 * wave + (lane & 31), cl = c0 + 16 * hw;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-            C[r * kWideCS + cl] = acc[rg][0][i];
-            C[r * kWideCS + cl + 32] = acc[rg][1][i];
-        }
+        store_tile(C, acc[rg], wave, lane);
         __syncthreads();
         const int m = 32 * rg + rr;
         if (m >= cnt || half >= nhalf) continue;

@@ -44,7 +44,7 @@ METRIC = "EXL3 MoE layer µs/token + achieved HBM GB/s (% of peak), 1 MI355X"
 HBM_PEAK_GBS = 8000.0
 MFMA_F16_PEAK_TFLOPS = 2500.0
 VALU_PEAK_LANE_OPS = 256 * 64 * 2.4e9           # 256 CUs x 4 SIMDs x 16 lanes per clock x 2.4 GHz
-MFMA_ROWS = 64                                  # the library's MFMA row block (kMfmaRows) and its row classes
+MFMA_ROWS, WIDE_ROWS = 64, 128                  # the library's MFMA row blocks: per-tile K, uniform K (<= 5)
 
 exl3 = importlib.import_module("b70-inference_amd")
 
@@ -292,13 +292,13 @@ class Mlp:
         return cpu_time(lambda: O.gated_mlp(x, *ps, O.ACT_GELU_TANH)), self.M, "one layer call"
 
 
-def mfma_blocks(rows):
-    """Row blocks of one expert with `rows` rows in the MFMA path: up to MFMA_ROWS rows each -> class index
-    (0: <= 16 rows, 1: <= 32, 2: <= 64) per block."""
+def mfma_blocks(rows, block=MFMA_ROWS):
+    """Row blocks of one expert with `rows` rows in the MFMA path: up to `block` rows each -> class index
+    (0: <= block / 4 rows, 1: <= block / 2, 2: <= block) per block."""
     out = []
-    for q in range(0, rows, MFMA_ROWS):
-        c = min(MFMA_ROWS, rows - q)
-        out.append((0 if c <= 16 else 1 if c <= 32 else 2, c))
+    for q in range(0, rows, block):
+        c = min(block, rows - q)
+        out.append((0 if 4 * c <= block else 1 if 2 * c <= block else 2, c))
     return out
 
 
@@ -320,6 +320,7 @@ class MoE:
         self.logits = [torch.randn(M, self.E, device="cuda", generator=g) for _ in range(nrout)]
         self.routing = [exl3.route_softmax_topk(lg, topk, bias) for lg in self.logits]
         self.ids = [ids.cpu() for ids, _ in self.routing]
+        self.block = MFMA_ROWS if t.K_gate == 0 or t.K_down == 0 else WIDE_ROWS
         self.exp_bytes = [[weight_bytes(t.projs[q][e]) for q in range(3)] for e in range(t.E)]
         self.out = torch.empty(M, self.H, dtype=torch.float32, device="cuda")
 
@@ -362,7 +363,7 @@ class MoE:
         for proj, tag in ((0, "gateup"), (2, "down")):
             if name.startswith(f"moe_{tag}_mfma_r"):
                 cl = {"1": 0, "2": 1, "4": 2}[name[-1]]
-                experts = {e: sum(c for k, c in mfma_blocks(r) if k == cl) for e, r in rpe.items()}
+                experts = {e: sum(c for k, c in mfma_blocks(r, self.block) if k == cl) for e, r in rpe.items()}
                 experts = {e: r for e, r in experts.items() if r > 0}
                 rows = sum(experts.values())
                 if proj == 0:      # gate + up weights, xh rows in (two fp16 planes), fp16 down inputs out
@@ -384,7 +385,7 @@ class MoE:
         for per, tag in ((2, "gateup"), (1, "down")):
             if name.startswith(f"moe_{tag}_mfma_r"):
                 cl = {"1": 0, "2": 1, "4": 2}[name[-1]]
-                return per * self.H * self.I * sum(1 for r in rpe.values() for k, _ in mfma_blocks(r) if k == cl)
+                return per * self.H * self.I * sum(1 for r in rpe.values() for k, _ in mfma_blocks(r, self.block) if k == cl)
         return None
 
     def cpu(self, O, np, rows=None):

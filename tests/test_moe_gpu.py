@@ -648,3 +648,33 @@ def test_moe_prefill_hot_experts_many_blocks(exl3, oracle, monkeypatch, Kgu, Kd)
     perm = torch.randperm(M, generator=g)
     c = exl3.moe_forward(x[perm].cuda(), ids[perm].cuda(), w[perm].cuda(), tables)
     assert torch.equal(a[perm.cuda()], c)
+
+
+# rows per expert at the edges of the row classes (32 / 64 / 128 rows; 16 / 32 / 64 for K > 5 or a per-tile K), several
+# blocks of one expert among them, and an expert without rows
+CLASS_ROWS = (1, 31, 32, 33, 0, 64, 65, 128, 129, 260, 17)
+
+
+@pytest.mark.parametrize("Kgu,Kd", [(1, 1), (2, 3), (5, 4), (5, 6), (8, 3), (7, 8), (3, 0), (0, 2), (0, 6)])
+def test_moe_row_classes(exl3, oracle, monkeypatch, Kgu, Kd):
+    """Row blocks of every class, at a width with a half column block (H = 384), for both fragment orders and for a
+    uniform projection beside a per-tile one (0), against the oracle."""
+    monkeypatch.setenv("EXL3MI_MOE_MFMA", "1")
+    from moe_util import gpu_proj, make_proj, oracle_proj
+    E, H, I = len(CLASS_ROWS), 384, 256
+    pt = ((1, 2, 5), (0.4, 0.4, 0.2))
+    cpu = [[make_proj(H, I, Kgu, 9100 + 10 * e, None if Kgu else pt) for e in range(E)],
+           [make_proj(H, I, Kgu, 9101 + 10 * e, None if Kgu else pt) for e in range(E)],
+           [make_proj(I, H, Kd, 9102 + 10 * e, None if Kd else pt) for e in range(E)]]
+    tables = exl3.ExpertTables(*[[gpu_proj(exl3, c, "cuda") for c in q] for q in cpu])
+    orc = [tuple(oracle_proj(oracle, q[e]) for q in cpu) for e in range(E)]
+    M = 300
+    ids = torch.full((M, E), -1, dtype=torch.int32)
+    g = torch.Generator().manual_seed(9200 + Kgu)
+    for e, n in enumerate(CLASS_ROWS):
+        ids[torch.randperm(M, generator=g)[:n], e] = e
+    w = torch.rand(M, E, generator=g)
+    x = torch.randn(M, H, generator=g).half()
+    for dt in (torch.float32, torch.float16):
+        y, ref = _run(exl3, oracle, tables, orc, x, ids, w, out_dtype=dt)
+        assert max_rel(y, ref) <= MAX_REL, dt
