@@ -206,6 +206,9 @@ struct LinArgs {
     int m, k, n, nblk;
     int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits, 128-blocks per split
     int f32;
+    const int64_t* tab;                              // not null: an expert's addresses (ItemDesc::tab), its down projection
+                                                     // in place of tr and svh
+    const int32_t* rowmap;                           // not null: output row of each row
 };
 
 typedef void (*lin_fn)(LinArgs);

@@ -822,6 +822,129 @@ static int fork3(hipStream_t st, F launch) {
     return EXL3_OK;
 }
 
+// Split-K finish: wave per (row, 128-column block): the split partials summed in split order (eight splits' loads in
+// flight at a time), Hadamard, * svh / sqrt(128).
+__global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = blockIdx.x * 4 + wave;
+    if (row >= a.m) return;
+    const int col = blockIdx.y * 128 + lane;
+    const uint16_t* sv = (a.tab ? reinterpret_cast<const uint16_t*>(a.tab[8]) : a.svh) + col;
+    const float s0 = h2f(ldg(sv)) * kRsqrt128, s1 = h2f(ldg(sv + 64)) * kRsqrt128;
+    const float* q = a.part + (size_t)row * a.n + col;
+    const size_t ps = (size_t)a.m * a.n;
+    float v0 = 0.f, v1 = 0.f;
+    for (int p0 = 0; p0 < a.P; p0 += 8) {
+        float t0[8], t1[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int pp = p0 + i < a.P ? p0 + i : a.P - 1;
+            t0[i] = ldg(q + pp * ps);
+            t1[i] = ldg(q + pp * ps + 64);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (p0 + i < a.P) {
+                v0 += t0[i];
+                v1 += t1[i];
+            }
+    }
+    fwht128_wave(v0, v1, lane);
+    linear_store(a, a.rowmap ? a.rowmap[row] : row, col, v0 * s0, v1 * s1);
+}
+
+
+
+lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
+
+struct LinPlan {
+    int RG, P, bps;                                  // row groups of 32 per block, k-splits, 128-blocks of k per split
+};
+
+// Row block and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
+// each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
+// workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
+// and that kernel's launch. Fitted to 878 measured points at K = 4 (1024 x 4096 .. 5376 x 21504, 16 .. 1024 rows, 1 .. 16
+// splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
+// blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
+// the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
+// `rg` > 0 fixes the row block, `cap` bounds the splits.
+static int linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, LinPlan* best) {
+    const int nblk = (int)(k / 128);
+    int dev = 0, cus = 0, occ[4];
+    EXL3_CHECK_HIP(hipGetDevice(&dev));
+    EXL3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    for (int g = 0; g < 4; ++g) {
+        int resident = 0;
+        const int rc = resident_blocks((const void*)linear_wide_pick(1 << g, S, K), 256, &resident);
+        if (rc) return rc;
+        occ[g] = resident / cus < 1 ? 1 : resident / cus > 4 ? 4 : resident / cus;
+    }
+    static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
+                                        {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
+    static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
+    const int64_t ncb = (n + 255) / 256;
+    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
+    *best = {rg > 0 ? rg : 1, 1, nblk};
+    float tb = 1e30f;
+    for (int g = 0; g < 4; ++g) {
+        if (rg > 0 && rg != 1 << g) continue;
+        const int64_t tiles = (m + (32 << g) - 1) / (32 << g) * ncb;
+        for (int p = 1; p <= pmax && p <= cap; ++p) {
+            const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
+            if (P != p) continue;
+            const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
+            const float mb = (float)P * (float)m * (float)n * 4e-6f;
+            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
+                      kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
+            if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
+            if (t < tb) {
+                tb = t;
+                *best = {1 << g, P, bps};
+            }
+        }
+    }
+    return EXL3_OK;
+}
+
+// k-splits of a dense MLP's down projection (m rows in blocks of `block` rows), at most `cap`.
+int dense_down_splits(int64_t m, int64_t n, int64_t k, int K, int block, int64_t cap, int* P) {
+    LinPlan pl;
+    const int rc = linear_plan(m, n, k, 1, K, block / 32, cap, &pl);
+    *P = pl.P;
+    return rc;
+}
+
+// The down projection of a dense MLP: the gate|up kernel's output blocks are a dense linear's input. Unlike the grouped
+// kernel's, its k is split (5376 <- 21504 at 397 rows: 84 workgroups of 672 steps without).
+static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
+    LinArgs l = {};
+    l.xh = reinterpret_cast<const _Float16*>(a.abuf);
+    l.xsum = a.asum;
+    l.S = 1;
+    l.tab = a.blocks[0].tab;                                       // (address only: device memory)
+    l.rowmap = a.pair_tok;
+    l.out = a.out;
+    l.out_ld = a.out_ld;
+    l.f32 = a.out_f32;
+    l.part = a.y;
+    l.m = a.M;
+    l.k = a.I;
+    l.n = a.H;
+    l.nblk = a.I / 128;
+    l.nrb = (a.M + a.block_rows - 1) / a.block_rows;
+    l.ncb = (a.H + 255) / 256;
+    l.bps = (l.nblk + a.dense_P - 1) / a.dense_P;
+    l.P = (l.nblk + l.bps - 1) / l.bps;
+    const int64_t nx = ((int64_t)l.nrb * l.ncb * l.P + 7) / 8 * 8;
+    if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: grid too large");
+    EXL3_LAUNCH("mlp_down_wide", linear_wide_pick(a.block_rows / 32, 1, a.Kd), dim3((unsigned)nx), dim3(256), 0, st, l);
+    if (l.P > 1)
+        EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, dim3((unsigned)((l.m + 3) / 4), (unsigned)(l.n / 128)),
+                    dim3(256), 0, st, l);
+    return EXL3_OK;
+}
+
 int launch_gateup_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);     // exl3_moe_wide.hip (uniform K)
 int launch_down_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);
 int launch_moe_combine(const MoeArgs& a, hipStream_t st);
@@ -844,87 +967,15 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
         } else if (const int e = launch_gateup_wide(a, cl, grid_gu, s)) {
             return e;
         }
+        if (a.dense_P > 0) return EXL3_OK;             // after the classes have joined
         if (a.Kd > 0) return launch_down_wide(a, cl, grid_dn, s);
         mfma_fn dn = rga == 4 ? down_mix_kernel<4> : rga == 2 ? down_mix_kernel<2> : down_mix_kernel<1>;
         EXL3_LAUNCH(rga == 4 ? "moe_down_mfma_r4" : rga == 2 ? "moe_down_mfma_r2" : "moe_down_mfma_r1", dn, grid_dn,
                     dim3(256), 0, s, a);
         return EXL3_OK;
     });
-    return rc || a.Kd == 0 ? rc : launch_moe_combine(a, st);
-}
-
-// Split-K finish: wave per (row, 128-column block): the split partials summed in split order (eight splits' loads in
-// flight at a time), Hadamard, * svh / sqrt(128).
-__global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int row = blockIdx.x * 4 + wave;
-    if (row >= a.m) return;
-    const int col = blockIdx.y * 128 + lane;
-    const float s0 = h2f(ldg(a.svh + col)) * kRsqrt128, s1 = h2f(ldg(a.svh + col + 64)) * kRsqrt128;
-    const float* q = a.part + (size_t)row * a.n + col;
-    const size_t ps = (size_t)a.m * a.n;
-    float v0 = 0.f, v1 = 0.f;
-    for (int p0 = 0; p0 < a.P; p0 += 8) {
-        float t0[8], t1[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int pp = p0 + i < a.P ? p0 + i : a.P - 1;
-            t0[i] = ldg(q + pp * ps);
-            t1[i] = ldg(q + pp * ps + 64);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (p0 + i < a.P) {
-                v0 += t0[i];
-                v1 += t1[i];
-            }
-    }
-    fwht128_wave(v0, v1, lane);
-    linear_store(a, row, col, v0 * s0, v1 * s1);
-}
-
-
-
-lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
-
-// Row block (RG groups of 32 rows) and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
-// each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
-// workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
-// and that kernel's launch. Fitted to 878 measured points at K = 4 (1024 x 4096 .. 5376 x 21504, 16 .. 1024 rows, 1 .. 16
-// splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
-// blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
-// the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
-struct LinPlan {
-    int RG, P, bps;
-};
-static LinPlan linear_plan(int64_t m, int64_t n, int nblk, const int (&occ)[4], int cus) {
-    static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
-                                        {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
-    static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
-    const int64_t ncb = (n + 255) / 256;
-    // at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the scratch of the partials)
-    const int r0 = m <= 16 ? 16 : m <= 32 ? 32 : 64;
-    const int64_t t0 = (m + r0 - 1) / r0 * ncb, cap = ((m <= 32 ? 3 : 2) * (int64_t)cus + t0 - 1) / t0;
-    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
-    LinPlan best = {1, 1, nblk};
-    float tb = 1e30f;
-    for (int g = 0; g < 4; ++g) {
-        const int64_t tiles = (m + (32 << g) - 1) / (32 << g) * ncb;
-        for (int p = 1; p <= pmax && p <= cap; ++p) {
-            const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
-            if (P != p) continue;
-            const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
-            const float mb = (float)P * (float)m * (float)n * 4e-6f;
-            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
-                      kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
-            if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
-            if (t < tb) {
-                tb = t;
-                best = {1 << g, P, bps};
-            }
-        }
-    }
-    return best;
+    if (rc || a.Kd == 0) return rc;
+    return a.dense_P > 0 ? launch_dense_down(a, st) : launch_moe_combine(a, st);
 }
 
 // Dense linear on MFMA (m > the GEMV's rows per pass): input transform, blocks of 32 .. 256 rows x 256 columns and, with
@@ -935,16 +986,12 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     const int nblk = (int)(k / 128);
     if (m > 0x7FFFFFFF / 64 || k > 0x7FFFFFFF || n > 0x7FFFFFFF || nblk > 65535)
         return fail(EXL3_ERR_INVALID, "exl3_gemm: shape too large");
-    int dev = 0, cus = 0, occ[4];
-    EXL3_CHECK_HIP(hipGetDevice(&dev));
-    EXL3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    for (int g = 0; g < 4; ++g) {
-        int resident = 0;
-        const int rc = resident_blocks((const void*)linear_wide_pick(1 << g, S, K), 256, &resident);
-        if (rc) return rc;
-        occ[g] = resident / cus < 1 ? 1 : resident / cus > 4 ? 4 : resident / cus;
-    }
-    LinPlan pl = linear_plan(m, n, nblk, occ, cus);
+    // at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the scratch of the partials)
+    const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
+    const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
+    LinPlan pl;
+    int rc = linear_plan(m, n, k, S, K, 0, ((m <= 32 ? 768 : 512) + ts - 1) / ts, &pl);
+    if (rc) return rc;
     const int force = env_int("EXL3MI_LINEAR_BLOCK", 0);           // row groups of 32 per block: 1, 2, 4 or 8
     if (force == 1 || force == 2 || force == 4 || force == 8) pl.RG = force;
     const int R = 32 * pl.RG;
@@ -954,7 +1001,7 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
         pl.bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
         pl.P = (nblk + pl.bps - 1) / pl.bps;
     }
-    LinArgs a;
+    LinArgs a = {};
     a.m = (int)m;
     a.k = (int)k;
     a.n = (int)n;
@@ -966,7 +1013,7 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     const size_t xh_b = carve_size((size_t)S * m * k, 2), xs_b = carve_size((size_t)S * m * nblk, 4);
     const size_t part_b = a.P > 1 ? carve_size((size_t)a.P * m * n, 4) : 0;
     Workspace ws;
-    int rc = workspace(xh_b + xs_b + part_b, 0, st, &ws);
+    rc = workspace(xh_b + xs_b + part_b, 0, st, &ws);
     if (rc) return rc;
     Carve cv{ws.scratch, ws.scratch_bytes};
     _Float16* xh = cv.take<_Float16>((size_t)S * m * k);

@@ -116,7 +116,10 @@ struct MoeArgs {
     // intermediates (workspace)
     uint16_t* abuf;                    // [pairs][I] fp16, Hadamard-domain down input (MFMA rows at uniform down K: per
                                        // block in block_unit order)
-    float* y;                          // [pairs][H] fp32, weighted expert outputs
+    float* y;                          // [pairs][H] fp32, weighted expert outputs (dense_P > 0: [dense_P][M][H] down
+                                       // partials)
+    int dense_P;                       // > 0: one expert takes every token with weight 1 (a dense MLP) on the MFMA
+                                       // path: k-splits of its down projection, which runs as a dense linear
     float* part_gu;
     int* cnt_gu;
     int P_gu, nblk_h;

@@ -1102,6 +1102,7 @@ static moe_fn down_select(int K, int MR, bool pl) {
 }
 
 int launch_moe_mfma(const MoeArgs& a, hipStream_t st);          // exl3_mfma.hip
+int dense_down_splits(int64_t m, int64_t n, int64_t k, int K, int block, int64_t cap, int* P);
 bool moe_fused_ok(const MoeArgs& a);                            // exl3_moe_fused.hip
 bool moe_fused_take(const MoeArgs& a);
 double moe_expected_items(const MoeArgs& m, int mr);
@@ -1120,7 +1121,9 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     Workspace ws;
     const size_t n_gu = (size_t)max_items * nbI, n_d = (size_t)max_items * nbH;
     const bool use_mfma = a.max_blocks > 0;
-    size_t bytes = carve_size(1, 4) + carve_size(max_items, sizeof(ItemDesc)) +
+    size_t y_elems = (size_t)npairs * a.H;
+    const auto scratch = [&] {
+        return carve_size(1, 4) + carve_size(max_items, sizeof(ItemDesc)) +
                    carve_size(a.max_blocks, sizeof(ItemDesc)) +
                    (use_mfma ? carve_size(npairs * 2 * a.H, 2) + carve_size(npairs * 2 * (a.H / 128), 4) +
                                    carve_size(npairs, 4) +
@@ -1128,8 +1131,20 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
                              : 0) +
                    carve_size(npairs * 2, 4) + carve_size(npairs, 4) +
                    carve_size(a.M, 4) +
-                   carve_size(npairs * a.I, 2) + carve_size(npairs * a.H, 4) +
+                   carve_size(npairs * a.I, 2) + carve_size(y_elems, 4) +
                    carve_size(n_gu * a.P_gu * 2 * MR * 128, 4) + carve_size(n_d * a.P_d * MR * 128, 4);
+    };
+    if (use_mfma && a.E == 1 && a.topk == 0 && a.shared == 0 && a.Kg > 0 && a.Kd > 0) {
+        // a dense MLP: its down projection as a dense linear; under stream capture with the splits that the scratch holds
+        const size_t room = workspace_room(st);
+        for (int cap = 8;; cap = a.dense_P - 1) {
+            const int rc = dense_down_splits(a.M, a.H, a.I, a.Kd, a.block_rows, cap, &a.dense_P);
+            if (rc) return rc;
+            y_elems = (size_t)a.dense_P * npairs * a.H;
+            if (a.dense_P == 1 || scratch() <= room) break;
+        }
+    }
+    const size_t bytes = scratch();
     const size_t n_tok = (size_t)a.M * nbH;
     int rc = workspace(bytes, n_gu + n_d + n_tok, st, &ws);
     if (rc) return rc;
@@ -1152,7 +1167,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.pair_w = c.take<float>(npairs);
     a.tok_nvalid = c.take<int>(a.M);
     a.abuf = c.take<uint16_t>(npairs * a.I);
-    a.y = c.take<float>(npairs * a.H);
+    a.y = c.take<float>(y_elems);
     a.part_gu = c.take<float>(n_gu * a.P_gu * 2 * MR * 128);
     a.part_d = c.take<float>(n_d * a.P_d * MR * 128);
     if (!a.part_d) return fail(EXL3_ERR_INVALID, "moe: workspace carve failed");

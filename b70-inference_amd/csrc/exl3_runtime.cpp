@@ -172,6 +172,14 @@ int workspace(size_t bytes, size_t ncounters, hipStream_t st, Workspace* out) {
     return EXL3_OK;
 }
 
+size_t workspace_room(hipStream_t st) {
+    if (!capturing(st)) return SIZE_MAX;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    return g_ws[dev].scratch_bytes;
+}
+
 int spin_limit() { return env_int("EXL3MI_SPIN_LIMIT", 1 << 20); }
 
 namespace {

@@ -42,6 +42,9 @@ struct Workspace {
 };
 int workspace(size_t bytes, size_t ncounters, hipStream_t stream, Workspace* out);
 
+// Scratch bytes a call on `stream` can take now: what the workspace holds while the stream is being captured, else no limit.
+size_t workspace_room(hipStream_t stream);
+
 // Wait bound of the kernels' cross-workgroup waits (polls): EXL3MI_SPIN_LIMIT, default 2^20. A small value makes a
 // wait give up early (failure-path tests); every kernel still exits.
 int spin_limit();

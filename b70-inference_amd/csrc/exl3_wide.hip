@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     L.nsteps = nkb * 4;
     L.lane = lane;
     L.setup_w(tn, reinterpret_cast<uint32_t*>(smem + kStage) + wave * 8 * Pipe::TS,
-              a.tr + (size_t)kb0 * 8 * tn * (8 * K), [&](int pair) {
+              (a.tab ? reinterpret_cast<const uint32_t*>(a.tab[6]) : a.tr) + (size_t)kb0 * 8 * tn * (8 * K), [&](int pair) {
                   const int ct = nb * 16 + 4 * wave + 2 * pair;
                   return ct < tn ? ct : tn - 2;      // a last half block: in-bounds loads, results unused
               });
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     const int col = nb * 256 + 128 * half + 4 * sub;
     float sd[8][4];
     {
-        const uint16_t* sv = a.svh + (half < nhalf ? col : col - 128);
+        const uint16_t* sv = (a.tab ? reinterpret_cast<const uint16_t*>(a.tab[8]) : a.svh) + (half < nhalf ? col : col - 128);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -117,6 +117,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
         __syncthreads();
         const int m = 32 * rg + rr;
         if (m >= cnt || half >= nhalf) continue;
+        const int64_t orow = a.rowmap ? a.rowmap[r0 + m] : r0 + m;
         const float sx = kMul1C2 * rsum[NPL > 1 ? half : 0][m];
         f4_t v[8];
 #pragma unroll
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
         }
         fwht128_quad(v, lane);
         if (a.f32) {
-            float* o = reinterpret_cast<float*>(a.out) + (int64_t)(r0 + m) * a.out_ld + col;
+            float* o = reinterpret_cast<float*>(a.out) + orow * a.out_ld + col;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 f4_t y;
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
                 }
             }
         } else {
-            uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + (int64_t)(r0 + m) * a.out_ld + col;
+            uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + orow * a.out_ld + col;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 uint32_t y[4];

@@ -678,3 +678,37 @@ def test_moe_row_classes(exl3, oracle, monkeypatch, Kgu, Kd):
     for dt in (torch.float32, torch.float16):
         y, ref = _run(exl3, oracle, tables, orc, x, ids, w, out_dtype=dt)
         assert max_rel(y, ref) <= MAX_REL, dt
+
+
+@pytest.mark.parametrize("K,M,out_dtype", [(4, 150, torch.float32), (3, 300, torch.float16), (6, 200, torch.float32)])
+def test_gated_mlp_prefill_split_down(exl3, oracle, K, M, out_dtype):
+    """A dense MLP on the MFMA path with the k of its down projection split, a ragged last row block, into output rows
+    wider than H; replays of a captured call give the eager result."""
+    from importlib import import_module
+    L_ = import_module("b70-inference_amd._lib")
+    H, I = 384, 2048
+    tables, orc = make_experts(exl3, oracle, 1, H, I, K, K, 9400 + K)
+    x = torch.randn(M, H, generator=torch.Generator().manual_seed(9410 + K)).half()
+    ref = oracle.moe_layer(x.numpy(), [], np.zeros((M, 0), np.int32), np.zeros((M, 0), np.float32), 0, 0.0, orc[0])
+    ids, w = torch.empty(M, 0, dtype=torch.int32).cuda(), torch.empty(M, 0).cuda()
+    buf = torch.full((M, H + 5), 7.0, dtype=out_dtype, device="cuda")
+    xc = x.cuda()
+
+    def run():
+        L_.check(L_.lib().exl3_moe_forward(
+            L_.ptr(xc), H, M, H, I, L_.ptr(ids), L_.ptr(w), 0, 1, L_.ptr(tables.tables), None, K, K, K, 0, 0.0, 0,
+            L_.ptr(buf), H + 5, 1 if out_dtype == torch.float32 else 0, L_.stream_of(xc)), "exl3_moe_forward")
+
+    run()
+    torch.cuda.synchronize()
+    assert max_rel(buf[:, :H].float().cpu().numpy(), ref) <= MAX_REL
+    assert (buf[:, H:] == 7.0).all()
+    eager = buf.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run()
+    for _ in range(3):
+        buf.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(buf, eager)
