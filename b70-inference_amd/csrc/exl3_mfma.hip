@@ -51,57 +51,56 @@ __host__ __device__ constexpr bool had_sign_neg(int ks, int nb) {
     return (((ks & 1) & ((nb >> 1) & 1)) ^ (((ks >> 1) & 1) & ((nb >> 2) & 1))) != 0;
 }
 
-// fp16(H128(fp16(x * s)) / sqrt(128)) of one wave's 16 rows: xv holds the rows' x in A-fragment layout (lane L: row
-// L & 15, columns 32 ks + 8 (L >> 4) + j), sv points at s + 8 (L >> 4) (16-byte loads when vs). The results go to the
-// wave's LDS tile (16 x 128 fp16) and part[i] gets the sum of the fp16 results of row 4 (L >> 4) + i over this lane's
-// 8 columns (the caller reduces over the 16 lanes of a row).
-__device__ __forceinline__ void had16_rows(const h8_t (&xv)[4], const h8_t (&sg)[4], const h8_t (&F)[2], int lane,
-                                           _Float16 (*tile)[136], float (&part)[4]) {
+// fp16(H128(A) / sqrt(128)) of one wave's 16 rows, A = fp16(x * s) in A-fragment layout (lane L: row L & 15, columns
+// 32 ks + 8 (L >> 4) + j). The results go to the wave's LDS tile (16 x 128 fp16) and part[i] gets the sum of the fp16
+// results of row 4 (L >> 4) + i over this lane's 8 columns (the caller reduces over the 16 lanes of a row). The signs of
+// the base fragments sit in B (F, then -F), and four output tiles are in flight at a time: few enough registers for four
+// waves per SIMD in the prefill's input transform, which waits on two memory round trips per job.
+__device__ __forceinline__ void had16_rows(const h8_t (&A)[4], const h8_t (&F)[4], int lane, _Float16 (*tile)[136],
+                                           float (&part)[4]) {
     const int m = lane & 15, g = lane >> 4;
-    h8_t A[4], An[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        A[ks] = xv[ks] * sg[ks];
-        An[ks] = -A[ks];
-    }
-    f4_t acc[8];
-#pragma unroll
-    for (int nb = 0; nb < 8; ++nb) {
-        acc[nb] = f4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had_sign_neg(ks, nb) ? An[ks] : A[ks], F[nb & 1],
-                                                             acc[nb], 0, 0, 0);
-    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) part[i] = 0.f;
 #pragma unroll
-    for (int nb = 0; nb < 8; ++nb)
+    for (int n0 = 0; n0 < 8; n0 += 4) {
+        f4_t acc[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const _Float16 h = (_Float16)(acc[nb][i] * kRsqrt128);
-            part[i] += (float)h;
-            tile[4 * g + i][16 * nb + m] = h;
+        for (int n = 0; n < 4; ++n) {
+            acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    A[ks], F[(n & 1) + (had_sign_neg(ks, n0 + n) ? 2 : 0)], acc[n], 0, 0, 0);
         }
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const _Float16 h = (_Float16)(acc[n][i] * kRsqrt128);
+                part[i] += (float)h;
+                tile[4 * g + i][16 * (n0 + n) + m] = h;
+            }
+    }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// the signs from sv + 32 ks (16-byte loads when vs)
-__device__ __forceinline__ void had16_rows(const h8_t (&xv)[4], const uint16_t* sv, bool vs, const h8_t (&F)[2],
-                                           int lane, _Float16 (*tile)[136], float (&part)[4]) {
-    h8_t sg[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) sg[ks] = load_h8(sv + 32 * ks, vs);
-    had16_rows(xv, sg, F, lane, tile, part);
+__device__ __forceinline__ void had_fragments(int lane, h8_t (&F)[4]) {
+    F[0] = had_fragment(lane, 0);
+    F[1] = had_fragment(lane, 1);
+    F[2] = -F[0];
+    F[3] = -F[1];
 }
 
-// Sum of v over the 16 lanes of a row (lanes with equal L >> 4).
+// Sum of v over the 16 lanes of a row (lanes with equal L >> 4): quads, then the mirrored lane of the half row and row.
 __device__ __forceinline__ float row16_sum(float v) {
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    v += __shfl_xor(v, 4);
-    v += __shfl_xor(v, 8);
+#define EXL3_ROW_ADD(ctrl) \
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false))
+    EXL3_ROW_ADD(0xB1);
+    EXL3_ROW_ADD(0x4E);
+    EXL3_ROW_ADD(0x141);
+    EXL3_ROW_ADD(0x140);
+#undef EXL3_ROW_ADD
     return v;
 }
 
@@ -113,7 +112,7 @@ __device__ __forceinline__ float row16_sum(float v) {
 // the reference's fp16(x * suh)), the Hadamard is 8 output tiles x 4 k-steps of v_mfma_f32_16x16x32_f16 against the
 // two base fragments (fp32 accumulation of exact +-x products), and the sums of the fp16-rounded outputs reduce over
 // the 16 lanes of a row.
-__global__ __launch_bounds__(256) void pairs_had_kernel(MoeArgs a) {
+__global__ __launch_bounds__(256, 4) void pairs_had_kernel(MoeArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 s_out[4][16][136];    // per wave: 16 rows x 128 (+ pad)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nblk = a.H / 128, np = a.M * a.slots;
@@ -147,11 +146,17 @@ __global__ __launch_bounds__(256) void pairs_had_kernel(MoeArgs a) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) sg[proj][ks] = load_h8(sv + 32 * ks, vs);
     }
-    const h8_t F[2] = {had_fragment(lane, 0), had_fragment(lane, 1)};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        sg[0][ks] = xv[ks] * sg[0][ks];                 // A fragments
+        sg[1][ks] = xv[ks] * sg[1][ks];
+    }
+    h8_t F[4];
+    had_fragments(lane, F);
 #pragma unroll
     for (int proj = 0; proj < 2; ++proj) {
         float part[4];
-        had16_rows(xv, sg[proj], F, lane, s_out[wave], part);
+        had16_rows(sg[proj], F, lane, s_out[wave], part);
         if (a.Kg > 0) {                                 // per block in block_unit order: lane = row, 16-byte units
             const int row = pair_row(pw), cnt = pair_block_rows(pw);
             u32x4_t* dst = reinterpret_cast<u32x4_t*>(a.xh + ((size_t)(r0 + m - row) * 2 + (size_t)proj * cnt) * a.H);
@@ -775,10 +780,14 @@ __global__ __launch_bounds__(256) void linear_had_kernel(const uint16_t* __restr
     h8_t xv[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) xv[ks] = load_h8(xr + 32 * ks, vx);
-    const h8_t F[2] = {had_fragment(lane, 0), had_fragment(lane, 1)};
     const uint16_t* sv = suh + kb * 128 + 8 * g;
+    const bool vs = ((uintptr_t)sv & 15) == 0;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) xv[ks] = xv[ks] * load_h8(sv + 32 * ks, vs);
+    h8_t F[4];
+    had_fragments(lane, F);
     float part[4];
-    had16_rows(xv, sv, ((uintptr_t)sv & 15) == 0, F, lane, s_out[wave], part);
+    had16_rows(xv, F, lane, s_out[wave], part);
     const int b0 = r0 / R * R, cnt = m - b0 < R ? m - b0 : R;    // the block that holds the wave's rows
     u32x4_t* dst = reinterpret_cast<u32x4_t*>(xh + (size_t)b0 * k);
 #pragma unroll

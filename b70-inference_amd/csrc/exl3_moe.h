@@ -57,10 +57,11 @@ struct RouteArgs {
     void* out;
     int64_t out_ld;
     int out_f32, H;
-    int held;                          // align_kernel: each thread holds its (at most 8) pairs in registers and
+    int held;                          // align_kernel: each thread holds its (at most 8 or 12) pairs in registers and
                                        // counts the tokens' valid slots in LDS (M more ints of dynamic LDS)
-    int staged;                        // align_kernel (held): the sorted pair arrays are built in LDS (3 * M * slots
-                                       // more ints) and written out with coalesced stores
+    int staged;                        // align_kernel (held): the sorted order is built in LDS (M * slots more ints;
+                                       // 2: and the weights, as many floats) and the pair arrays written out from it
+                                       // with coalesced stores
 };
 
 constexpr int kFusedRouteMaxE = 512;    // logits per row that the fused layer's in-layer routing handles (8 per lane)

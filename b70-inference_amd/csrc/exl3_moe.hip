@@ -187,11 +187,12 @@ __device__ __forceinline__ void write_desc(ItemDesc& d, int e, int p0, int cnt, 
     d.km[5] = v[14];
 }
 
-// The memory round trips are the kernel's cost, so with held pairs (np <= 8 * 1024) every load is issued at the start:
+// The memory round trips are the kernel's cost, so with held pairs (np <= HP * 1024) every load is issued at the start:
 // the thread's pairs (kept in registers for the scatter) and its first expert's table entries; the tokens' valid
 // slots are counted in LDS with the experts' rows instead of reloading each token's slots, and the counting atomics'
 // values (a pair's rank within its expert) place the pairs, so the scatter needs no second atomic. The barriers order
 // LDS only: the tables written here are read by later kernels, so their stores drain behind the rest of the kernel.
+template <int HP>
 __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     extern __shared__ int sm[];
     int* cnt = sm;                 // [E]
@@ -201,17 +202,17 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     int* nbl = sm + 4 * r.E;       // [E] MFMA blocks of the expert, then their first index
     int* tmp = sm + 5 * r.E;       // [1024]
     int* tokn = sm + 5 * r.E + 1024;   // [M] valid slots per token (held pairs)
-    int* stok = tokn + r.M;            // [M * slots] x 3: pair_tok, pair_w, pair_e in sorted order (staged)
-    float* sw = reinterpret_cast<float*>(stok + r.M * r.slots);
-    int* se = stok + 2 * r.M * r.slots;
+    int* sperm = tokn + r.M;           // [M * slots] expert << 21 | slot << 14 | token of the pairs in sorted order
+                                       // (staged: at most 12 Ki tokens, 127 slots, 2 Ki experts)
+    float* sw = reinterpret_cast<float*>(sperm + r.M * r.slots);   // [M * slots] their weights (staged == 2)
     __shared__ int s_cls[3];
     const int t = threadIdx.x, T = blockDim.x;
     if (t < 3) s_cls[t] = 0;
     const int np = r.M * r.slots;
     const int mr = r.MR > 0 ? r.MR : 1;   // MR == 0: every expert with rows is an MFMA expert (no GEMV items)
-    int hev[8], htk[8];
-    float hwv[8];
-    if (r.held) load_pairs<8>(r, t, T, np, hev, hwv, htk);
+    int hev[HP], htk[HP];
+    float hwv[HP];
+    if (r.held) load_pairs<HP>(r, t, T, np, hev, hwv, htk);
     // this thread's first expert's table entries (index clamped: unconditional loads)
     int64_t tb0[9], km0[6];
     {
@@ -228,10 +229,10 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     if (r.held)
         for (int m = t; m < r.M; m += T) tokn[m] = 0;
     lds_barrier();
-    int hrk[8];                        // held pairs: each pair's rank within its expert (the counting atomic's value)
+    int hrk[HP];                       // held pairs: each pair's rank within its expert (the counting atomic's value)
     if (r.held) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < HP; ++k)
             if (hev[k] >= 0) {
                 hrk[k] = atomicAdd(&cnt[hev[k]], 1);
                 atomicAdd(&tokn[htk[k]], 1);
@@ -329,55 +330,75 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
         }
     }
     lds_barrier();
-    for (int i0 = t; i0 < np; i0 += 8 * T) {
-        int ev[8], tk[8];
-        float wv[8];
-        if (r.held) {                  // i0 == t: the pairs loaded at the start
+    // pair_e of the expert's f-th pair
+    const auto sorted_word = [&](int e, int f) {
+        const int row = f & (r.MB - 1);        // MB is a power of two (or 0: no blocks)
+        return r.MB ? pair_word(e, row, min(r.MB, cnt[e] - f + row)) : e;
+    };
+    const auto place = [&](int i, int tok, int e, float wt, int f) {      // flat pair i: its expert's f-th
+        if (e < 0) {
+            r.pair_of[i] = -1;
+            return;
+        }
+        const int pos = start[e] + f;
+        if (r.staged) {
+            sperm[pos] = (int)((uint32_t)e << 21 | (uint32_t)(i - tok * r.slots) << 14 | (uint32_t)tok);
+            if (r.staged == 2) sw[pos] = wt;
+        } else {
+            r.pair_tok[pos] = tok;
+            r.pair_w[pos] = wt;
+            if (r.pair_e) r.pair_e[pos] = sorted_word(e, f);
+        }
+        r.pair_of[i] = pos;
+        if (r.items && !(r.use_mfma && cnt[e] > r.MR)) {
+            ItemDesc& d = r.items[nch[e] + f / mr];
+            d.tok[f % mr] = tok;
+            d.w[f % mr] = wt;
+        }
+    };
+    if (r.held) {                      // the pairs loaded at the start
+#pragma unroll
+        for (int k = 0; k < HP; ++k) {
+            const int i = t + k * T;
+            if (i < np) place(i, htk[k], hev[k], hwv[k], hev[k] >= 0 ? hrk[k] : 0);
+        }
+    } else {
+        for (int i0 = t; i0 < np; i0 += 8 * T) {
+            int ev[8], tk[8];
+            float wv[8];
+            load_pairs<8>(r, i0, T, np, ev, wv, tk);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                ev[k] = hev[k];
-                wv[k] = hwv[k];
-                tk[k] = htk[k];
-            }
-        } else {
-            load_pairs<8>(r, i0, T, np, ev, wv, tk);
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int i = i0 + k * T;
-            if (i >= np) break;
-            const int tok = tk[k], e = ev[k];
-            if (e >= 0) {
-                const int f = r.held ? hrk[k] : atomicAdd(&fill[e], 1);
-                const int pos = start[e] + f, row = r.MB ? f % r.MB : 0;
-                const int pw = r.MB ? pair_word(e, row, min(r.MB, cnt[e] - f + row)) : e;
-                const float wt = wv[k];
-                if (r.staged) {
-                    stok[pos] = tok;
-                    sw[pos] = wt;
-                    se[pos] = pw;
-                } else {
-                    r.pair_tok[pos] = tok;
-                    r.pair_w[pos] = wt;
-                    if (r.pair_e) r.pair_e[pos] = pw;
-                }
-                r.pair_of[i] = pos;
-                if (r.items && !(r.use_mfma && cnt[e] > r.MR)) {
-                    ItemDesc& d = r.items[nch[e] + f / mr];
-                    d.tok[f % mr] = tok;
-                    d.w[f % mr] = wt;
-                }
-            } else {
-                r.pair_of[i] = -1;
+                const int i = i0 + k * T;
+                if (i < np) place(i, tk[k], ev[k], wv[k], ev[k] >= 0 ? atomicAdd(&fill[ev[k]], 1) : 0);
             }
         }
     }
     if (r.staged) {                    // the sorted pairs out of LDS, coalesced
         lds_barrier();
-        for (int q = t; q < nvalid; q += T) {
-            r.pair_tok[q] = stok[q];
-            r.pair_w[q] = sw[q];
-            if (r.pair_e) r.pair_e[q] = se[q];
+        for (int q0 = t; q0 < nvalid; q0 += 4 * T) {
+            int v[4];
+            float w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int q = min(q0 + k * T, nvalid - 1);
+                v[k] = sperm[q];
+                if (r.staged == 2) {
+                    w[k] = sw[q];
+                } else {
+                    const int tok = v[k] & 0x3FFF, j = v[k] >> 14 & 0x7F;
+                    w[k] = r.topk > 0 ? ldg(r.tw + tok * r.topk + (j < r.topk ? j : 0)) : 1.0f;
+                    if (j >= r.topk) w[k] = 1.0f;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int q = q0 + k * T, e = (int)((uint32_t)v[k] >> 21);
+                if (q >= nvalid) break;
+                r.pair_tok[q] = v[k] & 0x3FFF;
+                r.pair_w[q] = w[k];
+                if (r.pair_e) r.pair_e[q] = sorted_word(e, q - start[e]);
+            }
         }
     }
 }
@@ -1013,13 +1034,18 @@ int launch_align(const RouteArgs& r, hipStream_t st) {
         EXL3_LAUNCH("moe_align", align_small_kernel, dim3(1), dim3(kAlignSmall), 0, st, r);
         return EXL3_OK;
     }
-    // held pairs when every pair fits the threads' registers and the token counts fit the 64 KB of dynamic LDS
+    // held pairs when every pair fits the threads' registers (12 per thread: more was not needed by a 1024-token top-10
+    // batch, whose pairs were read three times without) and the token counts fit the 64 KB of dynamic LDS
     RouteArgs h = r;
+    const int64_t np = (int64_t)r.M * r.slots;
     const size_t lds0 = align_lds_bytes(r.E), ldsh = lds0 + (size_t)r.M * sizeof(int);
-    h.held = (int64_t)r.M * r.slots <= 8 * 1024 && ldsh <= 65536;
-    const size_t ldss = ldsh + 3 * (size_t)r.M * r.slots * sizeof(int);
-    h.staged = h.held && ldss + 256 <= 65536;        // (room for the kernel's static LDS)
-    EXL3_LAUNCH("moe_align", align_kernel, dim3(1), dim3(1024), h.staged ? ldss : h.held ? ldsh : lds0, st, h);
+    h.held = np <= 12 * 1024 && ldsh <= 65536;
+    const size_t ldss = ldsh + (size_t)np * sizeof(int);
+    const size_t room = 65536 - 256;                 // (less the kernel's static LDS)
+    h.staged = !h.held || ldss > room || r.slots > 127 ? 0 : ldss + (size_t)np * sizeof(float) > room ? 1 : 2;
+    const size_t lds = h.staged == 2 ? ldss + (size_t)np * sizeof(float) : h.staged ? ldss : h.held ? ldsh : lds0;
+    if (np <= 8 * 1024) EXL3_LAUNCH("moe_align", align_kernel<8>, dim3(1), dim3(1024), lds, st, h);
+    else EXL3_LAUNCH("moe_align", align_kernel<12>, dim3(1), dim3(1024), lds, st, h);
     return EXL3_OK;
 }
 

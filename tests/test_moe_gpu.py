@@ -712,3 +712,33 @@ def test_gated_mlp_prefill_split_down(exl3, oracle, K, M, out_dtype):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(buf, eager)
+
+
+@pytest.mark.parametrize("M,k,E,shared", [
+    (1000, 7, 37, -1),      # held 8 per thread, order and weights built in LDS
+    (1024, 10, 512, -1),    # 12 per thread, the weights read again for the copy-out
+    (1117, 10, 64, 63),     # the same with a shared expert (11 slots: 12287 pairs), whose weight is 1
+    (3100, 4, 37, -1),      # more than 12 per thread: reloaded per phase
+    (60, 130, 200, -1),     # more slots than the packed order holds
+])
+def test_align_tables_large(exl3, M, k, E, shared):
+    """Every way the 1024-thread kernel keeps and orders its pairs: pairs grouped by expert, each with its token and
+    weight, the inverse map consistent."""
+    ids, w = _ids_w(M, k, E - (shared >= 0), 1300 + M, dup=True, inactive=True)
+    counts, ptok, pw, pof = exl3.moe_align(ids.cuda(), w.cuda(), E, shared=shared)
+    counts, ptok, pw, pof = (t.cpu().numpy() for t in (counts, ptok, pw, pof))
+    flat, wf = ids.numpy(), w.numpy()
+    if shared >= 0:
+        flat = np.concatenate([flat, np.full((M, 1), shared, np.int32)], 1)
+        wf = np.concatenate([wf, np.ones((M, 1), np.float32)], 1)
+    slots = flat.shape[1]
+    flat, wf = flat.reshape(-1), wf.reshape(-1)
+    assert np.array_equal(counts, np.bincount(flat[flat >= 0], minlength=E))
+    starts = np.concatenate([[0], np.cumsum(counts)[:-1]])
+    valid = np.nonzero(flat >= 0)[0]
+    pof = pof.reshape(-1)
+    assert (pof[flat < 0] == -1).all()
+    pv, e = pof[valid], flat[valid]
+    assert ((starts[e] <= pv) & (pv < starts[e] + counts[e])).all()
+    assert (ptok[pv] == valid // slots).all() and (pw[pv] == wf[valid]).all()
+    assert np.unique(pv).size == pv.size == counts.sum()
