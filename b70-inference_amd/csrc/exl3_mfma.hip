@@ -809,25 +809,26 @@ __global__ __launch_bounds__(256) void linear_had_kernel(const uint16_t* __restr
 // ------------------------------------------------------------------------------------------------ host
 typedef void (*mfma_fn)(MoeArgs);
 
+// Row classes run concurrently: the largest on the caller's stream, the others on the side streams.
 template <typename F>
-static int fork3(hipStream_t st, F launch) {
-    // the three row classes run concurrently: 4 row groups on the caller's stream, 2 and 1 on the side streams
+static int fork_classes(hipStream_t st, int ncls, F launch) {
+    if (ncls == 1) return launch(0, st);
     if (env_int("EXL3MI_SERIAL_CLASSES", 0)) {            // every class on the caller's stream, one after another
-        int rc = 0;
-        if ((rc = launch(4, st)) || (rc = launch(2, st)) || (rc = launch(1, st))) return rc;
+        for (int cl = ncls - 1; cl >= 0; --cl)
+            if (const int rc = launch(cl, st)) return rc;
         return EXL3_OK;
     }
     AuxStreams ax;
     int rc = aux_streams(&ax);
     if (rc) return rc;
     EXL3_CHECK_HIP(hipEventRecord(ax.ev[0], st));
-    EXL3_CHECK_HIP(hipStreamWaitEvent(ax.s[0], ax.ev[0], 0));
-    EXL3_CHECK_HIP(hipStreamWaitEvent(ax.s[1], ax.ev[0], 0));
-    if ((rc = launch(4, st)) || (rc = launch(2, ax.s[0])) || (rc = launch(1, ax.s[1]))) return rc;
-    EXL3_CHECK_HIP(hipEventRecord(ax.ev[1], ax.s[0]));
-    EXL3_CHECK_HIP(hipEventRecord(ax.ev[2], ax.s[1]));
-    EXL3_CHECK_HIP(hipStreamWaitEvent(st, ax.ev[1], 0));
-    EXL3_CHECK_HIP(hipStreamWaitEvent(st, ax.ev[2], 0));
+    for (int i = 0; i < ncls - 1; ++i) EXL3_CHECK_HIP(hipStreamWaitEvent(ax.s[i], ax.ev[0], 0));
+    for (int cl = ncls - 1; cl >= 0; --cl)
+        if ((rc = launch(cl, cl == ncls - 1 ? st : ax.s[ncls - 2 - cl]))) return rc;
+    for (int i = 0; i < ncls - 1; ++i) {
+        EXL3_CHECK_HIP(hipEventRecord(ax.ev[1 + i], ax.s[i]));
+        EXL3_CHECK_HIP(hipStreamWaitEvent(st, ax.ev[1 + i], 0));
+    }
     return EXL3_OK;
 }
 
@@ -954,9 +955,12 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
     return EXL3_OK;
 }
 
-int launch_gateup_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);     // exl3_moe_wide.hip (uniform K)
-int launch_down_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st);
+int launch_gateup_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st);  // exl3_moe_wide.hip (uniform K)
+int launch_down_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st);
 int launch_moe_combine(const MoeArgs& a, hipStream_t st);
+// the same for a uniform projection beside a per-tile-K one (classes of 16, 32 and 64 rows)
+int launch_gateup_class(const MoeArgs& a, int cl, hipStream_t st);
+int launch_down_class(const MoeArgs& a, int cl, hipStream_t st);
 
 // The grouped GEMM of one layer call: the input transform, then per row class gate|up followed by down on that class's
 // stream (a class's down blocks read only the down inputs its own gate|up blocks wrote; tokens whose slots span
@@ -967,17 +971,24 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
     EXL3_CHECK_ARG(had_jobs / 4 < 0x7FFFFFFF, "exl3_moe_forward: too many rows");
     EXL3_LAUNCH("moe_pairs_had", pairs_had_kernel, dim3((unsigned)((had_jobs + 3) / 4)), dim3(256), 0, st, a);
     const dim3 grid_gu(nxb * (a.I / 128)), grid_dn(nxb * ((a.H / 128 + 1) / 2));
-    const int rc = fork3(st, [&](int rga, hipStream_t s) -> int {
-        const int cl = rga == 4 ? 2 : rga == 2 ? 1 : 0;
+    const bool wide = a.Kg > 0 && a.Kd > 0;
+    // uniform K: a block of more than 32 rows leaves room for at most one per 33 rows (65 where smaller remainders are cut)
+    const int np = a.M * a.slots, nbig = np / (a.block_rows > 64 && a.dense_P == 0 ? 65 : 33) + 1;
+    const int rc = fork_classes(st, wide ? (a.block_rows > 32 ? 2 : 1) : 3, [&](int cl, hipStream_t s) -> int {
+        if (wide) {
+            const int n = cl == 1 && nbig < a.max_blocks ? nbig : a.max_blocks;
+            const int e = launch_gateup_wide(a, cl, n, s);
+            return e || a.dense_P > 0 ? e : launch_down_wide(a, cl, n, s);   // (dense: after the classes have joined)
+        }
+        const int rga = 1 << cl;                       // row groups of 16
         if (a.Kg == 0) {
             mfma_fn gu = rga == 4 ? gateup_mix_kernel<4> : rga == 2 ? gateup_mix_kernel<2> : gateup_mix_kernel<1>;
             EXL3_LAUNCH(rga == 4 ? "moe_gateup_mfma_r4" : rga == 2 ? "moe_gateup_mfma_r2" : "moe_gateup_mfma_r1", gu,
                         grid_gu, dim3(256), 0, s, a);
-        } else if (const int e = launch_gateup_wide(a, cl, grid_gu, s)) {
+        } else if (const int e = launch_gateup_class(a, cl, s)) {
             return e;
         }
-        if (a.dense_P > 0) return EXL3_OK;             // after the classes have joined
-        if (a.Kd > 0) return launch_down_wide(a, cl, grid_dn, s);
+        if (a.Kd > 0) return launch_down_class(a, cl, s);
         mfma_fn dn = rga == 4 ? down_mix_kernel<4> : rga == 2 ? down_mix_kernel<2> : down_mix_kernel<1>;
         EXL3_LAUNCH(rga == 4 ? "moe_down_mfma_r4" : rga == 2 ? "moe_down_mfma_r2" : "moe_down_mfma_r1", dn, grid_dn,
                     dim3(256), 0, s, a);

@@ -7,13 +7,34 @@ namespace exl3 {
 
 constexpr int kMoeMaxExperts = 2048;   // expert tables per layer (routed + shared); the align kernel keeps 5 ints each in LDS
 constexpr int kMoeSmallRows = 8;       // experts with at most this many rows in a call take the GEMV kernels
-constexpr int kMfmaRows = 64;          // row block of the MFMA grouped GEMM
-constexpr int kWideRows = 128;         // the same with uniform K <= 5 (gate|up and down; above, 128 rows would spill)
+constexpr int kMfmaRows = 64;          // row block of the MFMA grouped GEMM with a per-tile K
+constexpr int kWideRows = 128;         // largest row block with uniform K
 
-// Row class of an MFMA block by the call's row block MB (class 0: <= MB / 4 rows, 1: <= MB / 2, 2: <= MB): each class runs
-// its own kernel instance sized for its rows, so that small blocks get the register budget (and occupancy) of a small
-// block.
-__host__ __device__ constexpr int mfma_row_class(int cnt, int MB) { return 4 * cnt <= MB ? 0 : 2 * cnt <= MB ? 1 : 2; }
+// How an expert's rows are cut into MFMA blocks. Per-tile K: blocks of MB = 64 rows, row classes of up to 16, 32 and 64 rows
+// (each runs its own kernel instance, so that small blocks get the register budget and occupancy of a small block).
+// Uniform K (wide): blocks of MB = 32, 64 or 128 rows, classes 0: up to 32 rows, 1: more. With MB = 128 a remainder of up to
+// 64 rows is cut into blocks of 32 (two 32-row blocks cost what one 128-row block does) unless `whole`: then it stays one
+// block (a dense MLP, whose down projection takes its rows in blocks of MB).
+constexpr int kRowClasses = 3;
+struct BlockCut {
+    int MB, wide, whole;
+    // number of blocks of an expert with c rows
+    __host__ __device__ int count(int c) const {
+        const int full = c / MB, rem = c - full * MB;
+        return full + (split(rem) ? (rem + 31) / 32 : rem > 0);
+    }
+    // block of the f-th of c rows: its first row and row count
+    __host__ __device__ void locate(int c, int f, int& first, int& cnt) const {
+        const int full = c / MB * MB, rem = c - full;
+        const int sz = f < full || !split(rem) ? MB : 32;
+        first = f < full ? f & ~(MB - 1) : full + (sz == 32 ? (f - full) & ~31 : 0);
+        cnt = c - first < sz ? c - first : sz;
+    }
+    __host__ __device__ int row_class(int cnt) const { return wide ? cnt > 32 : cnt <= 16 ? 0 : cnt <= 32 ? 1 : 2; }
+
+private:
+    __host__ __device__ bool split(int rem) const { return MB > 64 && !whole && rem <= 64; }
+};
 
 // A sorted pair's expert, its row in its MFMA block and the block's rows, in one word.
 static_assert(kMoeMaxExperts <= 1 << 11 && kWideRows <= 1 << 7 && kMfmaRows <= 1 << 7, "pair word");
@@ -43,11 +64,12 @@ struct RouteArgs {
     int max_items;
     const int64_t* tables;             // [9][E] (read when items are built)
     const int64_t* kmaps;              // [6][E] or null
-    int use_mfma, MB;                  // experts with more than MR rows -> blocks of MB rows for the MFMA kernels
+    int use_mfma;                      // experts with more than MR rows -> blocks for the MFMA kernels
+    BlockCut cut;                      // (MB a power of two; 1 without blocks)
     ItemDesc* blocks;                  // [max_blocks]
     int max_blocks;
-    int* cls_list;                     // optional [3][max_blocks]: block indices by row class
-    int* cls_cnt;                      // [3]
+    int* cls_list;                     // optional [kRowClasses][max_blocks]: block indices by row class
+    int* cls_cnt;                      // [kRowClasses]
     int* pair_tok;
     float* pair_w;
     int* pair_of;
@@ -57,11 +79,6 @@ struct RouteArgs {
     void* out;
     int64_t out_ld;
     int out_f32, H;
-    int held;                          // align_kernel: each thread holds its (at most 8 or 12) pairs in registers and
-                                       // counts the tokens' valid slots in LDS (M more ints of dynamic LDS)
-    int staged;                        // align_kernel (held): the sorted order is built in LDS (M * slots more ints;
-                                       // 2: and the weights, as many floats) and the pair arrays written out from it
-                                       // with coalesced stores
 };
 
 constexpr int kFusedRouteMaxE = 512;    // logits per row that the fused layer's in-layer routing handles (8 per lane)
@@ -100,8 +117,8 @@ struct MoeArgs {
     const ItemDesc* items;
     const ItemDesc* blocks;            // MFMA row blocks (cnt == 0 past the last)
     int max_blocks;
-    const int* cls_list;               // [3][max_blocks] block indices by row class
-    const int* cls_cnt;                // [3] blocks per class
+    const int* cls_list;               // [kRowClasses][max_blocks] block indices by row class
+    const int* cls_cnt;                // [kRowClasses] blocks per class
     _Float16* xh;                      // [pairs][2][H] transformed gate / up inputs of MFMA rows; uniform gate|up K:
                                        // per block [2][cnt * H] in block_unit order (exl3_mfma.h)
     float* xsum;                       // [pairs][2][H / 128] block sums of xh (the MFMA rows' affine term)
@@ -111,7 +128,7 @@ struct MoeArgs {
     int* pair_of;
     int* pair_e;                       // [pairs] pair_word of each pair in sorted order, -1 past the valid pairs
                                        // (MFMA path)
-    int block_rows;                    // row block of the call's MFMA blocks (kMfmaRows or kWideRows)
+    int block_rows;                    // row block of the call's MFMA blocks (BlockCut::MB)
     int* tok_nvalid;                   // [M] valid slots per token
     int* cnt_tok;                      // [M][H/128] combine arrival counters
     // intermediates (workspace)

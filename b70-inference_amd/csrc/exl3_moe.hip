@@ -192,7 +192,10 @@ __device__ __forceinline__ void write_desc(ItemDesc& d, int e, int p0, int cnt, 
 // slots are counted in LDS with the experts' rows instead of reloading each token's slots, and the counting atomics'
 // values (a pair's rank within its expert) place the pairs, so the scatter needs no second atomic. The barriers order
 // LDS only: the tables written here are read by later kernels, so their stores drain behind the rest of the kernel.
-template <int HP>
+// HP > 0: the pairs are held (at most HP per thread) and the sorted order is built in LDS: ST 2: the three pair arrays, ST 1:
+// packed into one word per pair, the weights read again. HP = 0: pairs reloaded per phase, stored directly. Instances rather
+// than branches: a cold single-workgroup kernel pays for its code size.
+template <int HP, int ST>
 __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     extern __shared__ int sm[];
     int* cnt = sm;                 // [E]
@@ -203,16 +206,18 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     int* tmp = sm + 5 * r.E;       // [1024]
     int* tokn = sm + 5 * r.E + 1024;   // [M] valid slots per token (held pairs)
     int* sperm = tokn + r.M;           // [M * slots] expert << 21 | slot << 14 | token of the pairs in sorted order
-                                       // (staged: at most 12 Ki tokens, 127 slots, 2 Ki experts)
-    float* sw = reinterpret_cast<float*>(sperm + r.M * r.slots);   // [M * slots] their weights (staged == 2)
-    __shared__ int s_cls[3];
+                                       // (ST 1: at most 12 Ki tokens, 127 slots, 2 Ki experts)
+    float* sw = reinterpret_cast<float*>(sperm + r.M * r.slots);   // ST 2: sperm holds the tokens, and beside it
+    int* se = sperm + 2 * r.M * r.slots;                           // the weights and the pair words, M * slots each
+    __shared__ int s_cls[kRowClasses];
     const int t = threadIdx.x, T = blockDim.x;
-    if (t < 3) s_cls[t] = 0;
+    if (t < kRowClasses) s_cls[t] = 0;
     const int np = r.M * r.slots;
     const int mr = r.MR > 0 ? r.MR : 1;   // MR == 0: every expert with rows is an MFMA expert (no GEMV items)
-    int hev[HP], htk[HP];
-    float hwv[HP];
-    if (r.held) load_pairs<HP>(r, t, T, np, hev, hwv, htk);
+    constexpr int HN = HP > 0 ? HP : 1;
+    int hev[HN], htk[HN];
+    float hwv[HN];
+    if constexpr (HP > 0) load_pairs<HN>(r, t, T, np, hev, hwv, htk);
     // this thread's first expert's table entries (index clamped: unconditional loads)
     int64_t tb0[9], km0[6];
     {
@@ -226,11 +231,11 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
         cnt[e] = 0;
         fill[e] = 0;
     }
-    if (r.held)
+    if constexpr (HP > 0)
         for (int m = t; m < r.M; m += T) tokn[m] = 0;
     lds_barrier();
-    int hrk[HP];                       // held pairs: each pair's rank within its expert (the counting atomic's value)
-    if (r.held) {
+    int hrk[HN];                       // held pairs: each pair's rank within its expert (the counting atomic's value)
+    if constexpr (HP > 0) {
 #pragma unroll
         for (int k = 0; k < HP; ++k)
             if (hev[k] >= 0) {
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
         const bool big = r.use_mfma && c > r.MR;
         start[e] = c;
         nch[e] = big ? 0 : (c + mr - 1) / mr;
-        nbl[e] = big ? (c + r.MB - 1) / r.MB : 0;
+        nbl[e] = big ? r.cut.count(c) : 0;
     }
     lds_barrier();
     int nvalid, nitems, nblocks;
@@ -286,14 +291,15 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
 #pragma unroll
             for (int i = 0; i < 6; ++i) km[i] = 0;
         }
-        for (int q = 0, b = nbl[e]; big && q * r.MB < c; ++q, ++b) {
-            ItemDesc& d = r.blocks[b];
-            const int dc = min(r.MB, c - q * r.MB);
-            write_desc(d, e, start[e] + q * r.MB, dc, tb, km);
+        for (int f = 0, b = nbl[e]; big && f < c; ++b) {
+            int first, dc;
+            r.cut.locate(c, f, first, dc);
+            write_desc(r.blocks[b], e, start[e] + first, dc, tb, km);
             if (r.cls_list) {
-                const int cl = mfma_row_class(dc, r.MB);
+                const int cl = r.cut.row_class(dc);
                 r.cls_list[cl * r.max_blocks + atomicAdd(&s_cls[cl], 1)] = b;
             }
+            f = first + dc;
         }
         for (int q = 0, it = nch[e]; !big && q * mr < c; ++q, ++it) {
             write_desc(r.items[it], e, start[e] + q * mr, min(mr, c - q * mr), tb, km);
@@ -305,11 +311,11 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
         for (int b = nblocks + t; b < r.max_blocks; b += T) r.blocks[b].cnt = 0;
     if (t == 0 && r.n_items) r.n_items[0] = nitems;
     lds_barrier();
-    if (t < 3 && r.cls_cnt) r.cls_cnt[t] = s_cls[t];
+    if (t < kRowClasses && r.cls_cnt) r.cls_cnt[t] = s_cls[t];
     if (r.tok_nvalid) {
         for (int tok = t; tok < r.M; tok += T) {
             int nv = 0;
-            if (r.held) {
+            if constexpr (HP > 0) {
                 nv = tokn[tok];
             } else {
                 for (int j0 = 0; j0 < r.slots; j0 += 8) {
@@ -332,8 +338,9 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
     lds_barrier();
     // pair_e of the expert's f-th pair
     const auto sorted_word = [&](int e, int f) {
-        const int row = f & (r.MB - 1);        // MB is a power of two (or 0: no blocks)
-        return r.MB ? pair_word(e, row, min(r.MB, cnt[e] - f + row)) : e;
+        int first, dc;
+        r.cut.locate(cnt[e], f, first, dc);
+        return pair_word(e, f - first, dc);
     };
     const auto place = [&](int i, int tok, int e, float wt, int f) {      // flat pair i: its expert's f-th
         if (e < 0) {
@@ -341,9 +348,12 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
             return;
         }
         const int pos = start[e] + f;
-        if (r.staged) {
+        if constexpr (ST == 2) {
+            sperm[pos] = tok;
+            sw[pos] = wt;
+            se[pos] = sorted_word(e, f);
+        } else if constexpr (ST == 1) {
             sperm[pos] = (int)((uint32_t)e << 21 | (uint32_t)(i - tok * r.slots) << 14 | (uint32_t)tok);
-            if (r.staged == 2) sw[pos] = wt;
         } else {
             r.pair_tok[pos] = tok;
             r.pair_w[pos] = wt;
@@ -356,7 +366,7 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
             d.w[f % mr] = wt;
         }
     };
-    if (r.held) {                      // the pairs loaded at the start
+    if constexpr (HP > 0) {            // the pairs loaded at the start
 #pragma unroll
         for (int k = 0; k < HP; ++k) {
             const int i = t + k * T;
@@ -374,22 +384,25 @@ __global__ __launch_bounds__(1024) void align_kernel(RouteArgs r) {
             }
         }
     }
-    if (r.staged) {                    // the sorted pairs out of LDS, coalesced
+    if constexpr (ST > 0) {            // the sorted pairs out of LDS, coalesced
         lds_barrier();
-        for (int q0 = t; q0 < nvalid; q0 += 4 * T) {
+        if constexpr (ST == 2) {
+            for (int q = t; q < nvalid; q += T) {
+                r.pair_tok[q] = sperm[q];
+                r.pair_w[q] = sw[q];
+                if (r.pair_e) r.pair_e[q] = se[q];
+            }
+            return;
+        }
+        for (int q0 = t; q0 < nvalid; q0 += 4 * T) {           // the weights read again
             int v[4];
             float w[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const int q = min(q0 + k * T, nvalid - 1);
-                v[k] = sperm[q];
-                if (r.staged == 2) {
-                    w[k] = sw[q];
-                } else {
-                    const int tok = v[k] & 0x3FFF, j = v[k] >> 14 & 0x7F;
-                    w[k] = r.topk > 0 ? ldg(r.tw + tok * r.topk + (j < r.topk ? j : 0)) : 1.0f;
-                    if (j >= r.topk) w[k] = 1.0f;
-                }
+                v[k] = sperm[min(q0 + k * T, nvalid - 1)];
+                const int tok = v[k] & 0x3FFF, j = v[k] >> 14 & 0x7F;
+                w[k] = r.topk > 0 ? ldg(r.tw + tok * r.topk + (j < r.topk ? j : 0)) : 1.0f;
+                if (j >= r.topk) w[k] = 1.0f;
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -412,9 +425,9 @@ constexpr int kAlignSmall = 256;
 __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
     __shared__ int s_e[kAlignSmall], s_pos[kAlignSmall];
     __shared__ uint8_t s_lead[kAlignSmall], s_blead[kAlignSmall];
-    __shared__ int s_cls[3];
+    __shared__ int s_cls[kRowClasses];
     const int t = threadIdx.x;
-    if (t < 3) s_cls[t] = 0;
+    if (t < kRowClasses) s_cls[t] = 0;
     const int np = r.M * r.slots;
     const int mr = r.MR > 0 ? r.MR : 1;   // MR == 0: every expert with rows is an MFMA expert (no GEMV items)
     int e = -1, tok = 0;
@@ -439,7 +452,9 @@ __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
     const int pos = below + before;
     const bool big = e >= 0 && r.use_mfma && cnt > r.MR;
     const bool lead = e >= 0 && !big && before % mr == 0;
-    const bool blead = big && before % r.MB == 0;
+    int bfirst = 0, bcnt = 0;
+    if (e >= 0) r.cut.locate(cnt, before, bfirst, bcnt);
+    const bool blead = big && before == bfirst;
     s_pos[t] = e >= 0 ? pos : 0x7FFFFFFF;
     s_lead[t] = lead;
     s_blead[t] = blead;
@@ -463,10 +478,7 @@ __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
             r.pair_tok[pos] = tok;
             r.pair_w[pos] = wt;
             r.pair_of[t] = pos;
-            if (r.pair_e) {
-                const int row = before % r.MB;
-                r.pair_e[pos] = pair_word(e, row, min(r.MB, cnt - before + row));
-            }
+            if (r.pair_e) r.pair_e[pos] = pair_word(e, before - bfirst, bcnt);
         } else {
             r.pair_of[t] = -1;
         }
@@ -494,18 +506,18 @@ __global__ __launch_bounds__(kAlignSmall) void align_small_kernel(RouteArgs r) {
             ItemDesc& d = r.blocks[block];
             d.e = e;
             d.p0 = pos;
-            d.cnt = min(r.MB, cnt - before);
+            d.cnt = bcnt;
             for (int i = 0; i < 9; ++i) d.tab[i] = ldg(r.tables + (int64_t)i * r.E + e);
             for (int i = 0; i < 6; ++i) d.km[i] = r.kmaps ? ldg(r.kmaps + (int64_t)i * r.E + e) : 0;
             if (r.cls_list) {
-                const int cl = mfma_row_class(d.cnt, r.MB);
+                const int cl = r.cut.row_class(d.cnt);
                 r.cls_list[cl * r.max_blocks + atomicAdd(&s_cls[cl], 1)] = block;
             }
         }
         for (int b = nblocks + t; b < r.max_blocks; b += kAlignSmall) r.blocks[b].cnt = 0;
     }
     __syncthreads();
-    if (t < 3 && r.cls_cnt) r.cls_cnt[t] = s_cls[t];
+    if (t < kRowClasses && r.cls_cnt) r.cls_cnt[t] = s_cls[t];
     if (r.counts)
         for (int x = t; x < r.E; x += kAlignSmall) {
             int c = 0;
@@ -1034,18 +1046,16 @@ int launch_align(const RouteArgs& r, hipStream_t st) {
         EXL3_LAUNCH("moe_align", align_small_kernel, dim3(1), dim3(kAlignSmall), 0, st, r);
         return EXL3_OK;
     }
-    // held pairs when every pair fits the threads' registers (12 per thread: more was not needed by a 1024-token top-10
-    // batch, whose pairs were read three times without) and the token counts fit the 64 KB of dynamic LDS
-    RouteArgs h = r;
+    // held pairs (8 or 12 per thread: a 1024-token top-10 batch read its pairs three times without) when the token counts
+    // and the sorted order fit the 64 KB of dynamic LDS (less the kernel's static LDS)
     const int64_t np = (int64_t)r.M * r.slots;
-    const size_t lds0 = align_lds_bytes(r.E), ldsh = lds0 + (size_t)r.M * sizeof(int);
-    h.held = np <= 12 * 1024 && ldsh <= 65536;
-    const size_t ldss = ldsh + (size_t)np * sizeof(int);
-    const size_t room = 65536 - 256;                 // (less the kernel's static LDS)
-    h.staged = !h.held || ldss > room || r.slots > 127 ? 0 : ldss + (size_t)np * sizeof(float) > room ? 1 : 2;
-    const size_t lds = h.staged == 2 ? ldss + (size_t)np * sizeof(float) : h.staged ? ldss : h.held ? ldsh : lds0;
-    if (np <= 8 * 1024) EXL3_LAUNCH("moe_align", align_kernel<8>, dim3(1), dim3(1024), lds, st, h);
-    else EXL3_LAUNCH("moe_align", align_kernel<12>, dim3(1), dim3(1024), lds, st, h);
+    const size_t lds0 = align_lds_bytes(r.E), room = 65536 - 256, ldsh = lds0 + (size_t)r.M * sizeof(int);
+    if (np <= 8 * 1024 && ldsh + 3 * (size_t)np * sizeof(int) <= room)
+        EXL3_LAUNCH("moe_align", (align_kernel<8, 2>), dim3(1), dim3(1024), ldsh + 3 * (size_t)np * sizeof(int), st, r);
+    else if (np <= 12 * 1024 && r.slots <= 127 && ldsh + (size_t)np * sizeof(int) <= room)
+        EXL3_LAUNCH("moe_align", (align_kernel<12, 1>), dim3(1), dim3(1024), ldsh + (size_t)np * sizeof(int), st, r);
+    else
+        EXL3_LAUNCH("moe_align", (align_kernel<0, 0>), dim3(1), dim3(1024), lds0, st, r);
     return EXL3_OK;
 }
 
@@ -1153,7 +1163,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
                    carve_size(a.max_blocks, sizeof(ItemDesc)) +
                    (use_mfma ? carve_size(npairs * 2 * a.H, 2) + carve_size(npairs * 2 * (a.H / 128), 4) +
                                    carve_size(npairs, 4) +
-                                   carve_size(npairs * (a.I / 128), 4) + carve_size(3 * (size_t)a.max_blocks + 3, 4)
+                                   carve_size(npairs * (a.I / 128), 4) + carve_size(kRowClasses * ((size_t)a.max_blocks + 1), 4)
                              : 0) +
                    carve_size(npairs * 2, 4) + carve_size(npairs, 4) +
                    carve_size(a.M, 4) +
@@ -1184,9 +1194,9 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.xsum = use_mfma ? c.take<float>(npairs * 2 * (a.H / 128)) : nullptr;
     a.asum = use_mfma ? c.take<float>(npairs * (a.I / 128)) : nullptr;
     a.pair_e = use_mfma ? c.take<int>(npairs) : nullptr;
-    int* cls = use_mfma ? c.take<int>(3 * (size_t)a.max_blocks + 3) : nullptr;
+    int* cls = use_mfma ? c.take<int>(kRowClasses * ((size_t)a.max_blocks + 1)) : nullptr;
     a.cls_list = cls;
-    a.cls_cnt = cls ? cls + 3 * (size_t)a.max_blocks : nullptr;
+    a.cls_cnt = cls ? cls + kRowClasses * (size_t)a.max_blocks : nullptr;
     int* pb = c.take<int>(npairs * 2);
     a.pair_tok = pb;
     a.pair_of = pb + npairs;
@@ -1216,11 +1226,11 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     r.tables = a.tables;
     r.kmaps = a.kmaps;
     r.use_mfma = use_mfma;
-    r.MB = a.block_rows;
+    r.cut = {a.block_rows, a.Kg > 0 && a.Kd > 0, a.dense_P > 0};
     r.blocks = blocks;
     r.max_blocks = a.max_blocks;
     r.cls_list = cls;
-    r.cls_cnt = cls ? cls + 3 * (size_t)a.max_blocks : nullptr;
+    r.cls_cnt = cls ? cls + kRowClasses * (size_t)a.max_blocks : nullptr;
     r.pair_tok = a.pair_tok;
     r.pair_w = a.pair_w;
     r.pair_of = a.pair_of;
@@ -1408,9 +1418,18 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     int64_t mi = mfma ? 0 : E + npairs / a.MR;
     if (mi > npairs) mi = npairs;
     a.max_items = (int)mi;
-    a.block_rows = a.Kg > 0 && a.Kd > 0 && a.Kg <= 5 && a.Kd <= 5 ? kWideRows : kMfmaRows;
-    a.max_blocks = mfma ? (int)(npairs / kMfmaRows + (E < npairs ? E : npairs) + 1) : 0;
-    EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= 65535,
+    // Row block with uniform K: 32 (one class, one launch per projection) up to 64 tokens, 160 where experts take few rows:
+    // forking the launches by class costs more there (10 to 25 us) than decoding the experts with more rows again; 64 where an expert takes 28 to 64
+    // rows on average (and for K > 5, where 128 rows would spill), else 128. Per 32-k step a workgroup of 32 / 64 / 128 rows
+    // takes 0.21 / 0.28 / 0.41 us.
+    const bool wide = a.Kg > 0 && a.Kd > 0;
+    const double mean = (double)npairs / (double)E;
+    a.block_rows = !wide ? kMfmaRows : E > 1 && (M <= 64 || (M <= 160 && mean <= 8)) ? 32 : (mean > 28 && mean <= 64) || a.Kg > 5 || a.Kd > 5 ? 64 : kWideRows;
+    if (const int rb = env_int("EXL3MI_MOE_BLOCK", 0); wide && (rb == 32 || rb == 64 || (rb == 128 && a.Kg <= 5 && a.Kd <= 5)))
+        a.block_rows = rb;
+    a.max_blocks = mfma ? (int)(npairs / (wide ? 32 : kMfmaRows) + (E < npairs ? E : npairs) + 1) : 0;
+    EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= (wide ? 1 << 21 : 65535) &&
+                       (int64_t)(a.max_blocks + 8) * (a.I > a.H ? a.I / 128 : a.H / 128) < 0x7FFFFFFF,
                    "exl3_moe_forward: grid too large");
     return moe_decode_path(a, npairs, st);
 }
@@ -1534,6 +1553,7 @@ int exl3_moe_align(const int32_t* topk_ids, const float* topk_w, int64_t M, int6
     r.E = (int)E;
     r.shared = (int)shared;
     r.MR = 1;
+    r.cut = {1, 0, 0};
     r.counts = counts;
     r.pair_tok = pair_tok;
     r.pair_w = pair_w;

@@ -15,6 +15,8 @@
 
 namespace exl3 {
 
+// RG: row groups of 32 in a block. Every class accumulates and reduces in the same order, so a row's result does not depend
+// on the class its block falls into.
 // Waves per SIMD the kernels are compiled for (no spills in the loop).
 template <int K, int RG>
 constexpr int moe_wide_occ() {
@@ -41,14 +43,12 @@ __device__ __forceinline__ const ItemDesc* moe_block(const MoeArgs& a, int cl, i
     return a.blocks + a.cls_list[cl * a.max_blocks + idx];
 }
 
-template <int RG>
-__device__ __forceinline__ void zero_acc(f16_t (&acc)[RG][2]) {
+template <int G>
+__device__ __forceinline__ void zero_acc(f16_t (&acc)[G][2]) {
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg)
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-        for (int np = 0; np < 2; ++np)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[rg][np][i] = 0.f;
+        for (int n = 0; n < 2; ++n) acc[g][n] = f16_t{};
 }
 
 template <int K, int RG, bool PL>
@@ -61,8 +61,8 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
     const ItemDesc* d = moe_block(a, cl, a.I / 128, nb);
     if (!d) return;
     const int cnt = d->cnt, p0 = d->p0, nblk = a.H / 128;
-    for (int i = threadIdx.x; i < 2 * 32 * RG; i += 256) {     // the rows' sums (block sums in order)
-        const int p = i / (32 * RG), m = i - p * 32 * RG;
+    for (int i = threadIdx.x; i < 2 * 32 * RG; i += 256) {   // the rows' sums (block sums in order)
+        const int p = i / (32 * RG), m = i - p * (32 * RG);
         rsum[p][m] = sum_ordered(a.xsum + ((size_t)(p0 + (m < cnt ? m : cnt - 1)) * 2 + p) * nblk, nblk);
     }
     const int pw = wave >> 1;                                  // this wave's projection
@@ -82,24 +82,25 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
         L.setup_a(cnt, plane);
     }
     f16_t acc[RG][2];
-    zero_acc<RG>(acc);
+    zero_acc(acc);
     L.run(acc);
 
-    // per 32-row group: the gate and up columns through LDS, eight lanes to a row
+    // per row group: the gate and up columns through LDS, eight lanes to a row
+    constexpr int LR = 8, N = 32 / LR;
     float* C = reinterpret_cast<float*>(smem);
-    const int rr = threadIdx.x >> 3, sub = lane & 7, col = nb * 128 + 4 * sub;
-    h2_t sg[4][2], su[4][2], sd[4][2];                         // fp16 pairs: as floats they would spill
+    const int rr = threadIdx.x / LR, sub = row_sub<LR>(lane), col = nb * 128 + 4 * sub;
+    h2_t sg[N][2], su[N][2], sd[N][2];                         // fp16 pairs: as floats they would spill
     {
         const uint16_t *pg = reinterpret_cast<const uint16_t*>(d->tab[2]) + col,
                        *pu = reinterpret_cast<const uint16_t*>(d->tab[5]) + col,
                        *pd = reinterpret_cast<const uint16_t*>(d->tab[7]) + col;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < N; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                sg[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pg + 32 * i + j));
-                su[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pu + 32 * i + j));
-                sd[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pd + 32 * i + j));
+                sg[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pg + 4 * LR * i + j));
+                su[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pu + 4 * LR * i + j));
+                sd[i][j >> 1][j & 1] = __builtin_bit_cast(_Float16, ldg(pd + 4 * LR * i + j));
             }
     }
     const bool tiled = a.Kd > 0, kp = a.Kd <= 5;               // the down kernel's A: block order (uniform K), or rows
@@ -113,21 +114,21 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
         const int m = 32 * rg + rr;
         if (m >= cnt) continue;
         const float xg = kMul1C2 * rsum[0][m], xu = kMul1C2 * rsum[1][m];
-        f4_t g[4], u[4];
+        f4_t g[N], u[N];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            g[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 32 * i + 4 * sub]);
-            u[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 144 + 32 * i + 4 * sub]);
+        for (int i = 0; i < N; ++i) {
+            g[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 4 * LR * i + 4 * sub]);
+            u[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 144 + 4 * LR * i + 4 * sub]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 g[i][j] = kMul1C1 * g[i][j] + xg;
                 u[i][j] = kMul1C1 * u[i][j] + xu;
             }
         }
-        fwht128_oct(g, lane);
-        fwht128_oct(u, lane);
+        fwht128_lanes<LR>(g, sub);
+        fwht128_lanes<LR>(u, sub);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < N; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float gv = (float)(_Float16)(g[i][j] * kRsqrt128 * (float)sg[i][j >> 1][j & 1]);
@@ -135,27 +136,24 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
                 const float av = (float)(_Float16)act_mul_dev(gv, uv, a.act, a.limit);
                 g[i][j] = (float)(_Float16)(av * (float)sd[i][j >> 1][j & 1]);
             }
-        fwht128_oct(g, lane);
-        float bs = 0.f;
+        fwht128_lanes<LR>(g, sub);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < N; ++i) {
             uint32_t h[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const _Float16 hv = (_Float16)(g[i][j] * kRsqrt128);
-                bs += (float)hv;
+                u[i][j] = (float)hv;
                 h[j] = __builtin_bit_cast(uint16_t, hv);
             }
             const uint2 v = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
             if (tiled) {
-                *reinterpret_cast<uint2*>(ab + unit_elem(cnt, col + 32 * i, m, kp)) = v;
+                *reinterpret_cast<uint2*>(ab + unit_elem(cnt, col + 4 * LR * i, m, kp)) = v;
             } else {
-                *reinterpret_cast<uint2*>(ab + (size_t)m * a.I + col + 32 * i) = v;
+                *reinterpret_cast<uint2*>(ab + (size_t)m * a.I + col + 4 * LR * i) = v;
             }
         }
-        bs += lane_xor<1>(bs, lane);
-        bs += lane_xor<2>(bs, lane);
-        bs += lane_xor<4>(bs, lane);
+        const float bs = row_sum128<LR>(u);
         if (sub == 0) a.asum[(size_t)(p0 + m) * (a.I / 128) + nb] = bs;
     }
 }
@@ -190,18 +188,19 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_down_wide_ke
         L.setup_a(cnt, plane);
     }
     f16_t acc[RG][2];
-    zero_acc<RG>(acc);
+    zero_acc(acc);
     L.run(acc);
 
     float* C = reinterpret_cast<float*>(smem);
-    const int rr = threadIdx.x >> 3, half = (threadIdx.x >> 2) & 1, sub = lane & 3;
-    float sd[8][4];
+    constexpr int LR = 4, N = 32 / LR;                         // lanes per 128-column half of a row
+    const int rr = threadIdx.x / (2 * LR), half = (threadIdx.x / LR) & 1, sub = row_sub<LR>(lane);
+    float sd[N][4];
     {
         const uint16_t* sv = reinterpret_cast<const uint16_t*>(d->tab[8]) + nb * 256 + 128 * (half < nhalf ? half : 0) + 4 * sub;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < N; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) sd[i][j] = h2f(ldg(sv + 16 * i + j));
+            for (int j = 0; j < 4; ++j) sd[i][j] = h2f(ldg(sv + 4 * LR * i + j));
     }
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
@@ -213,20 +212,20 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_down_wide_ke
         __syncthreads();
         if (m >= cnt || half >= nhalf) continue;
         const float sx = kMul1C2 * rsum[m];
-        f4_t v[8];
+        f4_t v[N];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            v[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 144 * half + 16 * i + 4 * sub]);
+        for (int i = 0; i < N; ++i) {
+            v[i] = *reinterpret_cast<const f4_t*>(&C[rr * kWideCS + 144 * half + 4 * LR * i + 4 * sub]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[i][j] = kMul1C1 * v[i][j] + sx;
         }
-        fwht128_quad(v, lane);
+        fwht128_lanes<LR>(v, sub);
         float* dst = a.y + (size_t)(p0 + m) * a.H + nb * 256 + 128 * half + 4 * sub;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < N; ++i) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[i][j] = v[i][j] * kRsqrt128 * sd[i][j] * w;
-            *reinterpret_cast<f4_t*>(dst + 16 * i) = v[i];
+            *reinterpret_cast<f4_t*>(dst + 4 * LR * i) = v[i];
         }
     }
 }
@@ -300,24 +299,34 @@ static moe_wide_fn pick_down(int K, bool pl) {
     EXL3_WIDE_PICK(moe_down_wide_kernel)
 }
 
-// Row groups of 32 in a block of row class `cl` (exl3_moe.h).
-static int class_groups(const MoeArgs& a, int cl) { return a.block_rows == kWideRows ? 1 << cl : cl == 2 ? 2 : 1; }
-
-int launch_gateup_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st) {
-    static const char* const names[3] = {"moe_gateup_mfma_r1", "moe_gateup_mfma_r2", "moe_gateup_mfma_r4"};
-    const int rg = class_groups(a, cl);
-    moe_wide_fn fn = rg == 4 ? pick_gateup<4>(a.Kg, a.planar) : rg == 2 ? pick_gateup<2>(a.Kg, a.planar)
-                                                                       : pick_gateup<1>(a.Kg, a.planar);
-    EXL3_LAUNCH(names[cl], fn, grid, dim3(256), 0, st, a, cl);
+// gate|up or down of one row class: 0: blocks of up to 32 rows, 1: up to a.block_rows
+int launch_gateup_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st) {
+    const dim3 grid((unsigned)((nblocks + 7) / 8 * 8 * (a.I / 128)));
+    moe_wide_fn fn = cl == 0 ? pick_gateup<1>(a.Kg, a.planar)
+                   : a.block_rows > 64 ? pick_gateup<4>(a.Kg, a.planar) : pick_gateup<2>(a.Kg, a.planar);
+    EXL3_LAUNCH(cl == 0 ? "moe_gateup_wide_32" : "moe_gateup_wide_big", fn, grid, dim3(256), 0, st, a, cl);
     return EXL3_OK;
 }
 
-int launch_down_wide(const MoeArgs& a, int cl, dim3 grid, hipStream_t st) {
-    static const char* const names[3] = {"moe_down_mfma_r1", "moe_down_mfma_r2", "moe_down_mfma_r4"};
-    const int rg = class_groups(a, cl);
-    moe_wide_fn fn = rg == 4 ? pick_down<4>(a.Kd, a.planar) : rg == 2 ? pick_down<2>(a.Kd, a.planar)
-                                                                     : pick_down<1>(a.Kd, a.planar);
-    EXL3_LAUNCH(names[cl], fn, grid, dim3(256), 0, st, a, cl);
+int launch_down_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st) {
+    const dim3 grid((unsigned)((nblocks + 7) / 8 * 8 * ((a.H / 128 + 1) / 2)));
+    moe_wide_fn fn = cl == 0 ? pick_down<1>(a.Kd, a.planar)
+                   : a.block_rows > 64 ? pick_down<4>(a.Kd, a.planar) : pick_down<2>(a.Kd, a.planar);
+    EXL3_LAUNCH(cl == 0 ? "moe_down_wide_32" : "moe_down_wide_big", fn, grid, dim3(256), 0, st, a, cl);
+    return EXL3_OK;
+}
+
+int launch_gateup_class(const MoeArgs& a, int cl, hipStream_t st) {
+    const dim3 grid((unsigned)((a.max_blocks + 7) / 8 * 8 * (a.I / 128)));
+    EXL3_LAUNCH("moe_gateup_wide", (cl == 2 ? pick_gateup<2>(a.Kg, a.planar) : pick_gateup<1>(a.Kg, a.planar)), grid,
+                dim3(256), 0, st, a, cl);
+    return EXL3_OK;
+}
+
+int launch_down_class(const MoeArgs& a, int cl, hipStream_t st) {
+    const dim3 grid((unsigned)((a.max_blocks + 7) / 8 * 8 * ((a.H / 128 + 1) / 2)));
+    EXL3_LAUNCH("moe_down_wide", (cl == 2 ? pick_down<2>(a.Kd, a.planar) : pick_down<1>(a.Kd, a.planar)), grid,
+                dim3(256), 0, st, a, cl);
     return EXL3_OK;
 }
 

@@ -269,6 +269,7 @@ struct DirectPipe : TileWords<K, PL> {
     typedef TileWords<K, PL> T;
     using T::decode_pair, T::lane, T::load_f, T::load_w, T::nsteps, T::NW, T::stage_w;
     static constexpr int AD = RG == 1 ? 4 : 2;               // steps of A in registers
+    static constexpr int WR = 4;                             // steps of words in registers
     __amdgpu_buffer_rsrc_t abuf;
     uint32_t aoff[RG];
     int astep, akk;                                          // bytes of A between steps and between 16-k blocks
@@ -280,7 +281,7 @@ struct DirectPipe : TileWords<K, PL> {
             A[i] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff[i % RG], so + i / RG * akk, 0));
     }
     template <int R>
-    __device__ __forceinline__ void step(int s, uint32_t (&W)[4][K], uint32_t (&F)[4][NW], h8_t (&A)[AD][2 * RG],
+    __device__ __forceinline__ void step(int s, uint32_t (&W)[WR][K], uint32_t (&F)[4][NW], h8_t (&A)[AD][2 * RG],
                                          f16_t (&acc)[RG][2]) const {
         typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -299,23 +300,23 @@ struct DirectPipe : TileWords<K, PL> {
                     __builtin_amdgcn_mfma_f32_32x32x16_f16(A[R % AD][(f >> 1) * RG + rg], b, acc[rg][f & 1], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        stage_w(W[(R + 2) % 4]);
+        stage_w(W[(R + 2) % WR]);
         load_a(A[R % AD], s + AD);
-        load_w(W[(R + 2) % 4], s + 6);
+        load_w(W[(R + 2) % WR], s + 2 + WR);
     }
     __device__ __forceinline__ void run(f16_t (&acc)[RG][2]) const {
-        uint32_t W[4][K], F[4][NW];
+        uint32_t W[WR][K], F[4][NW];
         h8_t A[AD][2 * RG];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) load_w(W[i], i);
+        for (int i = 0; i < WR; ++i) load_w(W[i], i);
 #pragma unroll
         for (int i = 0; i < AD; ++i) load_a(A[i], i);
         stage_w(W[0]);
 #pragma unroll
         for (int f = 0; f < 4; ++f) load_f(F[f], f);
         stage_w(W[1]);
-        load_w(W[0], 4);
-        load_w(W[1], 5);
+        load_w(W[0], WR);
+        load_w(W[1], WR + 1);
         for (int s = 0; s < nsteps; s += 4) {                  // nsteps is a multiple of 4
             step<0>(s, W, F, A, acc);
             step<1>(s + 1, W, F, A, acc);
@@ -337,59 +338,72 @@ struct DirectPipe : TileWords<K, PL> {
 };
 
 // ------------------------------------------------------------------------------------------------ epilogue
-// The 128-point transform of a row spread over four lanes of a quad: lane sub = lane & 3 holds columns
-// 16 i + 4 sub + j of v[i][j]. Bits 0, 1, 4, 5, 6 of the column are registers, bits 2 and 3 the lanes.
-__device__ __forceinline__ void fwht128_quad(f4_t (&v)[8], int lane) {
+// A row of 128 columns spread over L = 4, 8 or 16 adjacent lanes: lane index sub (row_sub) holds columns
+// 4 L i + 4 sub + j of v[i][j]. The transform's stages of column bits 0, 1 and of the bits of i are register additions,
+// those of sub exchange with the lane whose sub differs in one bit; column bits in ascending order whatever L is (the
+// same bits in every row class). sub is not the plain lane number: its bits are chosen
+// so that those lanes are at xor distances 1, 2, 7 and 15, each a single DPP move (quad permutes, half-row and row mirror).
+template <int L>
+__device__ __forceinline__ int row_sub(int lane) {
+    if (L == 4) return lane & 3;
+    const int l2 = (lane >> 2) & 1;
+    if (L == 8) return (lane & 7) ^ 3 * l2;
+    const int l3 = (lane >> 3) & 1;
+    return ((lane & 3) ^ 3 * l2) | (l2 ^ l3) << 2 | l3 << 3;
+}
+template <int B>                                             // value of the lane whose sub differs in bit B
+__device__ __forceinline__ float sub_xor(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 B == 0 ? 0xB1 : B == 1 ? 0x4E : B == 2 ? 0x141 : 0x140,
+                                                                 0xF, 0xF, false));
+}
+// Sum of a row's 128 values, pairwise by ascending column bit (the same bits whatever L is).
+template <int L>
+__device__ __forceinline__ float row_sum128(const f4_t (&v)[32 / L]) {
+    float t[32 / L];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < 32 / L; ++i) {
+        t[i] = (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        t[i] += sub_xor<0>(t[i]);
+        t[i] += sub_xor<1>(t[i]);
+        if constexpr (L >= 8) t[i] += sub_xor<2>(t[i]);
+        if constexpr (L >= 16) t[i] += sub_xor<3>(t[i]);
+    }
+#pragma unroll
+    for (int n = 16 / L; n > 0; n /= 2)
+#pragma unroll
+        for (int i = 0; i < n; ++i) t[i] = t[2 * i] + t[2 * i + 1];
+    return t[0];
+}
+template <int L>
+__device__ __forceinline__ void fwht128_lanes(f4_t (&v)[32 / L], int sub) {
+    constexpr int N = 32 / L;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
         const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
         v[i] = f4_t{a + c, b + d, a - c, b - d};
     }
+    const float s0 = sub & 1 ? -1.f : 1.f, s1 = sub & 2 ? -1.f : 1.f, s2 = sub & 4 ? -1.f : 1.f, s3 = sub & 8 ? -1.f : 1.f;
 #pragma unroll
-    for (int st = 1; st < 8; st *= 2)
+    for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int j = 0; j < 4; ++j) {
+            float x = v[i][j];
+            x = x * s0 + sub_xor<0>(x);
+            x = x * s1 + sub_xor<1>(x);
+            if constexpr (L >= 8) x = x * s2 + sub_xor<2>(x);
+            if constexpr (L >= 16) x = x * s3 + sub_xor<3>(x);
+            v[i][j] = x;
+        }
+#pragma unroll
+    for (int st = 1; st < N; st *= 2)
+#pragma unroll
+        for (int i = 0; i < N; ++i)
             if (!(i & st)) {
                 const f4_t a = v[i], b = v[i + st];
                 v[i] = a + b;
                 v[i + st] = a - b;
             }
-    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float x = v[i][j];
-            x = x * s1 + lane_xor<1>(x, lane);
-            x = x * s2 + lane_xor<2>(x, lane);
-            v[i][j] = x;
-        }
-}
-
-// The same over eight lanes: lane sub = lane & 7 holds columns 32 i + 4 sub + j of v[i][j]; bits 0, 1, 5, 6 of the column are
-// registers, bits 2 to 4 the lanes.
-__device__ __forceinline__ void fwht128_oct(f4_t (&v)[4], int lane) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
-        v[i] = f4_t{a + c, b + d, a - c, b - d};
-    }
-    const f4_t a = v[0] + v[1], b = v[0] - v[1], c = v[2] + v[3], d = v[2] - v[3];
-    v[0] = a + c;
-    v[1] = b + d;
-    v[2] = a - c;
-    v[3] = b - d;
-    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f, s4 = lane & 4 ? -1.f : 1.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float x = v[i][j];
-            x = x * s1 + lane_xor<1>(x, lane);
-            x = x * s2 + lane_xor<2>(x, lane);
-            x = x * s4 + lane_xor<4>(x, lane);
-            v[i][j] = x;
-        }
 }
 
 // Floats per row of a 32 x 256 output tile in LDS, column c at c + 16 (c >> 7): the 16-byte reads of the lanes of a row and

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     // operations per value for the transform); from LDS a quad of lanes takes a row half, five of seven stages in
     // registers.
     float* C = reinterpret_cast<float*>(smem);
-    const int rr = threadIdx.x >> 3, half = (threadIdx.x >> 2) & 1, sub = lane & 3;
+    const int rr = threadIdx.x >> 3, half = (threadIdx.x >> 2) & 1, sub = row_sub<4>(lane);
     const int col = nb * 256 + 128 * half + 4 * sub;
     float sd[8][4];
     {
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[i][j] = kMul1C1 * v[i][j] + sx;
         }
-        fwht128_quad(v, lane);
+        fwht128_lanes<4>(v, sub);
         if (a.f32) {
             float* o = reinterpret_cast<float*>(a.out) + orow * a.out_ld + col;
 #pragma unroll

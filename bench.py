@@ -44,7 +44,7 @@ METRIC = "EXL3 MoE layer µs/token + achieved HBM GB/s (% of peak), 1 MI355X"
 HBM_PEAK_GBS = 8000.0
 MFMA_F16_PEAK_TFLOPS = 2500.0
 VALU_PEAK_LANE_OPS = 256 * 64 * 2.4e9           # 256 CUs x 4 SIMDs x 16 lanes per clock x 2.4 GHz
-MFMA_ROWS, WIDE_ROWS = 64, 128                  # the library's MFMA row blocks: per-tile K, uniform K (<= 5)
+MFMA_ROWS = 64                                  # the library's MFMA row block with a per-tile K
 
 exl3 = importlib.import_module("b70-inference_amd")
 
@@ -292,13 +292,19 @@ class Mlp:
         return cpu_time(lambda: O.gated_mlp(x, *ps, O.ACT_GELU_TANH)), self.M, "one layer call"
 
 
-def mfma_blocks(rows, block=MFMA_ROWS):
-    """Row blocks of one expert with `rows` rows in the MFMA path: up to `block` rows each -> class index
-    (0: <= block / 4 rows, 1: <= block / 2, 2: <= block) per block."""
-    out = []
-    for q in range(0, rows, block):
-        c = min(block, rows - q)
-        out.append((0 if 4 * c <= block else 1 if 2 * c <= block else 2, c))
+def mfma_blocks(rows, wide=0):
+    """Row blocks of one expert with `rows` rows in the MFMA path -> (kernel label suffix, rows) per block. Per-tile K
+    (wide 0): up to 64 rows, labels mfma_r1 / r2 / r4 by 16, 32, 64 rows. Uniform K: up to `wide` rows (32, 64 or 128; with
+    128 a remainder of up to 64 in blocks of 32), labels wide_32 / wide_big."""
+    block, out, f = wide or MFMA_ROWS, [], 0
+    while f < rows:
+        left = rows - f
+        c = min(32 if block > 64 and left < block and left <= 64 else block, left)
+        if wide:
+            out.append(("wide_32" if c <= 32 else "wide_big", c))
+        else:
+            out.append(("mfma_r1" if c <= 16 else "mfma_r2" if c <= 32 else "mfma_r4", c))
+        f += c
     return out
 
 
@@ -320,7 +326,9 @@ class MoE:
         self.logits = [torch.randn(M, self.E, device="cuda", generator=g) for _ in range(nrout)]
         self.routing = [exl3.route_softmax_topk(lg, topk, bias) for lg in self.logits]
         self.ids = [ids.cpu() for ids, _ in self.routing]
-        self.block = MFMA_ROWS if t.K_gate == 0 or t.K_down == 0 else WIDE_ROWS
+        # the library's row block with uniform K (0: per-tile K)
+        mean, kmax = M * (topk + (1 if shared else 0)) / t.E, max(t.K_gate, t.K_down)
+        self.wide = (0 if t.K_gate == 0 or t.K_down == 0 else 32 if M <= 64 or (M <= 160 and mean <= 8) else 64 if 28 < mean <= 64 or kmax > 5 else 128)
         self.exp_bytes = [[weight_bytes(t.projs[q][e]) for q in range(3)] for e in range(t.E)]
         self.out = torch.empty(M, self.H, dtype=torch.float32, device="cuda")
 
@@ -361,9 +369,9 @@ class MoE:
         if name == "moe_fused":
             return self.bytes_per_step(j), self.flops_per_step(j)
         for proj, tag in ((0, "gateup"), (2, "down")):
-            if name.startswith(f"moe_{tag}_mfma_r"):
-                cl = {"1": 0, "2": 1, "4": 2}[name[-1]]
-                experts = {e: sum(c for k, c in mfma_blocks(r, self.block) if k == cl) for e, r in rpe.items()}
+            if name.startswith((f"moe_{tag}_mfma_r", f"moe_{tag}_wide_")):
+                cl = name[len(f"moe_{tag}_"):]
+                experts = {e: sum(c for k, c in mfma_blocks(r, self.wide) if k == cl) for e, r in rpe.items()}
                 experts = {e: r for e, r in experts.items() if r > 0}
                 rows = sum(experts.values())
                 if proj == 0:      # gate + up weights, xh rows in (two fp16 planes), fp16 down inputs out
@@ -383,9 +391,9 @@ class MoE:
         if name == "moe_fused":
             return 3 * len(rpe) * self.H * self.I
         for per, tag in ((2, "gateup"), (1, "down")):
-            if name.startswith(f"moe_{tag}_mfma_r"):
-                cl = {"1": 0, "2": 1, "4": 2}[name[-1]]
-                return per * self.H * self.I * sum(1 for r in rpe.values() for k, _ in mfma_blocks(r, self.block) if k == cl)
+            if name.startswith((f"moe_{tag}_mfma_r", f"moe_{tag}_wide_")):
+                cl = name[len(f"moe_{tag}_"):]
+                return per * self.H * self.I * sum(1 for r in rpe.values() for k, _ in mfma_blocks(r, self.wide) if k == cl)
         return None
 
     def cpu(self, O, np, rows=None):
@@ -584,7 +592,8 @@ def main():
         for j in range(args.steps):
             wl.step_fn(j)()
         torch.cuda.synchronize()
-        names = ["gemv", "moe_fused"] + [f"moe_{t}_mfma_r{c}" for t in ("gateup", "down") for c in (1, 2, 4)]
+        names = ["gemv", "moe_fused"] + [f"moe_{t}_{c}" for t in ("gateup", "down")
+                                          for c in ("mfma_r1", "mfma_r2", "mfma_r4", "wide_32", "wide_big")]
         dec, work = {}, {}
         for n in names:
             w = [wl.kernel_weights(n, j) for j in range(args.steps)]

@@ -650,16 +650,18 @@ def test_moe_prefill_hot_experts_many_blocks(exl3, oracle, monkeypatch, Kgu, Kd)
     assert torch.equal(a[perm.cuda()], c)
 
 
-# rows per expert at the edges of the row classes (32 / 64 / 128 rows; 16 / 32 / 64 for K > 5 or a per-tile K), several
-# blocks of one expert among them, and an expert without rows
-CLASS_ROWS = (1, 31, 32, 33, 0, 64, 65, 128, 129, 260, 17)
+# rows per expert at the edges of the blocks and row classes (32, 64, 128 rows; 16, 32, 64 with a per-tile K), several blocks
+# of one expert and remainders that are cut again among them, and an expert without rows
+CLASS_ROWS = (1, 31, 32, 33, 0, 64, 65, 128, 129, 260, 17, 170, 200)
 
 
-@pytest.mark.parametrize("Kgu,Kd", [(1, 1), (2, 3), (5, 4), (5, 6), (8, 3), (7, 8), (3, 0), (0, 2), (0, 6)])
-def test_moe_row_classes(exl3, oracle, monkeypatch, Kgu, Kd):
+@pytest.mark.parametrize("Kgu,Kd,block", [(1, 1, 128), (2, 3, 64), (2, 3, 32), (5, 4, 128), (5, 6, 64), (8, 3, 32),
+                                          (7, 8, 64), (3, 0, 0), (0, 2, 0), (0, 6, 0)])
+def test_moe_row_classes(exl3, oracle, monkeypatch, Kgu, Kd, block):
     """Row blocks of every class, at a width with a half column block (H = 384), for both fragment orders and for a
     uniform projection beside a per-tile one (0), against the oracle."""
     monkeypatch.setenv("EXL3MI_MOE_MFMA", "1")
+    monkeypatch.setenv("EXL3MI_MOE_BLOCK", str(block))
     from moe_util import gpu_proj, make_proj, oracle_proj
     E, H, I = len(CLASS_ROWS), 384, 256
     pt = ((1, 2, 5), (0.4, 0.4, 0.2))
@@ -678,6 +680,10 @@ def test_moe_row_classes(exl3, oracle, monkeypatch, Kgu, Kd):
     for dt in (torch.float32, torch.float16):
         y, ref = _run(exl3, oracle, tables, orc, x, ids, w, out_dtype=dt)
         assert max_rel(y, ref) <= MAX_REL, dt
+    if block:                                   # a row's bits do not depend on the block it lies in
+        a = exl3.moe_forward(x.cuda(), ids.cuda(), w.cuda(), tables)
+        monkeypatch.setenv("EXL3MI_MOE_BLOCK", "32" if block > 32 else "64")
+        assert torch.equal(a, exl3.moe_forward(x.cuda(), ids.cuda(), w.cuda(), tables))
 
 
 @pytest.mark.parametrize("K,M,out_dtype", [(4, 150, torch.float32), (3, 300, torch.float16), (6, 200, torch.float32)])
