@@ -1654,12 +1654,14 @@ int exl3_router_logits(const uint16_t* x, int64_t x_ld, int64_t M, int64_t H, co
     EXL3_CHECK_ARG(M <= 4 * 65535 && H <= 0x7FFFFFFF, "exl3_router_logits: shape too large");
     EXL3_CHECK_ARG(aligned(W, 16) && w_ld % 8 == 0, "exl3_router_logits: W must be 16-byte aligned, row stride a multiple of 8");
     hipStream_t st = (hipStream_t)stream;
-    const int MR = M >= 8 ? 8 : M >= 4 ? 4 : M >= 2 ? 2 : 1;       // rows per workgroup ([H, E]: at most 4)
     typedef void (*rfn)(const uint16_t*, int64_t, int, int, const uint16_t*, int64_t, int, int, float*, int64_t);
     if (w_layout == EXL3_ROUTER_W_HE) {
         EXL3_CHECK_ARG(E % 8 == 0 && w_ld >= E && aligned(x, 4) && x_ld % 2 == 0,
                        "exl3_router_logits: [H, E] weights need E a multiple of 8, w_ld >= E and a 4-byte aligned x");
-        const int mr = MR > 4 ? 4 : MR;
+        // rows per workgroup: as many as leave 256 workgroups, else one (a workgroup's FMAs are one CU's work: 2048 x 512
+        // at 8 rows 10.9 us with four rows per workgroup, 16 workgroups)
+        const int64_t strips = (E + 63) / 64;
+        const int mr = strips * ((M + 3) / 4) >= 256 ? 4 : strips * ((M + 1) / 2) >= 256 ? 2 : 1;
         rfn fn = mr == 4 ? router_cols_kernel<4> : mr == 2 ? router_cols_kernel<2> : router_cols_kernel<1>;
         const unsigned gy = (unsigned)((M + mr - 1) / mr);
         EXL3_LAUNCH("router_logits", fn, dim3((unsigned)((E + 63) / 64), gy), dim3(1024), 0, st, x, x_ld, (int)M,
@@ -1667,6 +1669,7 @@ int exl3_router_logits(const uint16_t* x, int64_t x_ld, int64_t M, int64_t H, co
     } else {
         EXL3_CHECK_ARG(w_ld >= H && aligned(x, 16) && x_ld % 8 == 0,
                        "exl3_router_logits: [E, H] weights need w_ld >= H and a 16-byte aligned x (row stride a multiple of 8)");
+        const int MR = M >= 8 ? 8 : M >= 4 ? 4 : M >= 2 ? 2 : 1;   // rows per workgroup
         rfn fn = MR == 8 ? router_rows_kernel<8> : MR == 4 ? router_rows_kernel<4> : MR == 2 ? router_rows_kernel<2>
                                                                                           : router_rows_kernel<1>;
         const unsigned gy = (unsigned)((M + MR - 1) / MR);
