@@ -456,11 +456,27 @@ static int gemv_splits(int strips, int nblk, int rows) {
     return P < 1 ? 1 : P;
 }
 
-// Dense linear on MFMA (exl3_mfma.hip), used from kLinearMfmaMinRows rows on.
+// Dense linear on MFMA (exl3_mfma.hip): scratch of a call, and the call (in `fixed` scratch if given).
+int linear_mfma_scratch(int64_t m, int64_t n, int64_t k, int S, int K, size_t* bytes);
 int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n, int K,
                        void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
-                       const uint16_t* svh, hipStream_t st);
+                       const uint16_t* svh, char* fixed, size_t fixed_bytes, hipStream_t st);
 constexpr int kLinearMfmaMinRows = 9;
+constexpr size_t kNoAllocPartBytes = 16u << 20;              // fixed scratch of the allocation-free entry point
+
+// Rows that take the MFMA GEMM: more than the GEMV takes per pass, and five or more on large matrices. The GEMV's time
+// grows with the rows, the GEMM's three launches cost about 15 us whatever the matrix; us, GEMV / GEMM: 5376 -> 21504 at
+// 4 / 6 / 8 rows 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096
+// 9.9 / 16.7, 12.1 / 16.5, 13.0 / 16.6. Below nine rows only where its scratch fits the allocation-free entry point's (the
+// two entry points give the same bits) and, under stream capture, what the workspace holds. forced > 0: the rows from which it is taken (tests).
+static int takes_mfma(int64_t m, int64_t k, int64_t n, int S, int K, size_t room, int forced, bool* yes) {
+    *yes = m >= (forced ? forced : kLinearMfmaMinRows);
+    if (*yes || forced || m < 5 || k * n < 200000000 / (m - 2)) return EXL3_OK;
+    size_t bytes = 0;
+    const int rc = linear_mfma_scratch(m, n, k, S, K, &bytes);
+    *yes = !rc && bytes <= kNoAllocPartBytes && bytes <= room;
+    return rc;
+}
 
 // Launches over chunks of up to kGemvMaxRows rows of `ga` (x, out and m describe all rows; the workspace holds
 // slots x strips x P partial blocks and slots x strips counters).
@@ -538,7 +554,6 @@ int launch_gemv(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uin
 // The decode GEMV of exl3_gemm with its split-K partials and arrival counters in a fixed device array instead of the
 // library workspace, for callers that cannot allocate (code under HIP graph capture, serving loops). The array lives
 // as long as the process, one copy per device; every call on a device shares it (calls that overlap race).
-constexpr size_t kNoAllocPartBytes = 16u << 20;              // split-K partials: strips x P x 8 rows x 128 fp32
 constexpr size_t kNoAllocCounters = 16384;                   // arrival counters: one per 128-column strip
 static __device__ __align__(256) char scratch[kNoAllocPartBytes + kNoAllocCounters * sizeof(int)];
 
@@ -699,9 +714,13 @@ int exl3_linear_sharded(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, c
                    "exl3_gemm: trellis of %lld x %lld at K=%d exceeds 2^32 words", (long long)k, (long long)n, K);
     const uint32_t* tr = reinterpret_cast<const uint32_t*>(B);
     const int S = (int)n_shards;
-    if (m >= env_int("EXL3MI_MFMA_MIN_ROWS", kLinearMfmaMinRows))
-        return launch_linear_mfma(A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh,
-                                  (hipStream_t)stream);
+    bool mfma = false;
+    const int rc = takes_mfma(m, k, n, S, K, workspace_room((hipStream_t)stream), env_int("EXL3MI_MFMA_MIN_ROWS", 0),
+                              &mfma);
+    if (rc) return rc;
+    if (mfma)
+        return launch_linear_mfma(A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh, nullptr,
+                                  0, (hipStream_t)stream);
     return launch_gemv(A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh,
                        (hipStream_t)stream);
 }
@@ -740,8 +759,13 @@ int exl3_gemm_noalloc(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, con
                    "scratch holds %zu", part, kNoAllocPartBytes);
     hipStream_t st = (hipStream_t)stream;
     char* sc = nullptr;
-    const int rc = noalloc_scratch(st, &sc);
+    int rc = noalloc_scratch(st, &sc);
     if (rc) return rc;
+    bool mfma = false;
+    if ((rc = takes_mfma(m, k, n, 1, K, kNoAllocPartBytes, 0, &mfma))) return rc;
+    if (mfma)
+        return launch_linear_mfma(A, a_ld, m, k, reinterpret_cast<const uint32_t*>(B), n, K, C, c_ld, c_dtype == EXL3_F32,
+                                  suh, 1, nullptr, svh, sc, kNoAllocPartBytes, st);
     GemvArgs ga = gemv_args(A, a_ld, k, reinterpret_cast<const uint32_t*>(B), n, C, c_ld, suh, 1, nullptr, svh, P);
     ga.part = reinterpret_cast<float*>(sc);
     ga.cnt = reinterpret_cast<int*>(sc + kNoAllocPartBytes);

@@ -879,17 +879,12 @@ struct LinPlan {
 // blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
 // the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
 // `rg` > 0 fixes the row block, `cap` bounds the splits.
-static int linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, LinPlan* best) {
+static int linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap, LinPlan* best) {
     const int nblk = (int)(k / 128);
-    int dev = 0, cus = 0, occ[4];
+    int dev = 0, cus = 0;
     EXL3_CHECK_HIP(hipGetDevice(&dev));
     EXL3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    for (int g = 0; g < 4; ++g) {
-        int resident = 0;
-        const int rc = resident_blocks((const void*)linear_wide_pick(1 << g, S, K), 256, &resident);
-        if (rc) return rc;
-        occ[g] = resident / cus < 1 ? 1 : resident / cus > 4 ? 4 : resident / cus;
-    }
+    const int occ[4] = {K <= 5 ? 4 : 3, K <= 5 ? 3 : 2, 2, 1};       // what the kernels are compiled for (exl3_wide.hip)
     static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
                                         {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
     static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
@@ -920,7 +915,7 @@ static int linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, in
 // k-splits of a dense MLP's down projection (m rows in blocks of `block` rows), at most `cap`.
 int dense_down_splits(int64_t m, int64_t n, int64_t k, int K, int block, int64_t cap, int* P) {
     LinPlan pl;
-    const int rc = linear_plan(m, n, k, 1, K, block / 32, cap, &pl);
+    const int rc = linear_plan(m, n, k, K, block / 32, cap, &pl);
     *P = pl.P;
     return rc;
 }
@@ -998,19 +993,34 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
     return a.dense_P > 0 ? launch_dense_down(a, st) : launch_moe_combine(a, st);
 }
 
-// Dense linear on MFMA (m > the GEMV's rows per pass): input transform, blocks of 32 .. 256 rows x 256 columns and, with
-// k-splits, the reduction.
+// Plan of a call of m rows, with at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the
+// scratch of the partials), and its scratch.
+static int linear_call_plan(int64_t m, int64_t n, int64_t k, int K, LinPlan* pl) {
+    const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
+    const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
+    return linear_plan(m, n, k, K, 0, ((m <= 32 ? 768 : 512) + ts - 1) / ts, pl);
+}
+static size_t linear_call_bytes(int64_t m, int64_t n, int64_t k, int S, int P) {
+    return carve_size((size_t)S * m * k, 2) + carve_size((size_t)S * m * (k / 128), 4) +
+           (P > 1 ? carve_size((size_t)P * m * n, 4) : 0);
+}
+int linear_mfma_scratch(int64_t m, int64_t n, int64_t k, int S, int K, size_t* bytes) {
+    LinPlan pl;
+    const int rc = linear_call_plan(m, n, k, K, &pl);
+    if (!rc) *bytes = linear_call_bytes(m, n, k, S, pl.P);
+    return rc;
+}
+
+// Dense linear on MFMA: input transform, blocks of 32 .. 256 rows x 256 columns and, with k-splits, the reduction. Scratch
+// from the workspace, or `fixed` (fixed_bytes of it; those launches also bypass the opt-in event profiler).
 int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n, int K,
                        void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
-                       const uint16_t* svh, hipStream_t st) {
+                       const uint16_t* svh, char* fixed, size_t fixed_bytes, hipStream_t st) {
     const int nblk = (int)(k / 128);
     if (m > 0x7FFFFFFF / 64 || k > 0x7FFFFFFF || n > 0x7FFFFFFF || nblk > 65535)
         return fail(EXL3_ERR_INVALID, "exl3_gemm: shape too large");
-    // at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the scratch of the partials)
-    const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
-    const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
     LinPlan pl;
-    int rc = linear_plan(m, n, k, S, K, 0, ((m <= 32 ? 768 : 512) + ts - 1) / ts, &pl);
+    int rc = linear_call_plan(m, n, k, K, &pl);
     if (rc) return rc;
     const int force = env_int("EXL3MI_LINEAR_BLOCK", 0);           // row groups of 32 per block: 1, 2, 4 or 8
     if (force == 1 || force == 2 || force == 4 || force == 8) pl.RG = force;
@@ -1030,12 +1040,14 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     a.ncb = (int)((n + 255) / 256);
     a.bps = pl.bps;
     a.P = pl.P;
-    const size_t xh_b = carve_size((size_t)S * m * k, 2), xs_b = carve_size((size_t)S * m * nblk, 4);
-    const size_t part_b = a.P > 1 ? carve_size((size_t)a.P * m * n, 4) : 0;
-    Workspace ws;
-    rc = workspace(xh_b + xs_b + part_b, 0, st, &ws);
-    if (rc) return rc;
-    Carve cv{ws.scratch, ws.scratch_bytes};
+    const size_t bytes = linear_call_bytes(m, n, k, S, a.P);
+    Carve cv{fixed, fixed_bytes};
+    if (!fixed) {
+        Workspace ws;
+        rc = workspace(bytes, 0, st, &ws);
+        if (rc) return rc;
+        cv = Carve{ws.scratch, ws.scratch_bytes};
+    }
     _Float16* xh = cv.take<_Float16>((size_t)S * m * k);
     float* xsum = cv.take<float>((size_t)S * m * nblk);
     a.part = a.P > 1 ? cv.take<float>((size_t)a.P * m * n) : nullptr;
@@ -1050,14 +1062,21 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     a.out_ld = c_ld;
     a.f32 = f32 ? 1 : 0;
     const dim3 hgrid((unsigned)((m + 63) / 64), (unsigned)nblk, (unsigned)S);
-    EXL3_LAUNCH("linear_had", linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum, R,
-                K <= 5);
     const int64_t nx = ((int64_t)a.nrb * a.ncb * a.P + 7) / 8 * 8;
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_gemm: grid too large");
-    EXL3_LAUNCH("linear_wide", linear_wide_pick(pl.RG, S, K), dim3((unsigned)nx), dim3(256), 0, st, a);
-    if (a.P > 1)
-        EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, dim3((unsigned)((m + 3) / 4), (unsigned)(n / 128)),
-                    dim3(256), 0, st, a);
+    const dim3 rgrid((unsigned)((m + 3) / 4), (unsigned)(n / 128));
+    const lin_fn fn = linear_wide_pick(pl.RG, S, K);
+    if (fixed) {
+        hipLaunchKernelGGL(linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum, R, K <= 5);
+        hipLaunchKernelGGL(fn, dim3((unsigned)nx), dim3(256), 0, st, a);
+        if (a.P > 1) hipLaunchKernelGGL(linear_reduce_kernel, rgrid, dim3(256), 0, st, a);
+        EXL3_CHECK_HIP(hipGetLastError());
+        return EXL3_OK;
+    }
+    EXL3_LAUNCH("linear_had", linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum, R,
+                K <= 5);
+    EXL3_LAUNCH("linear_wide", fn, dim3((unsigned)nx), dim3(256), 0, st, a);
+    if (a.P > 1) EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, rgrid, dim3(256), 0, st, a);
     return EXL3_OK;
 }
 

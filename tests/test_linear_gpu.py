@@ -222,6 +222,27 @@ def test_gemm_mfma_row_blocks(exl3, oracle, monkeypatch, block, k, n, K, M, out_
         assert max_rel(y, ref) <= MAX_REL, jobs
 
 
+@pytest.mark.parametrize("k,n,K,M", [(8192, 8192, 2, 5), (4096, 14336, 3, 6), (2048, 21504, 7, 7), (5376, 6400, 4, 8)])
+def test_gemm_few_rows_of_large_matrices(exl3, oracle, M, k, n, K):
+    """Five to eight rows on both sides of the size from which they take the MFMA GEMM: the first and last 128 columns
+    against the oracle, and the allocation-free entry point bit for bit."""
+    from importlib import import_module
+    L_ = import_module("b70-inference_amd._lib")
+    S_ = synth()
+    tr, suh, svh = S_.linear(k, n, K, 7600 + M)
+    x = S_.activations(M, k, 7610 + M)
+    xc, trc, suc, svc = x.cuda(), tr.cuda(), suh.cuda(), svh.cuda()
+    y = exl3.BC_LinearEXL3(trc, suc, svc, K, None, False, True, None).run_alloc(xc, n, True)
+    z = torch.full_like(y, float("nan"))
+    L_.check(L_.lib().exl3_gemm_noalloc(L_.ptr(xc), k, M, k, L_.ptr(trc), n, K, L_.ptr(z), n, 1, L_.ptr(suc),
+                                        L_.ptr(svc), 2, L_.stream_of(xc)), "exl3_gemm_noalloc")
+    assert torch.equal(y, z)
+    for t in (0, n // 16 - 8):                              # 128-column blocks do not depend on each other
+        ref = oracle.exl3_linear(x.numpy(), tr[:, t:t + 8].contiguous().numpy(), suh.numpy(),
+                                 svh[16 * t:16 * t + 128].numpy(), K, np.float32)
+        assert max_rel(y[:, 16 * t:16 * t + 128].cpu().numpy(), ref) <= MAX_REL
+
+
 @pytest.mark.parametrize("block", [1, 4, 8])
 def test_linear_sharded_row_blocks(exl3, oracle, monkeypatch, block):
     """Shards under every way a block reads its input planes (straight from memory, two staged planes), into rows
