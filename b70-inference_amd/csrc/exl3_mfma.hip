@@ -19,6 +19,7 @@
 #include "exl3_mfma.h"
 #include "exl3_moe.h"
 #include "exl3_moe_dev.h"
+#include "exl3_plan.h"
 #include "exl3_runtime.h"
 
 namespace exl3 {
@@ -867,56 +868,18 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
 
 lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
 
-struct LinPlan {
-    int RG, P, bps;                                  // row groups of 32 per block, k-splits, 128-blocks of k per split
-};
-
-// Row block and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
-// each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
-// workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
-// and that kernel's launch. Fitted to 878 measured points at K = 4 (1024 x 4096 .. 5376 x 21504, 16 .. 1024 rows, 1 .. 16
-// splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
-// blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
-// the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
-// `rg` > 0 fixes the row block, `cap` bounds the splits.
-static int linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap, LinPlan* best) {
-    const int nblk = (int)(k / 128);
-    int dev = 0, cus = 0;
+static int device_cus(int* cus) {
+    int dev = 0;
     EXL3_CHECK_HIP(hipGetDevice(&dev));
-    EXL3_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int occ[4] = {K <= 5 ? 4 : 3, K <= 5 ? 3 : 2, 2, 1};       // what the kernels are compiled for (exl3_wide.hip)
-    static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
-                                        {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
-    static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
-    const int64_t ncb = (n + 255) / 256;
-    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
-    *best = {rg > 0 ? rg : 1, 1, nblk};
-    float tb = 1e30f;
-    for (int g = 0; g < 4; ++g) {
-        if (rg > 0 && rg != 1 << g) continue;
-        const int64_t tiles = (m + (32 << g) - 1) / (32 << g) * ncb;
-        for (int p = 1; p <= pmax && p <= cap; ++p) {
-            const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
-            if (P != p) continue;
-            const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
-            const float mb = (float)P * (float)m * (float)n * 4e-6f;
-            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
-                      kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
-            if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
-            if (t < tb) {
-                tb = t;
-                *best = {1 << g, P, bps};
-            }
-        }
-    }
+    EXL3_CHECK_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
     return EXL3_OK;
 }
 
 // k-splits of a dense MLP's down projection (m rows in blocks of `block` rows), at most `cap`.
 int dense_down_splits(int64_t m, int64_t n, int64_t k, int K, int block, int64_t cap, int* P) {
-    LinPlan pl;
-    const int rc = linear_plan(m, n, k, K, block / 32, cap, &pl);
-    *P = pl.P;
+    int cus = 0;
+    const int rc = device_cus(&cus);
+    if (!rc) *P = linear_plan(m, n, k, K, block / 32, cap, cus).P;
     return rc;
 }
 
@@ -998,7 +961,13 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
 static int linear_call_plan(int64_t m, int64_t n, int64_t k, int K, LinPlan* pl) {
     const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
     const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
-    return linear_plan(m, n, k, K, 0, ((m <= 32 ? 768 : 512) + ts - 1) / ts, pl);
+    int cus = 0;
+    const int rc = device_cus(&cus);
+    const int rg = env_int("EXL3MI_LINEAR_BLOCK", 0);              // forced row groups of 32 per block: 1, 2, 4 or 8
+    if (!rc)
+        *pl = linear_plan(m, n, k, K, rg == 1 || rg == 2 || rg == 4 || rg == 8 ? rg : 0,
+                          ((m <= 32 ? 768 : 512) + ts - 1) / ts, cus);
+    return rc;
 }
 static size_t linear_call_bytes(int64_t m, int64_t n, int64_t k, int S, int P) {
     return carve_size((size_t)S * m * k, 2) + carve_size((size_t)S * m * (k / 128), 4) +
@@ -1022,15 +991,14 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     LinPlan pl;
     int rc = linear_call_plan(m, n, k, K, &pl);
     if (rc) return rc;
-    const int force = env_int("EXL3MI_LINEAR_BLOCK", 0);           // row groups of 32 per block: 1, 2, 4 or 8
-    if (force == 1 || force == 2 || force == 4 || force == 8) pl.RG = force;
-    const int R = 32 * pl.RG;
     if (const int jobs = env_int("EXL3MI_LINEAR_JOBS", 0)) {       // forced workgroup target
-        const int64_t tiles = (m + R - 1) / R * ((n + 255) / 256), want = (jobs + tiles - 1) / tiles;
+        const int64_t R = 32 * pl.RG, tiles = (m + R - 1) / R * ((n + 255) / 256), want = (jobs + tiles - 1) / tiles;
         const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
         pl.bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
         pl.P = (nblk + pl.bps - 1) / pl.bps;
+        while (pl.RG > 1 && !a_span_ok(m < 32 * pl.RG ? m : 32 * pl.RG, 128LL * pl.bps)) pl.RG /= 2;
     }
+    const int R = 32 * pl.RG;
     LinArgs a = {};
     a.m = (int)m;
     a.k = (int)k;

@@ -15,6 +15,7 @@
 #include "exl3_gemv.h"
 #include "exl3_moe.h"
 #include "exl3_moe_dev.h"
+#include "exl3_plan.h"
 #include "exl3_runtime.h"
 
 namespace exl3 {
@@ -1418,19 +1419,14 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     int64_t mi = mfma ? 0 : E + npairs / a.MR;
     if (mi > npairs) mi = npairs;
     a.max_items = (int)mi;
-    // Row block with uniform K: 32 (one class, one launch per projection) up to 64 tokens, 160 where experts take few rows:
-    // forking the launches by class costs more there (10 to 25 us) than decoding the experts with more rows again; 64 where an expert takes 28 to 64
-    // rows on average (and for K > 5, where 128 rows would spill), else 128. Per 32-k step a workgroup of 32 / 64 / 128 rows
-    // takes 0.21 / 0.28 / 0.41 us.
     const bool wide = a.Kg > 0 && a.Kd > 0;
-    const double mean = (double)npairs / (double)E;
-    a.block_rows = !wide ? kMfmaRows : E > 1 && (M <= 64 || (M <= 160 && mean <= 8)) ? 32 : (mean > 28 && mean <= 64) || a.Kg > 5 || a.Kd > 5 ? 64 : kWideRows;
-    if (const int rb = env_int("EXL3MI_MOE_BLOCK", 0); wide && (rb == 32 || rb == 64 || (rb == 128 && a.Kg <= 5 && a.Kd <= 5)))
-        a.block_rows = rb;
+    a.block_rows = wide ? moe_wide_rows(M, E, npairs, a.H, a.I, a.Kg, a.Kd, env_int("EXL3MI_MOE_BLOCK", 0)) : kMfmaRows;
     a.max_blocks = mfma ? (int)(npairs / (wide ? 32 : kMfmaRows) + (E < npairs ? E : npairs) + 1) : 0;
     EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= (wide ? 1 << 21 : 65535) &&
                        (int64_t)(a.max_blocks + 8) * (a.I > a.H ? a.I / 128 : a.H / 128) < 0x7FFFFFFF,
                    "exl3_moe_forward: grid too large");
+    EXL3_CHECK_ARG(!mfma || !wide || a_span_ok(npairs < a.block_rows ? npairs : a.block_rows, a.H > a.I ? a.H : a.I),
+                   "exl3_moe_forward: H=%d or I=%d too large", a.H, a.I);
     return moe_decode_path(a, npairs, st);
 }
 

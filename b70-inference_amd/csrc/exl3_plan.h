@@ -1,0 +1,68 @@
+// Host-side choices of the wide-block kernels (exl3_wide.h): row blocks and k-splits. Plain C++ without device code.
+#pragma once
+
+#include <stdint.h>
+
+namespace exl3 {
+
+// The wide kernels address the A rows of a block (`rows` rows, k columns, fp16) by 32-bit offsets from its first byte, in a
+// buffer resource of 2^31 - 1 bytes: loads past it return zero. Blocks are cut so that they stay inside.
+constexpr bool a_span_ok(int64_t rows, int64_t k) { return 2 * rows * k <= 0x7FFFFFFF; }
+
+struct LinPlan {
+    int RG, P, bps;                                  // row groups of 32 per block, k-splits, 128-blocks of k per split
+};
+
+// Row block and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
+// each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
+// workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
+// and that kernel's launch. Fitted to 878 measured points at K = 4 (1024 x 4096 .. 5376 x 21504, 16 .. 1024 rows, 1 .. 16
+// splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
+// blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
+// the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
+// `rg` > 0 asks for that row block (halved until the offsets of a block's A fit), `cap` bounds the splits.
+inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap, int cus) {
+    const int nblk = (int)(k / 128);
+    const int occ[4] = {K <= 5 ? 4 : 3, K <= 5 ? 3 : 2, 2, 1};       // what the kernels are compiled for (exl3_wide.hip)
+    static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
+                                        {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
+    static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
+    const int64_t ncb = (n + 255) / 256;
+    const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
+    LinPlan best = {1, 1, nblk};
+    float tb = 1e30f;
+    for (int g = 0; g < 4; ++g) {
+        if (rg > 0 && rg != 1 << g) continue;
+        const int64_t rows = 32 << g, tiles = (m + rows - 1) / rows * ncb;
+        for (int p = 1; p <= pmax && p <= cap; ++p) {
+            const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
+            if (P != p || !a_span_ok(m < rows ? m : rows, 128LL * bps)) continue;
+            const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
+            const float mb = (float)P * (float)m * (float)n * 4e-6f;
+            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
+                      kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
+            if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
+            if (t < tb) {
+                tb = t;
+                best = {1 << g, P, bps};
+            }
+        }
+    }
+    return tb == 1e30f && rg > 1 ? linear_plan(m, n, k, K, rg / 2, cap, cus) : best;
+}
+
+// Row block of the prefill MoE (M tokens, `npairs` rows over E experts, H -> I -> H; uniform K: 1 .. 8). 32 (one class, one
+// launch per projection) up to 64 tokens, 160 where experts take few rows: forking the launches by class costs more there
+// (10 to 25 us) than decoding the experts with more rows again; 64 where an expert takes 28 to 64 rows on average (and for
+// K > 5, where 128 rows would spill), else 128. Per 32-k step a workgroup of 32 / 64 / 128 rows takes 0.21 / 0.28 / 0.41 us.
+// `forced`: 32, 64 or 128 (where it may be taken), or 0.
+inline int moe_wide_rows(int64_t M, int64_t E, int64_t npairs, int64_t H, int64_t I, int Kg, int Kd, int forced) {
+    const double mean = (double)npairs / (double)E;
+    int rows = E > 1 && (M <= 64 || (M <= 160 && mean <= 8)) ? 32 : (mean > 28 && mean <= 64) ? 64 : 128;
+    if (forced == 32 || forced == 64 || forced == 128) rows = forced;
+    if (rows == 128 && (Kg > 5 || Kd > 5)) rows = 64;
+    while (rows > 32 && !a_span_ok(npairs < rows ? npairs : rows, H > I ? H : I)) rows /= 2;
+    return rows;
+}
+
+}  // namespace exl3
