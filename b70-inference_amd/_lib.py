@@ -89,6 +89,7 @@ def check(rc: int, what: str = ""):
 # The helpers below run several times per call, and a one-row linear is bound by its host path (4096 x 4096, K = 4: 6.8 us on
 # the GPU, 16 us per call with a c_void_p object per pointer, a Stream object and device objects; see run_alloc): plain
 # integers for the pointers (ctypes converts them by the declared argument types), the raw stream, the tensors' own flags.
+# A pointer does not keep its tensor alive: a temporary (x.contiguous()) needs a name until the call has been made.
 def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 

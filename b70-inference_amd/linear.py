@@ -84,9 +84,10 @@ def reconstruct_had_slice(unpacked: torch.Tensor, packed: torch.Tensor, suh: tor
         raise Exl3Error("reconstruct_had_slice: unpacked [k, n_slice], suh [k] and svh [>= n_slice] expected")
     if suh.dtype != torch.float16 or svh.dtype != torch.float16:
         raise Exl3Error("reconstruct_had_slice: suh / svh must be fp16")
-    check(lib().exl3_reconstruct_had_slice(ptr(packed), k, packed.shape[1] * 16, K, cb, ptr(suh.contiguous()),
-                                           ptr(svh.contiguous()), int(n_offset), n_slice, ptr(unpacked),
-                                           unpacked.stride(0), stream_of(unpacked)), "reconstruct_had_slice")
+    suh, svh = suh.contiguous(), svh.contiguous()     # (locals: a pointer does not keep its tensor alive)
+    check(lib().exl3_reconstruct_had_slice(ptr(packed), k, packed.shape[1] * 16, K, cb, ptr(suh), ptr(svh),
+                                           int(n_offset), n_slice, ptr(unpacked), unpacked.stride(0),
+                                           stream_of(unpacked)), "reconstruct_had_slice")
 
 
 def had_r_128(input: torch.Tensor, output: torch.Tensor, pre_scale, post_scale, scale: float) -> None:
@@ -149,8 +150,9 @@ def exl3_gemm_noalloc(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: to
     if C.numel() // n != m:
         raise Exl3Error("exl3_gemm_noalloc: A and C row counts differ")
     dt = EXL3_F32 if C.dtype == torch.float32 else EXL3_F16
-    check(lib().exl3_gemm_noalloc(ptr(A), k, m, k, ptr(B.contiguous()), n, K, ptr(C), n, dt, ptr(suh.contiguous()),
-                                  ptr(svh.contiguous()), CB_MUL1, stream_of(A)), "exl3_gemm_noalloc")
+    B, suh, svh = B.contiguous(), suh.contiguous(), svh.contiguous()
+    check(lib().exl3_gemm_noalloc(ptr(A), k, m, k, ptr(B), n, K, ptr(C), n, dt, ptr(suh), ptr(svh), CB_MUL1,
+                                  stream_of(A)), "exl3_gemm_noalloc")
 
 
 def exl3_mgemm(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: torch.Tensor, A_had, svh: torch.Tensor,
@@ -199,9 +201,9 @@ def exl3_mgemm(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: torch.Ten
     elif C.shape[0] != slots:
         raise Exl3Error(f"exl3_mgemm: C must be [slots={slots}, m, n]")
     dt = EXL3_F32 if C.dtype == torch.float32 else EXL3_F16
-    check(lib().exl3_mgemm(ptr(A3), a_batches, m, k, ptr(B.contiguous()), ptr(suh.contiguous()),
-                           ptr(svh.contiguous()), B.numel(), n, Ki, cb, ptr(idx), slots, ptr(w), num_tokens,
-                           min_index, max_index, ptr(C), dt, stream_of(A)), "exl3_mgemm")
+    B, suh, svh = B.contiguous(), suh.contiguous(), svh.contiguous()
+    check(lib().exl3_mgemm(ptr(A3), a_batches, m, k, ptr(B), ptr(suh), ptr(svh), B.numel(), n, Ki, cb, ptr(idx), slots,
+                           ptr(w), num_tokens, min_index, max_index, ptr(C), dt, stream_of(A)), "exl3_mgemm")
     return 0
 
 

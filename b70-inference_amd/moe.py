@@ -215,7 +215,8 @@ def blob_unplanarize(ptrs: torch.Tensor, H: int, I: int, K: int) -> None:
     require_device(ptrs)
     if ptrs.dtype != torch.int64:
         raise Exl3Error("blob_unplanarize: ptrs must be int64")
-    check(lib().exl3_blob_unplanarize(ptr(ptrs.contiguous()), ptrs.numel(), int(H), int(I), int(K), stream_of(ptrs)),
+    ptrs = ptrs.contiguous()
+    check(lib().exl3_blob_unplanarize(ptr(ptrs), ptrs.numel(), int(H), int(I), int(K), stream_of(ptrs)),
           "blob_unplanarize")
 
 
@@ -262,8 +263,9 @@ def moe_align(topk_ids: torch.Tensor, topk_w: torch.Tensor, E: int, shared: int 
     pair_tok = torch.full((M * slots,), -1, dtype=torch.int32, device=dev)
     pair_w = torch.zeros(M * slots, dtype=torch.float32, device=dev)
     pair_of = torch.empty(M * slots, dtype=torch.int32, device=dev)
-    check(lib().exl3_moe_align(ptr(topk_ids.contiguous()), ptr(topk_w.contiguous()), M, k, E, shared, ptr(counts),
-                               ptr(pair_tok), ptr(pair_w), ptr(pair_of), stream_of(topk_ids)), "moe_align")
+    topk_ids, topk_w = topk_ids.contiguous(), topk_w.contiguous()
+    check(lib().exl3_moe_align(ptr(topk_ids), ptr(topk_w), M, k, E, shared, ptr(counts), ptr(pair_tok), ptr(pair_w),
+                               ptr(pair_of), stream_of(topk_ids)), "moe_align")
     return counts, pair_tok, pair_w, pair_of
 
 
