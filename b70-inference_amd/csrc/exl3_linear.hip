@@ -456,26 +456,27 @@ static int gemv_splits(int strips, int nblk, int rows) {
     return P < 1 ? 1 : P;
 }
 
-// Dense linear on MFMA (exl3_mfma.hip): scratch of a call, and the call (in `fixed` scratch if given).
-int linear_mfma_scratch(int64_t m, int64_t n, int64_t k, int S, int K, size_t* bytes);
-int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n, int K,
-                       void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
+// Dense linear on MFMA (exl3_mfma.hip): its plan in at most `most` bytes of scratch, and the call (in `fixed` scratch if given).
+int linear_mfma_plan(int64_t m, int64_t n, int64_t k, int S, int K, size_t most, LinPlan* pl, bool* fits);
+int launch_linear_mfma(const LinPlan& pl, const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n,
+                       int K, void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
                        const uint16_t* svh, char* fixed, size_t fixed_bytes, hipStream_t st);
 constexpr int kLinearMfmaMinRows = 9;
 constexpr size_t kNoAllocPartBytes = 16u << 20;              // fixed scratch of the allocation-free entry point
 
-// Rows that take the MFMA GEMM: more than the GEMV takes per pass, and five or more on large matrices. The GEMV's time
-// grows with the rows, the GEMM's three launches cost about 15 us whatever the matrix; us, GEMV / GEMM: 5376 -> 21504 at
-// 4 / 6 / 8 rows 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096
-// 9.9 / 16.7, 12.1 / 16.5, 13.0 / 16.6. Below nine rows only where its scratch fits the allocation-free entry point's (the
-// two entry points give the same bits) and, under stream capture, what the workspace holds. forced > 0: the rows from which it is taken (tests).
-static int takes_mfma(int64_t m, int64_t k, int64_t n, int S, int K, size_t room, int forced, bool* yes) {
-    *yes = m >= (forced ? forced : kLinearMfmaMinRows);
-    if (*yes || forced || m < 5 || k * n < 200000000 / (m - 2)) return EXL3_OK;
-    size_t bytes = 0;
-    const int rc = linear_mfma_scratch(m, n, k, S, K, &bytes);
-    *yes = !rc && bytes <= kNoAllocPartBytes && bytes <= room;
-    return rc;
+// Split-K partials of the GEMV, in slots of kGemvMaxRows rows.
+static size_t gemv_part_bytes(int strips, int P) { return (size_t)strips * P * kGemvMaxRows * 128 * sizeof(float); }
+
+// Rows that take the MFMA GEMM: more than the GEMV takes per pass, and five to eight of large matrices (linear_few_rows). Those
+// keep to the scratch that the GEMV would take, so that a call fits wherever its GEMV does (a captured call's workspace, the
+// allocation-free entry point's array) and the choice follows from the shape. forced > 0: the rows from which it is taken (tests).
+static int takes_mfma(int64_t m, int64_t k, int64_t n, int S, int K, int forced, LinPlan* pl, bool* yes) {
+    *yes = false;
+    const bool few = !forced && m < kLinearMfmaMinRows;
+    if (few ? !linear_few_rows(m, n, k) : m < forced) return EXL3_OK;
+    const int strips = (int)(n / 128);
+    const size_t most = few ? gemv_part_bytes(strips, gemv_splits(strips, (int)(k / 128), (int)m)) : SIZE_MAX;
+    return linear_mfma_plan(m, n, k, S, K, most, pl, yes);
 }
 
 // Launches over chunks of up to kGemvMaxRows rows of `ga` (x, out and m describe all rows; the workspace holds
@@ -536,7 +537,7 @@ int launch_gemv(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uin
     const bool tagged = m == 1;
     Workspace ws;
     int rc = tagged ? workspace(0, (size_t)strips * P * 128, st, &ws)
-                    : workspace((size_t)strips * P * kGemvMaxRows * 128 * sizeof(float), (size_t)strips, st, &ws);
+                    : workspace(gemv_part_bytes(strips, P), (size_t)strips, st, &ws);
     if (rc) return rc;
     GemvArgs ga = gemv_args(A, a_ld, k, tr, n, C, c_ld, suh, S, sonb, svh, P);
     if (tagged) {
@@ -715,11 +716,11 @@ int exl3_linear_sharded(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, c
     const uint32_t* tr = reinterpret_cast<const uint32_t*>(B);
     const int S = (int)n_shards;
     bool mfma = false;
-    const int rc = takes_mfma(m, k, n, S, K, workspace_room((hipStream_t)stream), env_int("EXL3MI_MFMA_MIN_ROWS", 0),
-                              &mfma);
+    LinPlan pl;
+    const int rc = takes_mfma(m, k, n, S, K, env_int("EXL3MI_MFMA_MIN_ROWS", 0), &pl, &mfma);
     if (rc) return rc;
     if (mfma)
-        return launch_linear_mfma(A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh, nullptr,
+        return launch_linear_mfma(pl, A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh, nullptr,
                                   0, (hipStream_t)stream);
     return launch_gemv(A, a_ld, m, k, tr, n, K, C, c_ld, c_dtype == EXL3_F32, suh, S, shard_of_nb, svh,
                        (hipStream_t)stream);
@@ -754,7 +755,7 @@ int exl3_gemm_noalloc(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, con
     EXL3_CHECK_ARG(strips <= (int64_t)kNoAllocCounters, "exl3_gemm_noalloc: n=%lld exceeds the %zu columns of the "
                    "fixed scratch", (long long)n, kNoAllocCounters * 128);
     const int P = gemv_splits((int)strips, (int)(k / 128), (int)m);
-    const size_t part = (size_t)strips * P * kGemvMaxRows * 128 * sizeof(float);
+    const size_t part = gemv_part_bytes((int)strips, P);
     EXL3_CHECK_ARG(part <= kNoAllocPartBytes, "exl3_gemm_noalloc: %zu bytes of split-K partials needed, the fixed "
                    "scratch holds %zu", part, kNoAllocPartBytes);
     hipStream_t st = (hipStream_t)stream;
@@ -762,9 +763,10 @@ int exl3_gemm_noalloc(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, con
     int rc = noalloc_scratch(st, &sc);
     if (rc) return rc;
     bool mfma = false;
-    if ((rc = takes_mfma(m, k, n, 1, K, kNoAllocPartBytes, 0, &mfma))) return rc;
+    LinPlan pl;
+    if ((rc = takes_mfma(m, k, n, 1, K, 0, &pl, &mfma))) return rc;
     if (mfma)
-        return launch_linear_mfma(A, a_ld, m, k, reinterpret_cast<const uint32_t*>(B), n, K, C, c_ld, c_dtype == EXL3_F32,
+        return launch_linear_mfma(pl, A, a_ld, m, k, reinterpret_cast<const uint32_t*>(B), n, K, C, c_ld, c_dtype == EXL3_F32,
                                   suh, 1, nullptr, svh, sc, kNoAllocPartBytes, st);
     GemvArgs ga = gemv_args(A, a_ld, k, reinterpret_cast<const uint32_t*>(B), n, C, c_ld, suh, 1, nullptr, svh, P);
     ga.part = reinterpret_cast<float*>(sc);

@@ -202,9 +202,11 @@ struct LinArgs {
     const uint16_t* svh;
     void* out;
     int64_t out_ld;
-    float* part;                                     // [P][m][n] when P > 1
+    float* part;                                     // null: the epilogue writes out; else [P][m][n], the splits' partials
     int m, k, n, nblk;
-    int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits, 128-blocks per split
+    int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits of this launch, 128-blocks
+                                                     // per split
+    int p0;                                          // first split of this launch; > 0: added to part (P = 1)
     int f32;
     const int64_t* tab;                              // not null: an expert's addresses (ItemDesc::tab), its down projection
                                                      // in place of tr and svh

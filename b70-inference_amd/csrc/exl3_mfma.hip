@@ -895,7 +895,6 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
     l.out = a.out;
     l.out_ld = a.out_ld;
     l.f32 = a.out_f32;
-    l.part = a.y;
     l.m = a.M;
     l.k = a.I;
     l.n = a.H;
@@ -903,11 +902,14 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
     l.nrb = (a.M + a.block_rows - 1) / a.block_rows;
     l.ncb = (a.H + 255) / 256;
     l.bps = (l.nblk + a.dense_P - 1) / a.dense_P;
-    l.P = (l.nblk + l.bps - 1) / l.bps;
+    const int P = (l.nblk + l.bps - 1) / l.bps;                    // = dense_P
+    l.P = P > 1 && a.dense_sets == 1 ? 1 : P;                      // splits (and partials) of a launch
+    l.part = P > 1 ? a.y : nullptr;
     const int64_t nx = ((int64_t)l.nrb * l.ncb * l.P + 7) / 8 * 8;
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: grid too large");
-    EXL3_LAUNCH("mlp_down_wide", linear_wide_pick(a.block_rows / 32, 1, a.Kd), dim3((unsigned)nx), dim3(256), 0, st, l);
-    if (l.P > 1)
+    for (; l.p0 < P; l.p0 += l.P)                                  // (a later one adds: not to be run twice)
+        EXL3_LAUNCH("mlp_down_wide", linear_wide_pick(a.block_rows / 32, 1, a.Kd), dim3((unsigned)nx), dim3(256), 0, st, l);
+    if (P > 1)
         EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, dim3((unsigned)((l.m + 3) / 4), (unsigned)(l.n / 128)),
                     dim3(256), 0, st, l);
     return EXL3_OK;
@@ -956,49 +958,32 @@ int launch_moe_mfma(const MoeArgs& a, hipStream_t st) {
     return a.dense_P > 0 ? launch_dense_down(a, st) : launch_moe_combine(a, st);
 }
 
-// Plan of a call of m rows, with at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the
-// scratch of the partials), and its scratch.
-static int linear_call_plan(int64_t m, int64_t n, int64_t k, int K, LinPlan* pl) {
-    const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
-    const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
+// Plan of a call of m rows in at most `most` bytes of scratch; *fits: whether there is one.
+int linear_mfma_plan(int64_t m, int64_t n, int64_t k, int S, int K, size_t most, LinPlan* pl, bool* fits) {
     int cus = 0;
-    const int rc = device_cus(&cus);
-    const int rg = env_int("EXL3MI_LINEAR_BLOCK", 0);              // forced row groups of 32 per block: 1, 2, 4 or 8
-    if (!rc)
-        *pl = linear_plan(m, n, k, K, rg == 1 || rg == 2 || rg == 4 || rg == 8 ? rg : 0,
-                          ((m <= 32 ? 768 : 512) + ts - 1) / ts, cus);
-    return rc;
-}
-static size_t linear_call_bytes(int64_t m, int64_t n, int64_t k, int S, int P) {
-    return carve_size((size_t)S * m * k, 2) + carve_size((size_t)S * m * (k / 128), 4) +
-           (P > 1 ? carve_size((size_t)P * m * n, 4) : 0);
-}
-int linear_mfma_scratch(int64_t m, int64_t n, int64_t k, int S, int K, size_t* bytes) {
-    LinPlan pl;
-    const int rc = linear_call_plan(m, n, k, K, &pl);
-    if (!rc) *bytes = linear_call_bytes(m, n, k, S, pl.P);
-    return rc;
+    if (const int rc = device_cus(&cus)) return rc;
+    const int v = env_int("EXL3MI_LINEAR_BLOCK", 0);               // forced row groups of 32 per block: 1, 2, 4 or 8
+    *fits = linear_call_plan(m, n, k, S, K, v == 1 || v == 2 || v == 4 || v == 8 ? v : 0, cus, most, pl);
+    if (const int jobs = env_int("EXL3MI_LINEAR_JOBS", 0); jobs && *fits) {        // forced workgroup target
+        const int nblk = (int)(k / 128);
+        const int64_t R = 32 * pl->RG, tiles = (m + R - 1) / R * ((n + 255) / 256), want = (jobs + tiles - 1) / tiles;
+        const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
+        pl->bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
+        pl->P = (nblk + pl->bps - 1) / pl->bps;
+        while (pl->RG > 1 && !a_span_ok(m < 32 * pl->RG ? m : 32 * pl->RG, 128LL * pl->bps)) pl->RG /= 2;
+        *fits = linear_call_bytes(m, n, k, S, pl->P) <= most;
+    }
+    return EXL3_OK;
 }
 
-// Dense linear on MFMA: input transform, blocks of 32 .. 256 rows x 256 columns and, with k-splits, the reduction. Scratch
-// from the workspace, or `fixed` (fixed_bytes of it; those launches also bypass the opt-in event profiler).
-int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n, int K,
-                       void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
+// Dense linear on MFMA by `pl`: input transform, blocks of 32 .. 256 rows x 256 columns and, with k-splits, the reduction.
+// Scratch from the workspace, or `fixed` (fixed_bytes of it; those launches also bypass the opt-in event profiler).
+int launch_linear_mfma(const LinPlan& pl, const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const uint32_t* tr, int64_t n,
+                       int K, void* C, int64_t c_ld, bool f32, const uint16_t* suh, int S, const int32_t* sonb,
                        const uint16_t* svh, char* fixed, size_t fixed_bytes, hipStream_t st) {
-    const int nblk = (int)(k / 128);
+    const int nblk = (int)(k / 128), R = 32 * pl.RG;
     if (m > 0x7FFFFFFF / 64 || k > 0x7FFFFFFF || n > 0x7FFFFFFF || nblk > 65535)
         return fail(EXL3_ERR_INVALID, "exl3_gemm: shape too large");
-    LinPlan pl;
-    int rc = linear_call_plan(m, n, k, K, &pl);
-    if (rc) return rc;
-    if (const int jobs = env_int("EXL3MI_LINEAR_JOBS", 0)) {       // forced workgroup target
-        const int64_t R = 32 * pl.RG, tiles = (m + R - 1) / R * ((n + 255) / 256), want = (jobs + tiles - 1) / tiles;
-        const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
-        pl.bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
-        pl.P = (nblk + pl.bps - 1) / pl.bps;
-        while (pl.RG > 1 && !a_span_ok(m < 32 * pl.RG ? m : 32 * pl.RG, 128LL * pl.bps)) pl.RG /= 2;
-    }
-    const int R = 32 * pl.RG;
     LinArgs a = {};
     a.m = (int)m;
     a.k = (int)k;
@@ -1008,12 +993,10 @@ int launch_linear_mfma(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, co
     a.ncb = (int)((n + 255) / 256);
     a.bps = pl.bps;
     a.P = pl.P;
-    const size_t bytes = linear_call_bytes(m, n, k, S, a.P);
     Carve cv{fixed, fixed_bytes};
     if (!fixed) {
         Workspace ws;
-        rc = workspace(bytes, 0, st, &ws);
-        if (rc) return rc;
+        if (const int rc = workspace(linear_call_bytes(m, n, k, S, a.P), 0, st, &ws)) return rc;
         cv = Carve{ws.scratch, ws.scratch_bytes};
     }
     _Float16* xh = cv.take<_Float16>((size_t)S * m * k);

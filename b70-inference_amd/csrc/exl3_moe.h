@@ -120,7 +120,9 @@ struct MoeArgs {
     const int* cls_list;               // [kRowClasses][max_blocks] block indices by row class
     const int* cls_cnt;                // [kRowClasses] blocks per class
     _Float16* xh;                      // [pairs][2][H] transformed gate / up inputs of MFMA rows; uniform gate|up K:
-                                       // per block [2][cnt * H] in block_unit order (exl3_mfma.h)
+                                       // per block [2][cnt * H] in block_unit order (exl3_mfma.h). All uniform: shares
+                                       // its memory with y (a block's rows take the same bytes in both, and its down
+                                       // kernel runs after its gate|up kernel)
     float* xsum;                       // [pairs][2][H / 128] block sums of xh (the MFMA rows' affine term)
     float* asum;                       // [pairs][I / 128] block sums of abuf (MFMA rows)
     int* pair_tok;
@@ -134,10 +136,11 @@ struct MoeArgs {
     // intermediates (workspace)
     uint16_t* abuf;                    // [pairs][I] fp16, Hadamard-domain down input (MFMA rows at uniform down K: per
                                        // block in block_unit order)
-    float* y;                          // [pairs][H] fp32, weighted expert outputs (dense_P > 0: [dense_P][M][H] down
+    float* y;                          // [pairs][H] fp32, weighted expert outputs (dense_P > 0: [dense_sets][M][H] down
                                        // partials)
     int dense_P;                       // > 0: one expert takes every token with weight 1 (a dense MLP) on the MFMA
                                        // path: k-splits of its down projection, which runs as a dense linear
+    int dense_sets;                    // partials held: dense_P, or 1: the splits run one after another and add up
     float* part_gu;
     int* cnt_gu;
     int P_gu, nblk_h;

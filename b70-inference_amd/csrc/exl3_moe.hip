@@ -1158,11 +1158,12 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     Workspace ws;
     const size_t n_gu = (size_t)max_items * nbI, n_d = (size_t)max_items * nbH;
     const bool use_mfma = a.max_blocks > 0;
+    const bool xy = use_mfma && a.Kg > 0 && a.Kd > 0;           // xh and y share their memory
     size_t y_elems = (size_t)npairs * a.H;
     const auto scratch = [&] {
         return carve_size(1, 4) + carve_size(max_items, sizeof(ItemDesc)) +
                    carve_size(a.max_blocks, sizeof(ItemDesc)) +
-                   (use_mfma ? carve_size(npairs * 2 * a.H, 2) + carve_size(npairs * 2 * (a.H / 128), 4) +
+                   (use_mfma ? (xy ? 0 : carve_size(npairs * 2 * a.H, 2)) + carve_size(npairs * 2 * (a.H / 128), 4) +
                                    carve_size(npairs, 4) +
                                    carve_size(npairs * (a.I / 128), 4) + carve_size(kRowClasses * ((size_t)a.max_blocks + 1), 4)
                              : 0) +
@@ -1171,14 +1172,14 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
                    carve_size(npairs * a.I, 2) + carve_size(y_elems, 4) +
                    carve_size(n_gu * a.P_gu * 2 * MR * 128, 4) + carve_size(n_d * a.P_d * MR * 128, 4);
     };
-    if (use_mfma && a.E == 1 && a.topk == 0 && a.shared == 0 && a.Kg > 0 && a.Kd > 0) {
-        // a dense MLP: its down projection as a dense linear; under stream capture with the splits that the scratch holds
-        const size_t room = workspace_room(st);
-        for (int cap = 8;; cap = a.dense_P - 1) {
-            const int rc = dense_down_splits(a.M, a.H, a.I, a.Kd, a.block_rows, cap, &a.dense_P);
-            if (rc) return rc;
-            y_elems = (size_t)a.dense_P * npairs * a.H;
-            if (a.dense_P == 1 || scratch() <= room) break;
+    if (a.dense_P > 0) {
+        // Under stream capture a workspace without room for all splits' partials holds one set, and the splits run one after
+        // another: the same sums, the scratch of an unsplit call.
+        a.dense_sets = a.dense_P;
+        y_elems = (size_t)a.dense_sets * npairs * a.H;
+        if (scratch() > workspace_room(st)) {
+            a.dense_sets = 1;
+            y_elems = (size_t)npairs * a.H;
         }
     }
     const size_t bytes = scratch();
@@ -1191,7 +1192,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.items = items;
     ItemDesc* blocks = a.max_blocks ? c.take<ItemDesc>(a.max_blocks) : nullptr;
     a.blocks = blocks;
-    a.xh = use_mfma ? c.take<_Float16>(npairs * 2 * a.H) : nullptr;
+    a.xh = use_mfma && !xy ? c.take<_Float16>(npairs * 2 * a.H) : nullptr;
     a.xsum = use_mfma ? c.take<float>(npairs * 2 * (a.H / 128)) : nullptr;
     a.asum = use_mfma ? c.take<float>(npairs * (a.I / 128)) : nullptr;
     a.pair_e = use_mfma ? c.take<int>(npairs) : nullptr;
@@ -1205,6 +1206,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.tok_nvalid = c.take<int>(a.M);
     a.abuf = c.take<uint16_t>(npairs * a.I);
     a.y = c.take<float>(y_elems);
+    if (xy) a.xh = reinterpret_cast<_Float16*>(a.y);
     a.part_gu = c.take<float>(n_gu * a.P_gu * 2 * MR * 128);
     a.part_d = c.take<float>(n_d * a.P_d * MR * 128);
     if (!a.part_d) return fail(EXL3_ERR_INVALID, "moe: workspace carve failed");
@@ -1421,7 +1423,11 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     a.max_items = (int)mi;
     const bool wide = a.Kg > 0 && a.Kd > 0;
     a.block_rows = wide ? moe_wide_rows(M, E, npairs, a.H, a.I, a.Kg, a.Kd, env_int("EXL3MI_MOE_BLOCK", 0)) : kMfmaRows;
-    a.max_blocks = mfma ? (int)(npairs / (wide ? 32 : kMfmaRows) + (E < npairs ? E : npairs) + 1) : 0;
+    if (mfma && wide && E == 1 && a.topk == 0 && a.shared == 0) {          // a dense MLP: its down projection as a dense linear
+        const int rc = dense_down_splits(M, a.H, a.I, a.Kd, a.block_rows, 8, &a.dense_P);
+        if (rc) return rc;
+    }
+    a.max_blocks = mfma ? (int)moe_max_blocks(npairs, E, a.block_rows, a.dense_P > 0) : 0;
     EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= (wide ? 1 << 21 : 65535) &&
                        (int64_t)(a.max_blocks + 8) * (a.I > a.H ? a.I / 128 : a.H / 128) < 0x7FFFFFFF,
                    "exl3_moe_forward: grid too large");

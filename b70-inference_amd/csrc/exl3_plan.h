@@ -1,9 +1,14 @@
-// Host-side choices of the wide-block kernels (exl3_wide.h): row blocks and k-splits. Plain C++ without device code.
+// Host-side choices of the wide-block kernels (exl3_wide.h): row blocks, k-splits, scratch. Plain C++ without device code.
+// They follow from the shape alone, never from what the workspace holds: a call gives the same bits eager and captured.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace exl3 {
+
+// Bytes that n elements take in a workspace request (Carve).
+inline size_t carve_size(size_t n, size_t elem) { return (n * elem + 255) & ~(size_t)255; }
 
 // The wide kernels address the A rows of a block (`rows` rows, k columns, fp16) by 32-bit offsets from its first byte, in a
 // buffer resource of 2^31 - 1 bytes: loads past it return zero. Blocks are cut so that they stay inside.
@@ -51,6 +56,29 @@ inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64
     return tb == 1e30f && rg > 1 ? linear_plan(m, n, k, K, rg / 2, cap, cus) : best;
 }
 
+// Scratch of a dense linear on the MFMA GEMM: transformed rows of S shards, their block sums, partials of P > 1 splits.
+inline size_t linear_call_bytes(int64_t m, int64_t n, int64_t k, int S, int P) {
+    return carve_size((size_t)S * m * k, 2) + carve_size((size_t)S * m * (k / 128), 4) +
+           (P > 1 ? carve_size((size_t)P * m * n, 4) : 0);
+}
+
+// Plan of such a call, with at most the splits that cover the device with blocks of 16, 32 or 64 rows (bounds the partials)
+// and that fit `most` bytes of scratch. False if not even one split fits.
+inline bool linear_call_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int cus, size_t most, LinPlan* pl) {
+    const int rs = m <= 16 ? 16 : m <= 32 ? 32 : 64;
+    const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
+    int64_t cap = ((m <= 32 ? 768 : 512) + ts - 1) / ts;
+    while (cap > 1 && linear_call_bytes(m, n, k, S, (int)cap) > most) --cap;
+    *pl = linear_plan(m, n, k, K, rg, cap, cus);
+    return linear_call_bytes(m, n, k, S, pl->P) <= most;
+}
+
+// Whether five to eight rows (what the decode GEMV takes in one pass) run on the MFMA GEMM instead. The GEMV's time grows with
+// the rows, the GEMM's three launches cost about 15 us on a small matrix; us, GEMV / GEMM: 5376 -> 21504 at 4 / 6 / 8 rows
+// 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096 9.9 / 16.7,
+// 12.1 / 16.5, 13.0 / 16.6.
+inline bool linear_few_rows(int64_t m, int64_t n, int64_t k) { return m >= 5 && m <= 8 && k * n >= 200000000 / (m - 2); }
+
 // Row block of the prefill MoE (M tokens, `npairs` rows over E experts, H -> I -> H; uniform K: 1 .. 8). 32 (one class, one
 // launch per projection) up to 64 tokens, 160 where experts take few rows: forking the launches by class costs more there
 // (10 to 25 us) than decoding the experts with more rows again; 64 where an expert takes 28 to 64 rows on average (and for
@@ -63,6 +91,12 @@ inline int moe_wide_rows(int64_t M, int64_t E, int64_t npairs, int64_t H, int64_
     if (rows == 128 && (Kg > 5 || Kd > 5)) rows = 64;
     while (rows > 32 && !a_span_ok(npairs < rows ? npairs : rows, H > I ? H : I)) rows /= 2;
     return rows;
+}
+
+// MFMA blocks of a call of npairs rows over E experts, at most: an expert's last block may hold few rows; with 32-row blocks
+// and with 128-row ones whose remainder is cut (`whole`: it is not) there is one per 32 rows more.
+inline int64_t moe_max_blocks(int64_t npairs, int64_t E, int rows, bool whole) {
+    return npairs / (rows == 32 || (rows > 64 && !whole) ? 32 : 64) + (E < npairs ? E : npairs) + 1;
 }
 
 }  // namespace exl3

@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include "../../include/exl3mi.h"
+#include "exl3_plan.h"
 
 namespace exl3 {
 
@@ -89,7 +90,6 @@ struct Carve {
         return r;
     }
 };
-inline size_t carve_size(size_t n, size_t elem) { return (n * elem + 255) & ~(size_t)255; }
 
 inline bool aligned(const void* p, size_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     if (!wide_tile(a, rb, nb, p)) return;
     const int r0 = rb * 32 * RG;
     const int cnt = a.m - r0 < 32 * RG ? a.m - r0 : 32 * RG;
-    const int kb0 = p * a.bps, nkb = a.nblk - kb0 < a.bps ? a.nblk - kb0 : a.bps;
+    const int kb0 = (a.p0 + p) * a.bps, nkb = a.nblk - kb0 < a.bps ? a.nblk - kb0 : a.bps;
     const int tn = a.n / 16;
     const int nhalf = 2 * nb + 1 < a.n / 128 ? 2 : 1;
     int shard[NPL];                                  // shard of each plane (the block's 128-column half; in [0, S))
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[rg][np][i] = 0.f;
     L.run(acc);
-    if (a.P > 1) {                                   // fp32 partials, affine applied
+    if (a.part) {                                    // fp32 partials, affine applied
         if (hw >= nhalf) return;
         float* part = a.part + (size_t)p * a.m * a.n + (size_t)r0 * a.n + nb * 256 + 64 * wave + (lane & 31);
 #pragma unroll
@@ -88,8 +88,14 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
                 const int r = 32 * rg + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
                 const float sx = kMul1C2 * rsum[NPL > 1 ? hw : 0][r];
                 if (r < cnt) {
-                    part[(size_t)r * a.n] = kMul1C1 * acc[rg][0][i] + sx;
-                    part[(size_t)r * a.n + 32] = kMul1C1 * acc[rg][1][i] + sx;
+                    float v0 = kMul1C1 * acc[rg][0][i] + sx, v1 = kMul1C1 * acc[rg][1][i] + sx;
+                    if (a.p0 > 0) {                  // the sum of the reduce kernel, in its order and with its roundings
+                        asm volatile("" : "+v"(v0), "+v"(v1));       // (no fused multiply-add across it)
+                        v0 += part[(size_t)r * a.n];
+                        v1 += part[(size_t)r * a.n + 32];
+                    }
+                    part[(size_t)r * a.n] = v0;
+                    part[(size_t)r * a.n + 32] = v1;
                 }
             }
         return;

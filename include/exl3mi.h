@@ -110,11 +110,12 @@ int exl3_gemm(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const int16
               int64_t c_ld, int c_dtype, const uint16_t* suh, uint16_t* A_had, const uint16_t* svh, int cb,
               void* stream);
 
-/* exl3_gemm for up to 8 rows (same kernels and results bit for bit) without the library workspace: its scratch (split-K
+/* exl3_gemm for up to 8 rows (same kernels and results bit for bit, eager or captured: the kernel follows from the shape;
+ * only the EXL3MI_MFMA_MIN_ROWS override moves exl3_gemm alone) without the library workspace: its scratch (split-K
  * partials, arrival counters, the transformed rows of calls on the MFMA GEMM) lives in a fixed device array (16 MiB +
  * 64 KiB per device, held until the process ends), so the call never allocates, e.g. under HIP graph capture or in a
- * serving loop that must not allocate. Limits: m <= 8, n <= 2 097 152 columns, and strips (n / 128) x k-splits x 8 x 128 x 4 bytes of partials
- * <= 16 MiB (k-splits <= 16; e.g. n = 21504 at any k fits); larger shapes return EXL3_ERR_INVALID. Every call on a
+ * serving loop that must not allocate. Limits: m <= 8, n <= 2 097 152 columns, and strips (n / 128) x k-splits x 8 x
+ * 128 x 4 bytes of partials <= 16 MiB (e.g. n = 21504 at any k fits); larger shapes return EXL3_ERR_INVALID. Every call on a
  * device shares that device's array: calls that overlap in time (two streams, two threads) race. A_had is dropped.
  * No counterpart in the reference: an entry point for callers that cannot allocate. */
 int exl3_gemm_noalloc(const uint16_t* A, int64_t a_ld, int64_t m, int64_t k, const int16_t* B, int64_t n, int K,

@@ -18,6 +18,11 @@ extern "C" void plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap
     out[1] = p.P;
     out[2] = p.bps;
 }
+extern "C" int64_t call_bytes(int64_t m, int64_t n, int64_t k, int S, int K, int cus, uint64_t most) {
+    LinPlan p;
+    return linear_call_plan(m, n, k, S, K, 0, cus, most, &p) ? (int64_t)linear_call_bytes(m, n, k, S, p.P) : -1;
+}
+extern "C" int64_t max_blocks(int64_t npairs, int64_t E, int rows, int whole) { return moe_max_blocks(npairs, E, rows, whole); }
 extern "C" int moe_rows(int64_t M, int64_t E, int64_t npairs, int64_t H, int64_t I, int Kg, int Kd, int forced) {
     return moe_wide_rows(M, E, npairs, H, I, Kg, Kd, forced);
 }
@@ -39,6 +44,10 @@ def lib(tmp_path_factory):
     L.plan.restype = None
     L.moe_rows.argtypes = [i64] * 5 + [i32] * 3
     L.moe_rows.restype = i32
+    L.call_bytes.argtypes = [i64, i64, i64, i32, i32, i32, ctypes.c_uint64]
+    L.call_bytes.restype = i64
+    L.max_blocks.argtypes = [i64, i64, i32, i32]
+    L.max_blocks.restype = i64
     return L
 
 
@@ -76,3 +85,54 @@ def test_moe_block_offsets_fit_32_bits(lib, width, forced):
             rows = lib.moe_rows(M, E, M * slots, H, I, 2, 2, forced)
             assert rows in (32, 64, 128)
             assert last_byte(rows, width) <= (1 << 31) - 1
+
+
+SHAPES = [(1024, 4096), (4096, 4096), (4096, 14336), (5376, 21504), (21504, 5376), (2048, 131072), (8192, 1024), (12288, 128)]
+
+
+def gemv_bytes(m, n, k):
+    """The decode GEMV's partials (csrc/exl3_linear.hip: gemv_splits, gemv_part_bytes)."""
+    strips, nblk = n // 128, k // 128
+    P = min(-(-1024 // strips), 8 if m <= 2 else 16)
+    return strips * max(1, min(max(P, -(-nblk // 8)), nblk)) * 8 * 128 * 4
+
+
+@pytest.mark.parametrize("k,n", SHAPES)
+@pytest.mark.parametrize("S", [1, 3, 64])
+def test_few_rows_keep_to_the_gemv_scratch(lib, k, n, S):
+    """Five to eight rows on the MFMA GEMM never need more scratch than the GEMV that they replace, so that the choice can
+    follow from the shape alone; with one shard they always fit."""
+    for m in range(5, 9):
+        for K in range(1, 9):
+            b = lib.call_bytes(m, n, k, S, K, CUS, gemv_bytes(m, n, k))
+            assert b <= gemv_bytes(m, n, k)
+            assert b > 0 or S > 1 or n < 4096
+
+
+@pytest.mark.parametrize("k,n", SHAPES)
+def test_call_scratch_is_bounded(lib, k, n):
+    """Partials of at most as many splits as fill the device with blocks of 16, 32 or 64 rows (4, 3 or 2 workgroups per CU)."""
+    for m in (9, 16, 17, 32, 33, 100, 512, 2048):
+        rows, per_cu = (16, 4) if m <= 16 else (32, 3) if m <= 32 else (64, 2)
+        nblk, tiles = k // 128, -(-m // rows) * -(-n // 256)
+        P = min(-(-per_cu * CUS // tiles), max(1, nblk // 2))
+        P = -(-nblk // -(-nblk // P))
+        up = lambda v: -(-v // 256) * 256  # noqa: E731
+        for S in (1, 3):
+            most = up(2 * S * m * k) + up(4 * S * m * nblk) + (up(4 * P * m * n) if P > 1 else 0)
+            for K in (2, 4, 6, 8):
+                assert lib.call_bytes(m, n, k, S, K, CUS, 1 << 62) <= most
+
+
+def blocks_of(c, rows, whole):
+    """Row blocks of an expert with c rows (BlockCut in csrc/exl3_moe.h)."""
+    full, rem = divmod(c, rows)
+    return full + (-(-rem // 32) if rows > 64 and not whole and rem <= 64 else rem > 0)
+
+
+@pytest.mark.parametrize("rows,whole", [(32, False), (64, False), (128, False), (64, True), (128, True)])
+def test_block_list_holds_every_routing(lib, rows, whole):
+    for c in range(1, 600):
+        for E in (1, 2, 7):
+            assert E * blocks_of(c, rows, whole) <= lib.max_blocks(E * c, E, rows, whole)
+    assert blocks_of(33, rows, whole) + 5 * blocks_of(1, rows, whole) <= lib.max_blocks(38, 6, rows, whole)

@@ -2,6 +2,7 @@
 device status word and the next call clears it (the wait is forced to give up from the host with a tiny spin limit, so every kernel
 still exits normally), and workspace growth keeps buffers alive that a HIP graph captured earlier still uses."""
 import os
+import shutil
 
 import numpy as np
 import pytest
@@ -197,3 +198,87 @@ def test_timeout_in_replay_resets_outgrown_counters_and_not_under_capture(exl3, 
     del g_good, g_bad, g_cap
     torch.cuda.synchronize()
     lib.release_workspace()
+
+
+@pytest.fixture
+def fresh(exl3, monkeypatch, tmp_path):
+    """The library loaded once more, from a copy: its workspace starts empty, whatever ran before."""
+    lib = exl3._lib
+    path = shutil.copy(lib.LIB_PATH, tmp_path / "libexl3mi_copy.so")
+    monkeypatch.setattr(lib, "_lib", None)
+    monkeypatch.setattr(lib, "LIB_PATH", str(path))
+    return lib
+
+
+def _hold(lib, nbytes):
+    """A workspace that holds nbytes and little more (it is allocated with a quarter to spare, in whole MiB)."""
+    lib.reserve_workspace(nbytes * 4 // 5, 1 << 16)
+
+
+@pytest.mark.parametrize("k,n,M", [(8192, 8192, 8), (2048, 34816, 7), (5376, 21504, 6)])
+def test_few_rows_captured_in_the_gemv_scratch(exl3, oracle, fresh, k, n, M):
+    """Five to eight rows of a large matrix, captured where the workspace holds what a decode GEMV takes and no more: the
+    bits of the eager call and of the allocation-free one, whatever the workspace holds."""
+    lib = fresh
+    g = torch.Generator().manual_seed(4300 + M)
+    tr = torch.randint(-32768, 32768, (k // 16, n // 16, 32), generator=g, dtype=torch.int16).cuda()
+    suh, svh = ((torch.randint(0, 2, (d,), generator=g) * 2 - 1).half().cuda() for d in (k, n))
+    x = torch.randn(M, k, generator=g).half().cuda()
+    y, eager, noalloc = (torch.empty(M, n, device="cuda") for _ in range(3))
+    strips, nblk = n // 128, k // 128
+    splits = min(max(min(-(-1024 // strips), 16), -(-nblk // 8)), nblk)
+    _hold(lib, strips * splits * 8 * 128 * 4)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        exl3.exl3_gemm(x, tr, y, suh, None, svh)
+    for grow in (False, True):
+        if grow:
+            lib.reserve_workspace(1 << 28, 1 << 16)
+        exl3.exl3_gemm(x, tr, eager, suh, None, svh)
+        exl3.exl3_gemm_noalloc(x, tr, noalloc, suh, svh)
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager) and torch.equal(y, noalloc)
+    cols = slice(0, 128)
+    ref = oracle.exl3_linear(x.cpu().numpy(), tr[:, :8].contiguous().cpu().numpy(), suh.cpu().numpy(),
+                             svh[cols].cpu().numpy(), 2, np.float32)
+    assert max_rel(y[:, cols].cpu().numpy(), ref) <= MAX_REL
+    del graph
+    torch.cuda.synchronize()
+
+
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+@pytest.mark.parametrize("M,H,I", [(40, 8192, 1024), (300, 1024, 2048)])
+def test_dense_mlp_captured_in_the_scratch_of_one_split(exl3, oracle, fresh, monkeypatch, M, H, I):
+    """A dense MLP's k-split down projection captured where the workspace holds one set of partials only (a set is more than
+    the MiB to spare): the splits run one after another and give the eager call's bits."""
+    lib = fresh
+    tables, orc = make_experts(exl3, oracle, 1, H, I, 3, 3, 4400)
+    x = torch.randn(M, H, generator=torch.Generator().manual_seed(4401)).half().cuda()
+    ids, w = torch.empty(M, 0, dtype=torch.int32, device="cuda"), torch.empty(M, 0, device="cuda")
+    out = torch.empty(M, H, device="cuda")
+    assert 4 * M * H > 1 << 20
+    monkeypatch.setenv("EXL3MI_MOE_MFMA", "1")
+    _hold(lib, 0)
+    with pytest.raises(lib.Exl3Error, match="bytes of scratch needed") as e:
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            exl3.moe_forward(x, ids, w, tables, shared=0, out=out)
+    _hold(lib, int(str(e.value).split("workspace: ")[1].split()[0]))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        exl3.moe_forward(x, ids, w, tables, shared=0, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        lib.profile_enable(True)
+        eager = exl3.moe_forward(x, ids, w, tables, shared=0)
+        torch.cuda.synchronize()
+        runs = lib.profile_read()
+        lib.profile_enable(False)
+        assert runs["mlp_down_wide"][0] == 1 and runs["linear_reduce"][0] == 1      # several splits at once
+        assert torch.equal(out, eager)
+    ref = oracle.moe_layer(x.cpu().numpy(), orc, np.zeros((M, 1), np.int32), np.ones((M, 1), np.float32), oracle.ACT_SILU)
+    assert max_rel(eager.cpu().numpy(), ref) <= MAX_REL
+    del graph
+    torch.cuda.synchronize()
