@@ -473,7 +473,7 @@ static size_t gemv_part_bytes(int strips, int P) { return (size_t)strips * P * k
 static int takes_mfma(int64_t m, int64_t k, int64_t n, int S, int K, int forced, LinPlan* pl, bool* yes) {
     *yes = false;
     const bool few = !forced && m < kLinearMfmaMinRows;
-    if (few ? !linear_few_rows(m, n, k) : m < forced) return EXL3_OK;
+    if (few ? !linear_few_rows(m, n, k, K) : m < forced) return EXL3_OK;
     const int strips = (int)(n / 128);
     const size_t most = few ? gemv_part_bytes(strips, gemv_splits(strips, (int)(k / 128), (int)m)) : SIZE_MAX;
     return linear_mfma_plan(m, n, k, S, K, most, pl, yes);

@@ -76,8 +76,12 @@ inline bool linear_call_plan(int64_t m, int64_t n, int64_t k, int S, int K, int 
 // Whether five to eight rows (what the decode GEMV takes in one pass) run on the MFMA GEMM instead. The GEMV's time grows with
 // the rows, the GEMM's three launches cost about 15 us on a small matrix; us, GEMV / GEMM: 5376 -> 21504 at 4 / 6 / 8 rows
 // 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096 9.9 / 16.7,
-// 12.1 / 16.5, 13.0 / 16.6.
-inline bool linear_few_rows(int64_t m, int64_t n, int64_t k) { return m >= 5 && m <= 8 && k * n >= 200000000 / (m - 2); }
+// 12.1 / 16.5, 13.0 / 16.6. That is K = 4. The GEMM's decode grows faster with K than the GEMV's: at K = 6 the line lies higher
+// (4096 -> 12288 of three shards, 6 rows 21.4 / 22.1; 5376 -> 21504, 5 rows 32.0 / 28.6), at K = 7 too, and at K = 8 the
+// GEMV is the faster one up to 8 rows (5376 -> 21504 at 5 / 6 / 8 rows 35.1 / 40.3, 36.5 / 40.4, 40.4 / 40.4).
+inline bool linear_few_rows(int64_t m, int64_t n, int64_t k, int K) {
+    return m >= 5 && m <= 8 && K < 8 && k * n >= (K <= 5 ? 200000000 : 290000000) / (m - 2);
+}
 
 // Row block of the prefill MoE (M tokens, `npairs` rows over E experts, H -> I -> H; uniform K: 1 .. 8). 32 (one class, one
 // launch per projection) up to 64 tokens, 160 where experts take few rows: forking the launches by class costs more there

@@ -22,6 +22,7 @@ extern "C" int64_t call_bytes(int64_t m, int64_t n, int64_t k, int S, int K, int
     LinPlan p;
     return linear_call_plan(m, n, k, S, K, 0, cus, most, &p) ? (int64_t)linear_call_bytes(m, n, k, S, p.P) : -1;
 }
+extern "C" int few_rows(int64_t m, int64_t n, int64_t k, int K) { return linear_few_rows(m, n, k, K); }
 extern "C" int64_t max_blocks(int64_t npairs, int64_t E, int rows, int whole) { return moe_max_blocks(npairs, E, rows, whole); }
 extern "C" int moe_rows(int64_t M, int64_t E, int64_t npairs, int64_t H, int64_t I, int Kg, int Kd, int forced) {
     return moe_wide_rows(M, E, npairs, H, I, Kg, Kd, forced);
@@ -46,6 +47,8 @@ def lib(tmp_path_factory):
     L.moe_rows.restype = i32
     L.call_bytes.argtypes = [i64, i64, i64, i32, i32, i32, ctypes.c_uint64]
     L.call_bytes.restype = i64
+    L.few_rows.argtypes = [i64, i64, i64, i32]
+    L.few_rows.restype = i32
     L.max_blocks.argtypes = [i64, i64, i32, i32]
     L.max_blocks.restype = i64
     return L
@@ -136,3 +139,11 @@ def test_block_list_holds_every_routing(lib, rows, whole):
         for E in (1, 2, 7):
             assert E * blocks_of(c, rows, whole) <= lib.max_blocks(E * c, E, rows, whole)
     assert blocks_of(33, rows, whole) + 5 * blocks_of(1, rows, whole) <= lib.max_blocks(38, 6, rows, whole)
+
+
+def test_few_rows_take_the_gemm_where_it_is_faster(lib):
+    """Both sides of the measured lines: by size, by rows and by bitrate."""
+    for m, K, k, n, want in ((4, 4, 5376, 21504, 0), (5, 4, 5376, 21504, 1), (8, 4, 4096, 4096, 0), (8, 4, 4096, 14336, 1),
+                             (6, 5, 4096, 12288, 1), (6, 6, 4096, 12288, 0), (6, 7, 4096, 12288, 0), (5, 6, 5376, 21504, 1),
+                             (5, 7, 8192, 10240, 0), (5, 8, 5376, 21504, 0), (8, 8, 2048, 131072, 0), (9, 4, 5376, 21504, 0)):
+        assert lib.few_rows(m, n, k, K) == want, (m, K, k, n)
