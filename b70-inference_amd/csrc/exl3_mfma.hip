@@ -879,7 +879,7 @@ static int device_cus(int* cus) {
 int dense_down_splits(int64_t m, int64_t n, int64_t k, int K, int block, int64_t cap, int* P) {
     int cus = 0;
     const int rc = device_cus(&cus);
-    if (!rc) *P = linear_plan(m, n, k, K, block / 32, cap, cus).P;
+    if (!rc) *P = linear_plan(m, n, k, 1, K, block / 32, cap, cus).P;
     return rc;
 }
 
@@ -970,7 +970,9 @@ int linear_mfma_plan(int64_t m, int64_t n, int64_t k, int S, int K, size_t most,
         const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
         pl->bps = (nblk + (int)(want < pmax ? want : pmax) - 1) / (int)(want < pmax ? want : pmax);
         pl->P = (nblk + pl->bps - 1) / pl->bps;
-        while (pl->RG > 1 && !a_span_ok(m < 32 * pl->RG ? m : 32 * pl->RG, 128LL * pl->bps)) pl->RG /= 2;
+        while (pl->RG > 1 && !(a_span_ok(m < 32 * pl->RG ? m : 32 * pl->RG, 128LL * pl->bps) &&
+                               linear_block_built(pl->RG, S, K)))
+            pl->RG /= 2;
         *fits = linear_call_bytes(m, n, k, S, pl->P) <= most;
     }
     return EXL3_OK;
@@ -1017,6 +1019,7 @@ int launch_linear_mfma(const LinPlan& pl, const uint16_t* A, int64_t a_ld, int64
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_gemm: grid too large");
     const dim3 rgrid((unsigned)((m + 3) / 4), (unsigned)(n / 128));
     const lin_fn fn = linear_wide_pick(pl.RG, S, K);
+    if (!fn) return fail(EXL3_ERR_INVALID, "exl3_gemm: no %d-row kernel for %d shards at K=%d", R, S, K);
     if (fixed) {
         hipLaunchKernelGGL(linear_had_kernel, hgrid, dim3(256), 0, st, A, a_ld, (int)m, (int)k, suh, xh, xsum, R, K <= 5);
         hipLaunchKernelGGL(fn, dim3((unsigned)nx), dim3(256), 0, st, a);

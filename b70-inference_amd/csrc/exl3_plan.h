@@ -18,6 +18,9 @@ struct LinPlan {
     int RG, P, bps;                                  // row groups of 32 per block, k-splits, 128-blocks of k per split
 };
 
+// Row blocks of 32 RG rows that the dense linear has a kernel for, with S shards at K bits.
+constexpr bool linear_block_built(int RG, int S, int K) { return RG != 4 || S == 1 || K <= 5; }
+
 // Row block and k-splits P of a dense linear by estimated time: the workgroups spread over the CUs,
 // each CU running up to `occ` at a time. Per 32-k step a CU with j workgroups takes kStepUs[RG][j] microseconds, a
 // workgroup's start and end kEdgeUs[RG]; several splits add the partials (written once, read once by the reduce kernel)
@@ -25,26 +28,32 @@ struct LinPlan {
 // splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
 // blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
 // the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
-// `rg` > 0 asks for that row block (halved until the offsets of a block's A fit), `cap` bounds the splits.
-inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap, int cus) {
+// kBits: the steps at K = 6 and 7 and at K = 8 against K = 4 (medians over 1024 -> 3072 .. 5376 -> 10752, 300 .. 2048 rows; the
+// 32-row block decodes most, the 256-row one least). 128-row blocks of several shards are not built for K > 5: their two
+// A planes and the words spill 28 to 55 registers inside the loop (5376 -> 10752 of three shards, 512 rows, K = 7: 32 / 64 /
+// 128 / 256-row blocks 186 / 133 / 189 / 117 us).
+// `rg` > 0 asks for that row block (halved until there is one and the offsets of its A fit), `cap` bounds the splits.
+inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, int cus) {
     const int nblk = (int)(k / 128);
     const int occ[4] = {K <= 5 ? 4 : 3, K <= 5 ? 3 : 2, 2, 1};       // what the kernels are compiled for (exl3_wide.hip)
     static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
                                         {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
     static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
+    static const float kBits[3][4] = {{1.f, 1.f, 1.f, 1.f}, {1.25f, 1.2f, 1.3f, 1.1f}, {1.6f, 1.5f, 1.6f, 1.15f}};
+    const float* const bits = kBits[K <= 5 ? 0 : K <= 7 ? 1 : 2];
     const int64_t ncb = (n + 255) / 256;
     const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
     LinPlan best = {1, 1, nblk};
     float tb = 1e30f;
     for (int g = 0; g < 4; ++g) {
-        if (rg > 0 && rg != 1 << g) continue;
+        if ((rg > 0 && rg != 1 << g) || !linear_block_built(1 << g, S, K)) continue;
         const int64_t rows = 32 << g, tiles = (m + rows - 1) / rows * ncb;
         for (int p = 1; p <= pmax && p <= cap; ++p) {
             const int bps = (nblk + p - 1) / p, P = (nblk + bps - 1) / bps;
             if (P != p || !a_span_ok(m < rows ? m : rows, 128LL * bps)) continue;
             const int64_t w = (tiles * P + cus - 1) / cus, full = w / occ[g], rem = w % occ[g];
             const float mb = (float)P * (float)m * (float)n * 4e-6f;
-            float t = 4.f * bps * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
+            float t = 4.f * bps * bits[g] * ((float)full * kStepUs[g][occ[g] - 1] + (rem ? kStepUs[g][rem - 1] : 0.f)) +
                       kEdgeUs[g] * (float)(full + (rem ? 1 : 0));
             if (P > 1) t += 3.f + (0.125f + kPartUsPerMB[g]) * mb;
             if (t < tb) {
@@ -53,7 +62,7 @@ inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64
             }
         }
     }
-    return tb == 1e30f && rg > 1 ? linear_plan(m, n, k, K, rg / 2, cap, cus) : best;
+    return tb == 1e30f && rg > 1 ? linear_plan(m, n, k, S, K, rg / 2, cap, cus) : best;
 }
 
 // Scratch of a dense linear on the MFMA GEMM: transformed rows of S shards, their block sums, partials of P > 1 splits.
@@ -69,7 +78,7 @@ inline bool linear_call_plan(int64_t m, int64_t n, int64_t k, int S, int K, int 
     const int64_t ts = (m + rs - 1) / rs * ((n + 255) / 256);
     int64_t cap = ((m <= 32 ? 768 : 512) + ts - 1) / ts;
     while (cap > 1 && linear_call_bytes(m, n, k, S, (int)cap) > most) --cap;
-    *pl = linear_plan(m, n, k, K, rg, cap, cus);
+    *pl = linear_plan(m, n, k, S, K, rg, cap, cus);
     return linear_call_bytes(m, n, k, S, pl->P) <= most;
 }
 

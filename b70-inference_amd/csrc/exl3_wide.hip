@@ -165,17 +165,21 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     }
 }
 
+// (null: no such kernel)
 template <int RG, int NPL>
 static lin_fn pick_wide(int K) {
+    if constexpr (linear_block_built(RG, NPL, 8)) {
+        if (K == 6) return linear_wide_kernel<6, RG, NPL>;
+        if (K == 7) return linear_wide_kernel<7, RG, NPL>;
+        if (K == 8) return linear_wide_kernel<8, RG, NPL>;
+    }
     switch (K) {
         case 1: return linear_wide_kernel<1, RG, NPL>;
         case 2: return linear_wide_kernel<2, RG, NPL>;
         case 3: return linear_wide_kernel<3, RG, NPL>;
         case 4: return linear_wide_kernel<4, RG, NPL>;
         case 5: return linear_wide_kernel<5, RG, NPL>;
-        case 6: return linear_wide_kernel<6, RG, NPL>;
-        case 7: return linear_wide_kernel<7, RG, NPL>;
-        default: return linear_wide_kernel<8, RG, NPL>;
+        default: return nullptr;
     }
 }
 

@@ -12,8 +12,8 @@ CUS = 256
 SHIM = """
 #include "exl3_plan.h"
 using namespace exl3;
-extern "C" void plan(int64_t m, int64_t n, int64_t k, int K, int rg, int64_t cap, int cus, int* out) {
-    const LinPlan p = linear_plan(m, n, k, K, rg, cap, cus);
+extern "C" void plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, int cus, int* out) {
+    const LinPlan p = linear_plan(m, n, k, S, K, rg, cap, cus);
     out[0] = p.RG;
     out[1] = p.P;
     out[2] = p.bps;
@@ -41,7 +41,7 @@ def lib(tmp_path_factory):
                            str(d / "shim.cpp")])
     L = ctypes.CDLL(str(d / "plan.so"))
     i64, i32 = ctypes.c_int64, ctypes.c_int
-    L.plan.argtypes = [i64, i64, i64, i32, i32, i64, i32, ctypes.c_void_p]
+    L.plan.argtypes = [i64, i64, i64, i32, i32, i32, i64, i32, ctypes.c_void_p]
     L.plan.restype = None
     L.moe_rows.argtypes = [i64] * 5 + [i32] * 3
     L.moe_rows.restype = i32
@@ -54,9 +54,9 @@ def lib(tmp_path_factory):
     return L
 
 
-def plan(lib, m, n, k, K, rg=0, cap=1 << 30):
+def plan(lib, m, n, k, K, rg=0, cap=1 << 30, S=1):
     out = (ctypes.c_int * 3)()
-    lib.plan(m, n, k, K, rg, cap, CUS, out)
+    lib.plan(m, n, k, S, K, rg, cap, CUS, out)
     return list(out)
 
 
@@ -147,3 +147,14 @@ def test_few_rows_take_the_gemm_where_it_is_faster(lib):
                              (6, 5, 4096, 12288, 1), (6, 6, 4096, 12288, 0), (6, 7, 4096, 12288, 0), (5, 6, 5376, 21504, 1),
                              (5, 7, 8192, 10240, 0), (5, 8, 5376, 21504, 0), (8, 8, 2048, 131072, 0), (9, 4, 5376, 21504, 0)):
         assert lib.few_rows(m, n, k, K) == want, (m, K, k, n)
+
+
+@pytest.mark.parametrize("K", range(1, 9))
+@pytest.mark.parametrize("rg", [0, 4])
+def test_no_spilling_row_block(lib, K, rg):
+    """128-row blocks of several shards spill registers inside their loop for K > 5: not picked, not even when asked for."""
+    for k, n in ((1024, 3072), (4096, 6144), (5376, 10752), (8192, 2048)):
+        for m in (77, 128, 300, 397, 512, 800, 1024, 1500, 2048):
+            RG = plan(lib, m, n, k, K, rg, 2 * CUS, 3)[0]
+            assert RG != 4 or K <= 5
+            assert rg == 0 or RG == (4 if K <= 5 else 2)
