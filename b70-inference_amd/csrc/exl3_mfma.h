@@ -206,7 +206,7 @@ struct LinArgs {
     int m, k, n, nblk;
     int nrb, ncb, P, bps;                            // row blocks, 256-column blocks, k-splits of this launch, 128-blocks
                                                      // per split
-    int p0;                                          // first split of this launch; > 0: added to part (P = 1)
+    int p0;                                          // first split of this launch
     int f32;
     const int64_t* tab;                              // not null: an expert's addresses (ItemDesc::tab), its down projection
                                                      // in place of tr and svh

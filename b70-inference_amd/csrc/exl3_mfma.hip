@@ -868,6 +868,14 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
 
 lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
 
+// sum += part (n a multiple of 4): the reduce kernel's addition, for splits that run one after another.
+__global__ __launch_bounds__(256) void linear_add_kernel(float* sum, const float* __restrict__ part, int64_t n) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    f4_t* s = reinterpret_cast<f4_t*>(sum + i);
+    *s = *s + *reinterpret_cast<const f4_t*>(part + i);
+}
+
 static int device_cus(int* cus) {
     int dev = 0;
     EXL3_CHECK_HIP(hipGetDevice(&dev));
@@ -903,12 +911,19 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
     l.ncb = (a.H + 255) / 256;
     l.bps = (l.nblk + a.dense_P - 1) / a.dense_P;
     const int P = (l.nblk + l.bps - 1) / l.bps;                    // = dense_P
-    l.P = P > 1 && a.dense_sets == 1 ? 1 : P;                      // splits (and partials) of a launch
+    l.P = a.dense_sets < P ? 1 : P;                                // splits of a launch
     l.part = P > 1 ? a.y : nullptr;
     const int64_t nx = ((int64_t)l.nrb * l.ncb * l.P + 7) / 8 * 8;
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: grid too large");
-    for (; l.p0 < P; l.p0 += l.P)                                  // (a later one adds: not to be run twice)
+    const int64_t set = (int64_t)a.M * a.H;
+    for (; l.p0 < P; l.p0 += l.P) {                                // one launch, or the first split and the later ones added
         EXL3_LAUNCH("mlp_down_wide", linear_wide_pick(a.block_rows / 32, 1, a.Kd), dim3((unsigned)nx), dim3(256), 0, st, l);
+        if (l.p0 > 0)
+            EXL3_LAUNCH("linear_add", linear_add_kernel, dim3((unsigned)((set / 4 + 255) / 256)), dim3(256), 0, st, a.y, l.part,
+                        set);
+        if (l.P < P) l.part = a.y + set;
+    }
+    l.part = a.y;
     if (P > 1)
         EXL3_LAUNCH("linear_reduce", linear_reduce_kernel, dim3((unsigned)((l.m + 3) / 4), (unsigned)(l.n / 128)),
                     dim3(256), 0, st, l);

@@ -140,7 +140,7 @@ struct MoeArgs {
                                        // partials)
     int dense_P;                       // > 0: one expert takes every token with weight 1 (a dense MLP) on the MFMA
                                        // path: k-splits of its down projection, which runs as a dense linear
-    int dense_sets;                    // partials held: dense_P, or 1: the splits run one after another and add up
+    int dense_sets;                    // partials held: dense_P, or 2 (a sum and a split): the splits run one after another
     float* part_gu;
     int* cnt_gu;
     int P_gu, nblk_h;

@@ -1173,13 +1173,13 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
                    carve_size(n_gu * a.P_gu * 2 * MR * 128, 4) + carve_size(n_d * a.P_d * MR * 128, 4);
     };
     if (a.dense_P > 0) {
-        // Under stream capture a workspace without room for all splits' partials holds one set, and the splits run one after
-        // another: the same sums, the scratch of an unsplit call.
+        // Under stream capture a workspace without room for all splits' partials holds two sets, and the splits run one after
+        // another: the same sums, in the scratch of an unsplit call (whose transformed inputs and outputs take two sets).
         a.dense_sets = a.dense_P;
         y_elems = (size_t)a.dense_sets * npairs * a.H;
-        if (scratch() > workspace_room(st)) {
-            a.dense_sets = 1;
-            y_elems = (size_t)npairs * a.H;
+        if (a.dense_P > 2 && scratch() > workspace_room(st)) {
+            a.dense_sets = 2;
+            y_elems = (size_t)2 * npairs * a.H;
         }
     }
     const size_t bytes = scratch();

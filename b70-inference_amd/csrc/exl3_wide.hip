@@ -88,14 +88,8 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
                 const int r = 32 * rg + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
                 const float sx = kMul1C2 * rsum[NPL > 1 ? hw : 0][r];
                 if (r < cnt) {
-                    float v0 = kMul1C1 * acc[rg][0][i] + sx, v1 = kMul1C1 * acc[rg][1][i] + sx;
-                    if (a.p0 > 0) {                  // the sum of the reduce kernel, in its order and with its roundings
-                        asm volatile("" : "+v"(v0), "+v"(v1));       // (no fused multiply-add across it)
-                        v0 += part[(size_t)r * a.n];
-                        v1 += part[(size_t)r * a.n + 32];
-                    }
-                    part[(size_t)r * a.n] = v0;
-                    part[(size_t)r * a.n + 32] = v1;
+                    part[(size_t)r * a.n] = kMul1C1 * acc[rg][0][i] + sx;
+                    part[(size_t)r * a.n + 32] = kMul1C1 * acc[rg][1][i] + sx;
                 }
             }
         return;
