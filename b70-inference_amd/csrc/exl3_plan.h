@@ -28,10 +28,11 @@ constexpr bool linear_block_built(int RG, int S, int K) { return RG != 4 || S ==
 // splits): the point it picks is within 1 % of the best on average, 15 % at worst. Few rows and few columns want small
 // blocks and many splits (4096 x 4096 at 48 rows: 32-row blocks, 8 splits 15.5 us, 64-row 16.4, 128-row 19.4), many rows
 // the wide ones, which decode least (5376 -> 21504 at 2048 rows: 32 / 64 / 128 / 256-row blocks 888 / 616 / 488 / 445 us).
-// kBits: the steps at K = 6 and 7 and at K = 8 against K = 4 (medians over 1024 -> 3072 .. 5376 -> 10752, 300 .. 2048 rows; the
-// 32-row block decodes most, the 256-row one least). 128-row blocks of several shards are not built for K > 5: their two
-// A planes and the words spill 28 to 55 registers inside the loop (5376 -> 10752 of three shards, 512 rows, K = 7: 32 / 64 /
-// 128 / 256-row blocks 186 / 133 / 189 / 117 us).
+// kBits: the steps at K = 6 and 7 and at K = 8 against K = 4, fitted to 3891 points (1024 -> 3072 .. 5376 -> 21504, one and three
+// shards, 12 .. 2048 rows): the point picked is within 0.3 and 0.5 % of the best on average, 9 % at worst; without them 0.7 and
+// 2.6 %, 39 % at worst. 128-row blocks of several shards are not built for K > 5: their two A planes and the words spill
+// 28 to 55 registers inside the loop (5376 -> 10752 of three shards, 512 rows, K = 7: 32 / 64 / 128 / 256-row blocks 186 / 133 /
+// 189 / 117 us).
 // `rg` > 0 asks for that row block (halved until there is one and the offsets of its A fit), `cap` bounds the splits.
 inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, int cus) {
     const int nblk = (int)(k / 128);
@@ -39,7 +40,7 @@ inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg
     static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
                                         {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
     static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};
-    static const float kBits[3][4] = {{1.f, 1.f, 1.f, 1.f}, {1.25f, 1.2f, 1.3f, 1.1f}, {1.6f, 1.5f, 1.6f, 1.15f}};
+    static const float kBits[3][4] = {{1.f, 1.f, 1.f, 1.f}, {1.3f, 1.3f, 1.3f, 1.15f}, {1.6f, 1.45f, 1.45f, 0.95f}};
     const float* const bits = kBits[K <= 5 ? 0 : K <= 7 ? 1 : 2];
     const int64_t ncb = (n + 255) / 256;
     const int pmax = nblk / 2 > 1 ? nblk / 2 : 1;
@@ -86,10 +87,10 @@ inline bool linear_call_plan(int64_t m, int64_t n, int64_t k, int S, int K, int 
 // the rows, the GEMM's three launches cost about 15 us on a small matrix; us, GEMV / GEMM: 5376 -> 21504 at 4 / 6 / 8 rows
 // 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096 9.9 / 16.7,
 // 12.1 / 16.5, 13.0 / 16.6. That is K = 4. The GEMM's decode grows faster with K than the GEMV's: at K = 6 the line lies higher
-// (4096 -> 12288 of three shards, 6 rows 21.4 / 22.1; 5376 -> 21504, 5 rows 32.0 / 28.6), at K = 7 too, and at K = 8 the
+// (6 rows of 4096 -> 12288, three shards, 21.4 / 22.1, of 4096 -> 14336 23.1 / 21.5), at K = 7 too, and at K = 8 the
 // GEMV is the faster one up to 8 rows (5376 -> 21504 at 5 / 6 / 8 rows 35.1 / 40.3, 36.5 / 40.4, 40.4 / 40.4).
 inline bool linear_few_rows(int64_t m, int64_t n, int64_t k, int K) {
-    return m >= 5 && m <= 8 && K < 8 && k * n >= (K <= 5 ? 200000000 : 290000000) / (m - 2);
+    return m >= 5 && m <= 8 && K < 8 && k * n >= (K <= 5 ? 200000000 : 220000000) / (m - 2);
 }
 
 // Row block of the prefill MoE (M tokens, `npairs` rows over E experts, H -> I -> H; uniform K: 1 .. 8). 32 (one class, one
