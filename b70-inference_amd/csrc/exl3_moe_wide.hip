@@ -81,13 +81,24 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
         L.apl = pw;
         L.setup_a(cnt, plane);
     }
+    float* C = reinterpret_cast<float*>(smem);
     f16_t acc[RG][2];
-    zero_acc(acc);
-    L.run(acc);
+    bool stored = false;                                       // the accumulators are in C already
+    if constexpr (RG == 1) {
+        if (cnt <= 16) {
+            f4_t acc16[4] = {};
+            L.run16(cnt, acc16);
+            store_tile16(C, acc16, wave, lane);
+            stored = true;
+        }
+    }
+    if (!stored) {
+        zero_acc(acc);
+        L.run(acc);
+    }
 
     // per row group: the gate and up columns through LDS, eight lanes to a row
     constexpr int LR = 8, N = 32 / LR;
-    float* C = reinterpret_cast<float*>(smem);
     const int rr = threadIdx.x / LR, sub = row_sub<LR>(lane), col = nb * 128 + 4 * sub;
     h2_t sg[N][2], su[N][2], sd[N][2];                         // fp16 pairs: as floats they would spill
     {
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
     for (int rg = 0; rg < RG; ++rg) {
         if (32 * rg >= cnt) break;                             // uniform
         if (rg > 0) __syncthreads();
-        store_tile(C, acc[rg], wave, lane);
+        if (!stored) store_tile(C, acc[rg], wave, lane);
         __syncthreads();
         const int m = 32 * rg + rr;
         if (m >= cnt) continue;
@@ -187,11 +198,22 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_down_wide_ke
         L.apl = 0;
         L.setup_a(cnt, plane);
     }
-    f16_t acc[RG][2];
-    zero_acc(acc);
-    L.run(acc);
-
     float* C = reinterpret_cast<float*>(smem);
+    f16_t acc[RG][2];
+    bool stored = false;                                       // the accumulators are in C already
+    if constexpr (RG == 1) {
+        if (cnt <= 16) {
+            f4_t acc16[4] = {};
+            L.run16(cnt, acc16);
+            store_tile16(C, acc16, wave, lane);
+            stored = true;
+        }
+    }
+    if (!stored) {
+        zero_acc(acc);
+        L.run(acc);
+    }
+
     constexpr int LR = 4, N = 32 / LR;                         // lanes per 128-column half of a row
     const int rr = threadIdx.x / (2 * LR), half = (threadIdx.x / LR) & 1, sub = row_sub<LR>(lane);
     float sd[N][4];
@@ -206,7 +228,7 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_down_wide_ke
     for (int rg = 0; rg < RG; ++rg) {
         if (32 * rg >= cnt) break;                             // uniform
         if (rg > 0) __syncthreads();
-        store_tile(C, acc[rg], wave, lane);
+        if (!stored) store_tile(C, acc[rg], wave, lane);
         const int m = 32 * rg + rr;
         const float w = a.pair_w[p0 + (m < cnt ? m : cnt - 1)];
         __syncthreads();

@@ -71,9 +71,9 @@ struct TileWords {
         wl[wwrap] = D[K - 1];
     }
     // words of the lane's fragment f (tile-row f >> 1 of the step, tile pair f & 1)
-    __device__ __forceinline__ void load_f(uint32_t (&R)[NW], int f) const {
+    __device__ __forceinline__ void load_f(uint32_t (&R)[NW], int f) const { load_slot(R, 4 * (f & 1) + 2 * (f >> 1)); }
+    __device__ __forceinline__ void load_slot(uint32_t (&R)[NW], int slot) const {
         typedef const __attribute__((address_space(3))) uint32_t* lds_t;
-        const int slot = 4 * (f & 1) + 2 * (f >> 1);
         if constexpr (KP) {
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
@@ -114,9 +114,13 @@ struct TileWords {
         const int slot = 2 * g + ((lane & 15) >> 3), q = lane & 7;
         wdst = slot * TS + 4 + q * K;
         wwrap = q == 7 ? slot * TS + 3 : wdst + K - 1;
-        const int n = lane & 15, h = lane >> 5;
+        setup_f(lane >> 5, (lane >> 4) & 1);
+    }
+    // the lane reads k unit h of its column, from slots `slot` past the fragment's
+    __device__ __forceinline__ void setup_f(int h, int slot) {
+        const int n = lane & 15;
         const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)wl +
-                              4u * (uint32_t)(((lane >> 4) & 1) * TS);
+                              4u * (uint32_t)(slot * TS);
         if constexpr (KP) {
             const int t0 = 32 * (n & 7) + 4 * (n >> 3) + 16 * h;
 #pragma unroll
@@ -342,6 +346,62 @@ struct DirectPipe : TileWords<K, PL> {
             aoff[rg] = 16u * (uint32_t)((lane >> 5) * cnt + (row < cnt ? row : cnt - 1));
         }
     }
+
+    // Blocks of up to 16 rows: v_mfma_f32_16x16x32_f16, one tile column and the step's whole k per instruction. The 32-row
+    // form with half its rows empty spends 256 MFMA cycles beside 440 VALU cycles a step, this one 64 (us, 32-row form / this:
+    // 419 rows over 256 experts of 2304 -> 1280, top-4, K = 4 375 / 334; 9 rows of 5376 -> 21504, K = 8 40.6 / 30.2). Lane L: row
+    // or column L & 15, k unit (L >> 4) & 1 of tile-row L >> 5; the instruction adds its k in the order of the two 32x32x16
+    // ones it replaces, so that a row's bits do not depend on the form.
+    template <int R>
+    __device__ __forceinline__ void step16(int s, uint32_t (&W)[WR][K], uint32_t (&F)[4][NW], h8_t (&A)[4],
+                                           f4_t (&acc)[4]) const {
+        typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {                         // tile column f
+            u4_t v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = (i & 1) * 2 + (i >> 1);
+                v[c] = decode_pair(F[f], c);
+            }
+            T::load_slot(F[f], 4 * (f >> 1) + (f & 1));
+            acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[R], __builtin_bit_cast(h8_t, v), acc[f], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        stage_w(W[(R + 2) % WR]);
+        A[R] = load_a16(s + 4);
+        load_w(W[(R + 2) % WR], s + 2 + WR);
+    }
+    __device__ __forceinline__ h8_t load_a16(int s) const {
+        const int so = (s < nsteps ? s : nsteps - 1) * astep;
+        return __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(abuf, aoff[0], so, 0));
+    }
+    __device__ __forceinline__ void run16(int cnt, f4_t (&acc)[4]) {
+        static_assert(RG == 1 && WR == 4);
+        const int h = (lane >> 4) & 1, row = lane & 15;
+        T::setup_f(h, 2 * (lane >> 5));
+        aoff[0] = 16u * (uint32_t)(h * cnt + (row < cnt ? row : cnt - 1)) + (uint32_t)((lane >> 5) * akk);
+        uint32_t W[WR][K], F[4][NW];
+        h8_t A[4];
+#pragma unroll
+        for (int i = 0; i < WR; ++i) load_w(W[i], i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) A[i] = load_a16(i);
+        stage_w(W[0]);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) T::load_slot(F[f], 4 * (f >> 1) + (f & 1));
+        stage_w(W[1]);
+        load_w(W[0], WR);
+        load_w(W[1], WR + 1);
+        for (int s = 0; s < nsteps; s += 4) {
+            step16<0>(s, W, F, A, acc);
+            step16<1>(s + 1, W, F, A, acc);
+            step16<2>(s + 2, W, F, A, acc);
+            step16<3>(s + 3, W, F, A, acc);
+        }
+        drain_loads();
+        __syncthreads();                                       // every slot read done: callers may reuse the LDS
+    }
 };
 
 // ------------------------------------------------------------------------------------------------ epilogue
@@ -426,6 +486,14 @@ __device__ __forceinline__ void store_tile(float* C, const f16_t (&acc)[2], int 
         C[r * kWideCS + cl] = acc[0][i];
         C[r * kWideCS + cl + 32] = acc[1][i];
     }
+}
+// The same of the 16-row form: tile column f, row 4 (lane >> 4) + i, column lane & 15.
+__device__ __forceinline__ void store_tile16(float* C, const f4_t (&acc)[4], int wave, int lane) {
+    const int cl = 64 * wave + (lane & 15) + 16 * (wave >> 1);
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) C[(4 * (lane >> 4) + i) * kWideCS + cl + 16 * f] = acc[f][i];
 }
 
 }  // namespace exl3

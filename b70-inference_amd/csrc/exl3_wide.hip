@@ -20,6 +20,21 @@ __device__ __forceinline__ bool wide_tile(const LinArgs& a, int& rb, int& nb, in
     return true;
 }
 
+// The partials of a block of up to 16 rows (store_tile16's layout), 64 columns from col0.
+__device__ __forceinline__ void partials16(const LinArgs& a, int p, int r0, int cnt, int col0, int lane, const f4_t (&acc)[4],
+                                           const float* rsum) {
+    float* part = a.part + (size_t)p * a.m * a.n + (size_t)r0 * a.n + col0 + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * (lane >> 4) + i;
+        const float sx = kMul1C2 * rsum[r];
+        if (r < cnt) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) part[(size_t)r * a.n + 16 * f] = kMul1C1 * acc[f][i] + sx;
+        }
+    }
+}
+
 template <int K, int RG, int NPL>
 __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 ? 3 : 2) : (K <= 5 ? 4 : 3)) void linear_wide_kernel(LinArgs a) {
     constexpr bool kDirect = RG <= 2;
@@ -70,14 +85,28 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
         L.apl = NPL > 1 ? hw : 0;
         L.setup_a(cnt, plane);
     }
+    float* C = reinterpret_cast<float*>(smem);
     f16_t acc[RG][2];
+    bool stored = false;                             // the accumulators are in C already
+    if constexpr (RG == 1) {
+        if (cnt <= 16) {
+            f4_t acc16[4] = {};
+            L.run16(cnt, acc16);
+            if (a.part) {
+                if (hw < nhalf) partials16(a, p, r0, cnt, nb * 256 + 64 * wave, lane, acc16, rsum[NPL > 1 ? hw : 0]);
+                return;
+            }
+            store_tile16(C, acc16, wave, lane);
+            stored = true;
+        }
+    }
+    if (!stored) {
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg)
+        for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-        for (int np = 0; np < 2; ++np)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[rg][np][i] = 0.f;
-    L.run(acc);
+            for (int np = 0; np < 2; ++np) acc[rg][np] = f16_t{};
+        L.run(acc);
+    }
     if (a.part) {                                    // fp32 partials, affine applied
         if (hw >= nhalf) return;
         float* part = a.part + (size_t)p * a.m * a.n + (size_t)r0 * a.n + nb * 256 + 64 * wave + (lane & 31);
@@ -97,7 +126,6 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
     // Per 32-row group through LDS: the accumulators' layout has a row's columns across lanes (12 single-rate VALU
     // operations per value for the transform); from LDS a quad of lanes takes a row half, five of seven stages in
     // registers.
-    float* C = reinterpret_cast<float*>(smem);
     const int rr = threadIdx.x >> 3, half = (threadIdx.x >> 2) & 1, sub = row_sub<4>(lane);
     const int col = nb * 256 + 128 * half + 4 * sub;
     float sd[8][4];
@@ -113,7 +141,7 @@ __global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
         if (rg > 0) __syncthreads();
-        store_tile(C, acc[rg], wave, lane);
+        if (!stored) store_tile(C, acc[rg], wave, lane);
         __syncthreads();
         const int m = 32 * rg + rr;
         if (m >= cnt || half >= nhalf) continue;

@@ -222,6 +222,27 @@ def test_gemm_mfma_row_blocks(exl3, oracle, monkeypatch, block, k, n, K, M, out_
         assert max_rel(y, ref) <= MAX_REL, jobs
 
 
+@pytest.mark.parametrize("K", range(1, 9))
+@pytest.mark.parametrize("M", [9, 15, 16])
+def test_gemm_sixteen_row_form_bits(exl3, oracle, monkeypatch, K, M):
+    """Blocks of up to 16 rows run on the 16-row matrix instructions: the bits of the same rows in a 32-row block, with the
+    output written from the accumulators and from partials, half column block included, and the oracle's values."""
+    monkeypatch.setenv("EXL3MI_LINEAR_BLOCK", "1")
+    S_ = synth()
+    k, n = 1024, 384
+    tr, suh, svh = S_.linear(k, n, K, 7700 + K)
+    x = S_.activations(33, k, 7710 + K)
+    lin = exl3.BC_LinearEXL3(tr.cuda(), suh.cuda(), svh.cuda(), K, None, False, True, None)
+    ref = oracle.exl3_linear(x[:M].numpy(), tr.numpy(), suh.numpy(), svh.numpy(), K, np.float32)
+    for jobs in (("1", "1"), ("8", "16")):                     # one split; four, of one row block and of two
+        y = []
+        for rows, j in zip((M, 33), jobs):
+            monkeypatch.setenv("EXL3MI_LINEAR_JOBS", j)
+            y.append(lin.run_alloc(x[:rows].cuda(), n, True)[:M])
+        assert torch.equal(y[0], y[1]), jobs
+        assert max_rel(y[0].cpu().numpy(), ref) <= MAX_REL
+
+
 @pytest.mark.parametrize("k,n,K,M", [(8192, 8192, 2, 5), (4096, 14336, 3, 6), (2048, 21504, 7, 7), (5376, 6400, 4, 8)])
 def test_gemm_few_rows_of_large_matrices(exl3, oracle, M, k, n, K):
     """Five to eight rows on both sides of the size from which they take the MFMA GEMM: the first and last 128 columns
