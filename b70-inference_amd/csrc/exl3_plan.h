@@ -84,13 +84,15 @@ inline bool linear_call_plan(int64_t m, int64_t n, int64_t k, int S, int K, int 
 }
 
 // Whether five to eight rows (what the decode GEMV takes in one pass) run on the MFMA GEMM instead. The GEMV's time grows with
-// the rows, the GEMM's three launches cost about 15 us on a small matrix; us, GEMV / GEMM: 5376 -> 21504 at 4 / 6 / 8 rows
-// 24.9 / 24.8, 32.1 / 25.4, 37.3 / 25.6; 4096 -> 14336 16.7 / 17.7, 21.4 / 18.1, 25.8 / 18.6; 4096 x 4096 9.9 / 16.7,
-// 12.1 / 16.5, 13.0 / 16.6. That is K = 4. The GEMM's decode grows faster with K than the GEMV's: at K = 6 the line lies higher
-// (6 rows of 4096 -> 12288, three shards, 21.4 / 22.1, of 4096 -> 14336 23.1 / 21.5), at K = 7 too, and at K = 8 the
-// GEMV is the faster one up to 8 rows (5376 -> 21504 at 5 / 6 / 8 rows 35.1 / 40.3, 36.5 / 40.4, 40.4 / 40.4).
+// the rows, the GEMM's three launches cost about 15 us on a small matrix, and its decode grows faster with K than the GEMV's. us,
+// GEMV / GEMM, at K = 4: 5376 -> 21504 at 5 / 6 / 8 rows 29.9 / 23.6, 32.1 / 23.7, 37.3 / 24.0; 4096 -> 14336 at 6 / 8 rows
+// 21.8 / 17.6, 25.9 / 18.0; 8192 x 8192 at 5 rows 19.2 / 18.1; 4096 -> 8192 at 8 rows 16.4 / 17.5. At K = 6 / 7 / 8 the line lies
+// higher: 8192 x 8192 at 5 rows 19.6 / 21.9, 20.0 / 22.3, 20.6 / 23.2, at 7 rows 22.3 / 21.8, 22.3 / 22.2, 22.9 / 23.3;
+// 4096 -> 14336 at 8 rows 26.5 / 20.5, 26.8 / 21.4, 26.8 / 21.9.
 inline bool linear_few_rows(int64_t m, int64_t n, int64_t k, int K) {
-    return m >= 5 && m <= 8 && K < 8 && k * n >= (K <= 5 ? 200000000 : 220000000) / (m - 2);
+    if (m < 5 || m > 8) return false;
+    const int64_t least = (K <= 5 ? 200000000 : K == 6 ? 220000000 : K == 7 ? 290000000 : 340000000) / (m - 2);
+    return k * n >= (least > 40000000 ? least : 40000000);
 }
 
 // Row block of the prefill MoE (M tokens, `npairs` rows over E experts, H -> I -> H; uniform K: 1 .. 8). 32 (one class, one

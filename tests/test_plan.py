@@ -143,9 +143,10 @@ def test_block_list_holds_every_routing(lib, rows, whole):
 
 def test_few_rows_take_the_gemm_where_it_is_faster(lib):
     """Both sides of the measured lines: by size, by rows and by bitrate."""
-    for m, K, k, n, want in ((4, 4, 5376, 21504, 0), (5, 4, 5376, 21504, 1), (8, 4, 4096, 4096, 0), (8, 4, 4096, 14336, 1),
-                             (6, 5, 4096, 12288, 1), (6, 6, 4096, 12288, 0), (6, 7, 4096, 12288, 0), (5, 6, 5376, 21504, 1),
-                             (6, 6, 4096, 14336, 1), (5, 7, 8192, 8192, 0), (5, 8, 5376, 21504, 0), (8, 8, 2048, 131072, 0), (9, 4, 5376, 21504, 0)):
+    for m, K, k, n, want in ((4, 4, 5376, 21504, 0), (5, 4, 8192, 8192, 1), (5, 4, 4096, 14336, 0), (8, 4, 4096, 8192, 0),
+                             (8, 4, 4096, 11008, 1), (6, 5, 4096, 12288, 1), (6, 6, 4096, 12288, 0), (6, 6, 4096, 14336, 1),
+                             (6, 7, 8192, 8192, 0), (7, 7, 8192, 8192, 1), (7, 8, 8192, 8192, 0), (8, 8, 4096, 14336, 1),
+                             (5, 8, 5376, 21504, 1), (9, 4, 5376, 21504, 0)):
         assert lib.few_rows(m, n, k, K) == want, (m, K, k, n)
 
 
