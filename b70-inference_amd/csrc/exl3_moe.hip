@@ -1660,10 +1660,7 @@ int exl3_router_logits(const uint16_t* x, int64_t x_ld, int64_t M, int64_t H, co
     if (w_layout == EXL3_ROUTER_W_HE) {
         EXL3_CHECK_ARG(E % 8 == 0 && w_ld >= E && aligned(x, 4) && x_ld % 2 == 0,
                        "exl3_router_logits: [H, E] weights need E a multiple of 8, w_ld >= E and a 4-byte aligned x");
-        // rows per workgroup: as many as leave 256 workgroups, else one (a workgroup's FMAs are one CU's work: 2048 x 512
-        // at 8 rows 10.9 us with four rows per workgroup, 16 workgroups)
-        const int64_t strips = (E + 63) / 64;
-        const int mr = strips * ((M + 3) / 4) >= 256 ? 4 : strips * ((M + 1) / 2) >= 256 ? 2 : 1;
+        const int mr = router_rows(M, E, 256);
         rfn fn = mr == 4 ? router_cols_kernel<4> : mr == 2 ? router_cols_kernel<2> : router_cols_kernel<1>;
         const unsigned gy = (unsigned)((M + mr - 1) / mr);
         EXL3_LAUNCH("router_logits", fn, dim3((unsigned)((E + 63) / 64), gy), dim3(1024), 0, st, x, x_ld, (int)M,

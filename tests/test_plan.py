@@ -23,6 +23,7 @@ extern "C" int64_t call_bytes(int64_t m, int64_t n, int64_t k, int S, int K, int
     return linear_call_plan(m, n, k, S, K, 0, cus, most, &p) ? (int64_t)linear_call_bytes(m, n, k, S, p.P) : -1;
 }
 extern "C" int few_rows(int64_t m, int64_t n, int64_t k, int K) { return linear_few_rows(m, n, k, K); }
+extern "C" int router(int64_t M, int64_t E) { return router_rows(M, E, 256); }
 extern "C" int64_t max_blocks(int64_t npairs, int64_t E, int rows, int whole) { return moe_max_blocks(npairs, E, rows, whole); }
 extern "C" int moe_rows(int64_t M, int64_t E, int64_t npairs, int64_t H, int64_t I, int Kg, int Kd, int forced) {
     return moe_wide_rows(M, E, npairs, H, I, Kg, Kd, forced);
@@ -49,6 +50,8 @@ def lib(tmp_path_factory):
     L.call_bytes.restype = i64
     L.few_rows.argtypes = [i64, i64, i64, i32]
     L.few_rows.restype = i32
+    L.router.argtypes = [i64, i64]
+    L.router.restype = i32
     L.max_blocks.argtypes = [i64, i64, i32, i32]
     L.max_blocks.restype = i64
     return L
@@ -167,3 +170,11 @@ def test_dense_mlp_capture_shapes_have_many_splits(lib, M, H, I):
     than the two sets of partials that the workspace holds."""
     rows = lib.moe_rows(M, 1, M, H, I, 3, 3, 0)
     assert plan(lib, M, H, I, 3, rows // 32, 8)[1] > 2
+
+
+def test_router_rows_by_rounds(lib):
+    """Rows per workgroup of the router GEMV: few while every CU has at most one workgroup, more before a second round."""
+    for M, E, want in ((1, 512, 1), (8, 512, 1), (32, 512, 1), (48, 512, 2), (64, 512, 2), (96, 512, 4), (200, 160, 4),
+                       (256, 160, 4), (128, 256, 2), (200, 256, 4), (512, 8, 2), (512, 160, 2), (4 * 65535, 8, 4)):
+        assert lib.router(M, E) == want, (M, E)
+        assert -(-M // lib.router(M, E)) <= 65535              # the grid's second dimension
