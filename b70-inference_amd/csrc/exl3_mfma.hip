@@ -915,9 +915,11 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
     l.part = P > 1 ? a.y : nullptr;
     const int64_t nx = ((int64_t)l.nrb * l.ncb * l.P + 7) / 8 * 8;
     if (nx > 0x7FFFFFFF) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: grid too large");
+    const lin_fn fn = linear_wide_pick(a.block_rows / 32, 1, a.Kd);
+    if (!fn) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: no kernel for blocks of %d rows at K=%d", a.block_rows, a.Kd);
     const int64_t set = (int64_t)a.M * a.H;
     for (; l.p0 < P; l.p0 += l.P) {                                // one launch, or the first split and the later ones added
-        EXL3_LAUNCH("mlp_down_wide", linear_wide_pick(a.block_rows / 32, 1, a.Kd), dim3((unsigned)nx), dim3(256), 0, st, l);
+        EXL3_LAUNCH("mlp_down_wide", fn, dim3((unsigned)nx), dim3(256), 0, st, l);
         if (l.p0 > 0)
             EXL3_LAUNCH("linear_add", linear_add_kernel, dim3((unsigned)((set / 4 + 255) / 256)), dim3(256), 0, st, a.y, l.part,
                         set);

@@ -17,11 +17,6 @@ namespace exl3 {
 
 // RG: row groups of 32 in a block. Every class accumulates and reduces in the same order, so a row's result does not depend
 // on the class its block falls into.
-// Waves per SIMD the kernels are compiled for (no spills in the loop).
-template <int K, int RG>
-constexpr int moe_wide_occ() {
-    return RG == 4 ? 2 : RG == 2 ? (K <= 5 ? 3 : 2) : (K <= 5 ? 4 : 3);
-}
 
 template <int K, int RG, int NPL, bool PL>
 struct MoePipe {
@@ -52,7 +47,7 @@ __device__ __forceinline__ void zero_acc(f16_t (&acc)[G][2]) {
 }
 
 template <int K, int RG, bool PL>
-__global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_kernel(MoeArgs a, int cl) {
+__global__ __launch_bounds__(256, wide_occ(RG, K)) void moe_gateup_wide_kernel(MoeArgs a, int cl) {
     typedef MoePipe<K, RG, 2, PL> MP;
     __shared__ __attribute__((aligned(16))) char smem[MP::kSmem];
     __shared__ float rsum[2][32 * RG];
@@ -170,7 +165,7 @@ __global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_gateup_wide_
 }
 
 template <int K, int RG, bool PL>
-__global__ __launch_bounds__(256, (moe_wide_occ<K, RG>())) void moe_down_wide_kernel(MoeArgs a, int cl) {
+__global__ __launch_bounds__(256, wide_occ(RG, K)) void moe_down_wide_kernel(MoeArgs a, int cl) {
     typedef MoePipe<K, RG, 1, PL> MP;
     __shared__ __attribute__((aligned(16))) char smem[MP::kSmem];
     __shared__ float rsum[32 * RG];
@@ -289,7 +284,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(MoeArgs a) {
 
 typedef void (*moe_wide_fn)(MoeArgs, int);
 
-// PLANAR4 instantiations where that order differs from tile order (K = 3, 5, 6, 7); 128-row blocks for K <= 5 only
+// PLANAR4 instantiations where that order differs from tile order (K = 3, 5, 6, 7); 128-row blocks for K <= 5 only (null: no
+// such kernel)
 #define EXL3_WIDE_PICK(KERNEL)                              \
     if (pl) {                                               \
         if (K == 3) return KERNEL<3, RG, true>;             \
@@ -309,7 +305,8 @@ typedef void (*moe_wide_fn)(MoeArgs, int);
         case 2: return KERNEL<2, RG, false>;                \
         case 3: return KERNEL<3, RG, false>;                \
         case 4: return KERNEL<4, RG, false>;                \
-        default: return KERNEL<5, RG, false>;               \
+        case 5: return KERNEL<5, RG, false>;                \
+        default: return nullptr;                            \
     }
 
 template <int RG>
@@ -321,35 +318,33 @@ static moe_wide_fn pick_down(int K, bool pl) {
     EXL3_WIDE_PICK(moe_down_wide_kernel)
 }
 
+static int launch_wide(const char* name, moe_wide_fn fn, const MoeArgs& a, int cl, int nblocks, int ncb, hipStream_t st) {
+    if (!fn) return fail(EXL3_ERR_INVALID, "exl3_moe_forward: no kernel for blocks of %d rows at K=%d, %d", a.block_rows, a.Kg, a.Kd);
+    EXL3_LAUNCH(name, fn, dim3((unsigned)((nblocks + 7) / 8 * 8 * ncb)), dim3(256), 0, st, a, cl);
+    return EXL3_OK;
+}
+
 // gate|up or down of one row class: 0: blocks of up to 32 rows, 1: up to a.block_rows
 int launch_gateup_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st) {
-    const dim3 grid((unsigned)((nblocks + 7) / 8 * 8 * (a.I / 128)));
     moe_wide_fn fn = cl == 0 ? pick_gateup<1>(a.Kg, a.planar)
                    : a.block_rows > 64 ? pick_gateup<4>(a.Kg, a.planar) : pick_gateup<2>(a.Kg, a.planar);
-    EXL3_LAUNCH(cl == 0 ? "moe_gateup_wide_32" : "moe_gateup_wide_big", fn, grid, dim3(256), 0, st, a, cl);
-    return EXL3_OK;
+    return launch_wide(cl == 0 ? "moe_gateup_wide_32" : "moe_gateup_wide_big", fn, a, cl, nblocks, a.I / 128, st);
 }
 
 int launch_down_wide(const MoeArgs& a, int cl, int nblocks, hipStream_t st) {
-    const dim3 grid((unsigned)((nblocks + 7) / 8 * 8 * ((a.H / 128 + 1) / 2)));
     moe_wide_fn fn = cl == 0 ? pick_down<1>(a.Kd, a.planar)
                    : a.block_rows > 64 ? pick_down<4>(a.Kd, a.planar) : pick_down<2>(a.Kd, a.planar);
-    EXL3_LAUNCH(cl == 0 ? "moe_down_wide_32" : "moe_down_wide_big", fn, grid, dim3(256), 0, st, a, cl);
-    return EXL3_OK;
+    return launch_wide(cl == 0 ? "moe_down_wide_32" : "moe_down_wide_big", fn, a, cl, nblocks, (a.H / 128 + 1) / 2, st);
 }
 
 int launch_gateup_class(const MoeArgs& a, int cl, hipStream_t st) {
-    const dim3 grid((unsigned)((a.max_blocks + 7) / 8 * 8 * (a.I / 128)));
-    EXL3_LAUNCH("moe_gateup_wide", (cl == 2 ? pick_gateup<2>(a.Kg, a.planar) : pick_gateup<1>(a.Kg, a.planar)), grid,
-                dim3(256), 0, st, a, cl);
-    return EXL3_OK;
+    return launch_wide("moe_gateup_wide", cl == 2 ? pick_gateup<2>(a.Kg, a.planar) : pick_gateup<1>(a.Kg, a.planar), a, cl,
+                       a.max_blocks, a.I / 128, st);
 }
 
 int launch_down_class(const MoeArgs& a, int cl, hipStream_t st) {
-    const dim3 grid((unsigned)((a.max_blocks + 7) / 8 * 8 * ((a.H / 128 + 1) / 2)));
-    EXL3_LAUNCH("moe_down_wide", (cl == 2 ? pick_down<2>(a.Kd, a.planar) : pick_down<1>(a.Kd, a.planar)), grid,
-                dim3(256), 0, st, a, cl);
-    return EXL3_OK;
+    return launch_wide("moe_down_wide", cl == 2 ? pick_down<2>(a.Kd, a.planar) : pick_down<1>(a.Kd, a.planar), a, cl,
+                       a.max_blocks, (a.H / 128 + 1) / 2, st);
 }
 
 int launch_moe_combine(const MoeArgs& a, hipStream_t st) {

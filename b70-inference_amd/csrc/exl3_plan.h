@@ -14,6 +14,9 @@ inline size_t carve_size(size_t n, size_t elem) { return (n * elem + 255) & ~(si
 // buffer resource of 2^31 - 1 bytes: loads past it return zero. Blocks are cut so that they stay inside.
 constexpr bool a_span_ok(int64_t rows, int64_t k) { return 2 * rows * k <= 0x7FFFFFFF; }
 
+// Waves per SIMD (workgroups of four waves per CU) that the kernels of blocks of 32 RG rows are compiled for.
+constexpr int wide_occ(int RG, int K) { return RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 ? 3 : 2) : (K <= 5 ? 4 : 3); }
+
 struct LinPlan {
     int RG, P, bps;                                  // row groups of 32 per block, k-splits, 128-blocks of k per split
 };
@@ -36,7 +39,7 @@ constexpr bool linear_block_built(int RG, int S, int K) { return RG != 4 || S ==
 // `rg` > 0 asks for that row block (halved until there is one and the offsets of its A fit), `cap` bounds the splits.
 inline LinPlan linear_plan(int64_t m, int64_t n, int64_t k, int S, int K, int rg, int64_t cap, int cus) {
     const int nblk = (int)(k / 128);
-    const int occ[4] = {K <= 5 ? 4 : 3, K <= 5 ? 3 : 2, 2, 1};       // what the kernels are compiled for (exl3_wide.hip)
+    const int occ[4] = {wide_occ(1, K), wide_occ(2, K), wide_occ(4, K), wide_occ(8, K)};
     static const float kStepUs[4][4] = {{0.29f, 0.52f, 0.77f, 0.84f}, {0.36f, 0.63f, 0.84f, 0.84f},
                                         {0.48f, 0.82f, 0.82f, 0.82f}, {0.75f, 0.75f, 0.75f, 0.75f}};
     static const float kEdgeUs[4] = {4.8f, 7.1f, 8.8f, 11.3f}, kPartUsPerMB[4] = {0.146f, 0.044f, 0.071f, 0.305f};

@@ -36,7 +36,7 @@ __device__ __forceinline__ void partials16(const LinArgs& a, int p, int r0, int 
 }
 
 template <int K, int RG, int NPL>
-__global__ __launch_bounds__(256, RG == 8 ? 1 : RG == 4 ? 2 : RG == 2 ? (K <= 5 ? 3 : 2) : (K <= 5 ? 4 : 3)) void linear_wide_kernel(LinArgs a) {
+__global__ __launch_bounds__(256, wide_occ(RG, K)) void linear_wide_kernel(LinArgs a) {
     constexpr bool kDirect = RG <= 2;
     typedef std::conditional_t<kDirect, DirectPipe<K, RG>, WidePipe<K, kDirect ? 4 : RG, NPL>> Pipe;
     constexpr int kStage = kDirect ? 0 : WidePipe<K, kDirect ? 4 : RG, NPL>::kStageBytes;
