@@ -243,25 +243,40 @@ def test_gemm_sixteen_row_form_bits(exl3, oracle, monkeypatch, K, M):
         assert max_rel(y[0].cpu().numpy(), ref) <= MAX_REL
 
 
-@pytest.mark.parametrize("k,n,K,M", [(8192, 8192, 2, 5), (4096, 14336, 3, 6), (2048, 21504, 7, 7), (5376, 6400, 4, 8)])
-def test_gemm_few_rows_of_large_matrices(exl3, oracle, M, k, n, K):
-    """Five to eight rows on both sides of the size from which they take the MFMA GEMM: the first and last 128 columns
-    against the oracle, and the allocation-free entry point bit for bit."""
-    from importlib import import_module
-    L_ = import_module("b70-inference_amd._lib")
+# the last 128 columns below the size from which so many rows take the MFMA GEMM, and the first at or above it
+@pytest.mark.parametrize("M,K,k,n_below", [(5, 2, 8192, 8064), (6, 3, 4096, 12160), (7, 5, 4096, 9728), (8, 4, 4096, 9728),
+                                           (6, 6, 4096, 13312), (7, 7, 4096, 14080), (8, 8, 4096, 13824)])
+@pytest.mark.parametrize("above", [False, True])
+@pytest.mark.parametrize("S", [1, 3])
+def test_gemm_few_rows_of_large_matrices(exl3, oracle, M, K, k, n_below, above, S):
+    """Five to eight rows on both sides of the size from which they take the MFMA GEMM: the kernel that ran, the first and
+    last 128 columns against the oracle and, unsharded, the allocation-free entry point bit for bit."""
+    L_ = exl3._lib
     S_ = synth()
-    tr, suh, svh = S_.linear(k, n, K, 7600 + M)
+    n = n_below + 128 * above
+    widths = [n] if S == 1 else [n - 512, 128, 384]
+    shards = [S_.linear(k, w, K, 7600 + 10 * M + i) for i, w in enumerate(widths)]
     x = S_.activations(M, k, 7610 + M)
-    xc, trc, suc, svc = x.cuda(), tr.cuda(), suh.cuda(), svh.cuda()
-    y = exl3.BC_LinearEXL3(trc, suc, svc, K, None, False, True, None).run_alloc(xc, n, True)
-    z = torch.full_like(y, float("nan"))
-    L_.check(L_.lib().exl3_gemm_noalloc(L_.ptr(xc), k, M, k, L_.ptr(trc), n, K, L_.ptr(z), n, 1, L_.ptr(suc),
-                                        L_.ptr(svc), 2, L_.stream_of(xc)), "exl3_gemm_noalloc")
-    assert torch.equal(y, z)
-    for t in (0, n // 16 - 8):                              # 128-column blocks do not depend on each other
-        ref = oracle.exl3_linear(x.numpy(), tr[:, t:t + 8].contiguous().numpy(), suh.numpy(),
-                                 svh[16 * t:16 * t + 128].numpy(), K, np.float32)
-        assert max_rel(y[:, 16 * t:16 * t + 128].cpu().numpy(), ref) <= MAX_REL
+    xc = x.cuda()
+    lins = [exl3.BC_LinearEXL3(tr.cuda(), su.cuda(), sv.cuda(), K, None, False, True, None) for tr, su, sv in shards]
+    fused = exl3.fuse_linears(lins) if S > 1 else None
+    y = torch.empty(M, n, device="cuda")
+    L_.profile_enable(True)
+    if S == 1:
+        lins[0].run(xc, y)
+    else:
+        exl3.linear(xc, *fused, out=y)
+    runs = set(L_.profile_read())
+    L_.profile_enable(False)
+    assert runs == {"gemv"} if not above else "linear_wide" in runs and "gemv" not in runs, runs
+    if S == 1:
+        z = torch.full_like(y, float("nan"))
+        exl3.exl3_gemm_noalloc(xc, lins[0].trellis, z, lins[0].suh, lins[0].svh)
+        assert torch.equal(y, z)
+    for (tr, su, sv), t, at in ((shards[0], 0, 0), (shards[-1], widths[-1] // 16 - 8, n - 128)):
+        ref = oracle.exl3_linear(x.numpy(), tr[:, t:t + 8].contiguous().numpy(), su.numpy(),
+                                 sv[16 * t:16 * t + 128].numpy(), K, np.float32)   # 128-column blocks do not depend on each other
+        assert max_rel(y[:, at:at + 128].cpu().numpy(), ref) <= MAX_REL
 
 
 @pytest.mark.parametrize("block", [1, 4, 8])

@@ -178,3 +178,11 @@ def test_router_rows_by_rounds(lib):
                        (256, 160, 4), (128, 256, 2), (200, 256, 4), (512, 8, 2), (512, 160, 2), (4 * 65535, 8, 4)):
         assert lib.router(M, E) == want, (M, E)
         assert -(-M // lib.router(M, E)) <= 65535              # the grid's second dimension
+
+
+def test_row_block_by_load(lib):
+    """Row blocks of the prefill MoE by batch and load, at the sizes of the blob tests among others."""
+    for M, E, slots, K, want in ((160, 6, 2, 3, 64), (480, 12, 2, 3, 128), (700, 6, 2, 5, 128), (700, 6, 2, 6, 64),
+                                 (64, 16, 8, 3, 32), (160, 256, 8, 3, 32), (160, 64, 8, 3, 128), (512, 160, 8, 2, 128),
+                                 (1024, 512, 10, 3, 128), (40, 1, 1, 4, 64), (397, 1, 1, 4, 128), (397, 1, 1, 8, 64)):
+        assert lib.moe_rows(M, E, M * slots, 2048, 1024, K, K, 0) == want, (M, E, slots, K)
