@@ -379,8 +379,8 @@ def test_moe_c3_full_size(exl3, oracle):
 def test_align_tables(exl3, oracle, M, k, E):
     """Up to 256 pairs take the one-thread-per-pair kernel, more the 1024-thread one: with the pairs held in
     registers and the three sorted arrays built in LDS (300 x 4), held and the sorted order packed into one LDS word per
-    pair (1500 x 4 and 2600 x 4: the arrays would not fit 64 KB), and reloaded per phase (3300 x 4 = 13200 pairs, more than 12
-    per thread; 1024 x 8 over 2048 experts, whose tables leave no room for the order)."""
+    pair (1500 x 4 and 2600 x 4: the arrays would not fit 64 KB), held and written directly (1024 x 8 over 2048 experts,
+    whose tables leave no room for the order), and reloaded per phase (3300 x 4 = 13200 pairs, more than 12 per thread)."""
     ids, w = _ids_w(M, k, E, 1000 + M, dup=True, inactive=True)
     counts, ptok, pw, pof = exl3.moe_align(ids.cuda(), w.cuda(), E, shared=-1)
     counts, ptok, pw, pof = (t.cpu().numpy() for t in (counts, ptok, pw, pof))
