@@ -423,12 +423,11 @@ __device__ __forceinline__ h4_t decode4p_rt(const uint32_t* slot, int K, uint32_
 // whose tiles are all K <= 2 stages compactly (slot stride kMixTSF, the first load only) and decodes with per-lane funnel origins
 // and shifts precomputed for K = 1 and 2 (one select each per tile); other steps stage at stride kMixTS and decode
 // with the tile's K at run time. Rings of 4 (first tile words DW - 1 = 2 steps ahead, (K, woff) DW = 3 steps ahead) make
-// the loop a 4-step unroll; the step count (H / 32 or I / 32, H and I multiples of 128) is a multiple of 4. A is staged
-// as in MfmaPipe (four LDS stages written two steps ahead, a barrier every second step), but from a register ring of
-// two: loaded three steps ahead, stored one step later (the 1-row-group kernels fit five waves per SIMD that way); with
+// the loop a 4-step unroll; the step count (H / 32 or I / 32, H and I multiples of 128) is a multiple of 4. A goes
+// through four LDS stages written two steps ahead, a barrier every second step, from a register ring of two: loaded
+// three steps ahead, stored one step later (the 1-row-group kernels fit five waves per SIMD that way); with
 // one row group each wave stages its own plane in a private ring and the loop has no barrier.
 constexpr int kMixTSF = 20;                                 // compact slot: 3 pad, w(8K - 1), 16 words (K <= 2)
-
 
 template <int NPS, int RGA>
 struct MfmaPipeMix {
@@ -450,8 +449,8 @@ struct MfmaPipeMix {
     uint32_t fa1, fa2;                                       // fast path: LDS byte address of the lane's funnel
     uint32_t sh1, sh2;                                       // word in compact slot 0 at K = 1 and 2, and the
                                                              // funnel shifts
-    __amdgpu_buffer_rsrc_t abuf[CPT];                        // as in MfmaPipe
-    uint32_t aoff[CPT];
+    __amdgpu_buffer_rsrc_t abuf[CPT];                        // this thread's units of a stage: their plane's rows, offsets
+    uint32_t aoff[CPT];                                      // there at step 0, and units in the stage
     int adst[CPT];
     u32x4_t* lds;
     int lane;
@@ -863,8 +862,6 @@ __global__ __launch_bounds__(256) void linear_reduce_kernel(LinArgs a) {
     fwht128_wave(v0, v1, lane);
     linear_store(a, a.rowmap ? a.rowmap[row] : row, col, v0 * s0, v1 * s1);
 }
-
-
 
 lin_fn linear_wide_pick(int RG, int S, int K);           // exl3_wide.hip
 

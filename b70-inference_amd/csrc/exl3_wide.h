@@ -272,8 +272,8 @@ struct WidePipe : TileWords<K, PL> {
 };
 
 // Up to 64 rows (RG = 1, 2): several waves per SIMD, each on its own. A fragments come straight from memory (the block's
-// A is read by all workgroups of its row block, so from the L2, and by the workgroup's waves, so from the L1) three
-// steps ahead: no LDS traffic for A and no barrier in the loop; a fragment's MFMAs run while the next one is decoded.
+// A is read by all workgroups of its row block, so from the L2, and by the workgroup's waves, so from the L1) four
+// steps ahead (two with 64 rows): no LDS traffic for A and no barrier in the loop; a fragment's MFMAs run while the next one is decoded.
 template <int K, int RG, bool PL = false>
 struct DirectPipe : TileWords<K, PL> {
     typedef TileWords<K, PL> T;
@@ -405,23 +405,20 @@ struct DirectPipe : TileWords<K, PL> {
 };
 
 // ------------------------------------------------------------------------------------------------ epilogue
-// A row of 128 columns spread over L = 4, 8 or 16 adjacent lanes: lane index sub (row_sub) holds columns
+// A row of 128 columns spread over L = 4 or 8 adjacent lanes: lane index sub (row_sub) holds columns
 // 4 L i + 4 sub + j of v[i][j]. The transform's stages of column bits 0, 1 and of the bits of i are register additions,
 // those of sub exchange with the lane whose sub differs in one bit; column bits in ascending order whatever L is (the
 // same bits in every row class). sub is not the plain lane number: its bits are chosen
-// so that those lanes are at xor distances 1, 2, 7 and 15, each a single DPP move (quad permutes, half-row and row mirror).
+// so that those lanes are at xor distances 1, 2 and 7, each a single DPP move (quad permutes, half-row mirror).
 template <int L>
 __device__ __forceinline__ int row_sub(int lane) {
-    if (L == 4) return lane & 3;
-    const int l2 = (lane >> 2) & 1;
-    if (L == 8) return (lane & 7) ^ 3 * l2;
-    const int l3 = (lane >> 3) & 1;
-    return ((lane & 3) ^ 3 * l2) | (l2 ^ l3) << 2 | l3 << 3;
+    static_assert(L == 4 || L == 8);
+    return L == 4 ? lane & 3 : (lane & 7) ^ 3 * ((lane >> 2) & 1);
 }
 template <int B>                                             // value of the lane whose sub differs in bit B
 __device__ __forceinline__ float sub_xor(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
-                                                                 B == 0 ? 0xB1 : B == 1 ? 0x4E : B == 2 ? 0x141 : 0x140,
+                                                                 B == 0 ? 0xB1 : B == 1 ? 0x4E : 0x141,
                                                                  0xF, 0xF, false));
 }
 // Sum of a row's 128 values, pairwise by ascending column bit (the same bits whatever L is).
@@ -434,7 +431,6 @@ __device__ __forceinline__ float row_sum128(const f4_t (&v)[32 / L]) {
         t[i] += sub_xor<0>(t[i]);
         t[i] += sub_xor<1>(t[i]);
         if constexpr (L >= 8) t[i] += sub_xor<2>(t[i]);
-        if constexpr (L >= 16) t[i] += sub_xor<3>(t[i]);
     }
 #pragma unroll
     for (int n = 16 / L; n > 0; n /= 2)
@@ -450,7 +446,7 @@ __device__ __forceinline__ void fwht128_lanes(f4_t (&v)[32 / L], int sub) {
         const float a = v[i][0] + v[i][1], b = v[i][0] - v[i][1], c = v[i][2] + v[i][3], d = v[i][2] - v[i][3];
         v[i] = f4_t{a + c, b + d, a - c, b - d};
     }
-    const float s0 = sub & 1 ? -1.f : 1.f, s1 = sub & 2 ? -1.f : 1.f, s2 = sub & 4 ? -1.f : 1.f, s3 = sub & 8 ? -1.f : 1.f;
+    const float s0 = sub & 1 ? -1.f : 1.f, s1 = sub & 2 ? -1.f : 1.f, s2 = sub & 4 ? -1.f : 1.f;
 #pragma unroll
     for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -459,7 +455,6 @@ __device__ __forceinline__ void fwht128_lanes(f4_t (&v)[32 / L], int sub) {
             x = x * s0 + sub_xor<0>(x);
             x = x * s1 + sub_xor<1>(x);
             if constexpr (L >= 8) x = x * s2 + sub_xor<2>(x);
-            if constexpr (L >= 16) x = x * s3 + sub_xor<3>(x);
             v[i][j] = x;
         }
 #pragma unroll
