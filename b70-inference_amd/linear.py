@@ -138,7 +138,7 @@ def exl3_gemm(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: torch.Tens
 
 def exl3_gemm_noalloc(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor) -> None:
     """exl3_gemm for up to 8 rows with no allocation in the library (its scratch is a fixed per-device array); same
-    results as exl3_gemm bit for bit. Calls on one device must not overlap in time."""
+    results as exl3_gemm bit for bit, eager or captured. Calls on one device must not overlap in time."""
     require_device(A, B, C, suh, svh)
     K = _K_of(B)
     k, n = B.shape[0] * 16, B.shape[1] * 16

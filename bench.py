@@ -326,7 +326,7 @@ class MoE:
         self.logits = [torch.randn(M, self.E, device="cuda", generator=g) for _ in range(nrout)]
         self.routing = [exl3.route_softmax_topk(lg, topk, bias) for lg in self.logits]
         self.ids = [ids.cpu() for ids, _ in self.routing]
-        # the library's row block with uniform K (0: per-tile K)
+        # the library's row block with uniform K (0: per-tile K), as moe_wide_rows in csrc/exl3_plan.h picks it
         mean, kmax = M * (topk + (1 if shared else 0)) / t.E, max(t.K_gate, t.K_down)
         self.wide = (0 if t.K_gate == 0 or t.K_down == 0 else 32 if M <= 64 or (M <= 160 and mean <= 8) else 64 if 28 < mean <= 64 or kmax > 5 else 128)
         self.exp_bytes = [[weight_bytes(t.projs[q][e]) for q in range(3)] for e in range(t.E)]
