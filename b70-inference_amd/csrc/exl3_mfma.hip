@@ -920,7 +920,7 @@ static int launch_dense_down(const MoeArgs& a, hipStream_t st) {
         if (l.p0 > 0)
             EXL3_LAUNCH("linear_add", linear_add_kernel, dim3((unsigned)((set / 4 + 255) / 256)), dim3(256), 0, st, a.y, l.part,
                         set);
-        if (l.P < P) l.part = a.y + set;
+        if (l.P < P) l.part = reinterpret_cast<float*>(a.xh);
     }
     l.part = a.y;
     if (P > 1)

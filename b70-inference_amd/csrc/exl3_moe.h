@@ -121,9 +121,7 @@ struct MoeArgs {
     const int* cls_list;               // [kRowClasses][max_blocks] block indices by row class
     const int* cls_cnt;                // [kRowClasses] blocks per class
     _Float16* xh;                      // [pairs][2][H] transformed gate / up inputs of MFMA rows; uniform gate|up K:
-                                       // per block [2][cnt * H] in block_unit order (exl3_mfma.h). All uniform: shares
-                                       // its memory with y (a block's rows take the same bytes in both, and its down
-                                       // kernel runs after its gate|up kernel)
+                                       // per block [2][cnt * H] in block_unit order (exl3_mfma.h)
     float* xsum;                       // [pairs][2][H / 128] block sums of xh (the MFMA rows' affine term)
     float* asum;                       // [pairs][I / 128] block sums of abuf (MFMA rows)
     int* pair_tok;
@@ -141,7 +139,8 @@ struct MoeArgs {
                                        // partials)
     int dense_P;                       // > 0: one expert takes every token with weight 1 (a dense MLP) on the MFMA
                                        // path: k-splits of its down projection, which runs as a dense linear
-    int dense_sets;                    // partials held: dense_P, or 2 (a sum and a split): the splits run one after another
+    int dense_sets;                    // partials held: dense_P, or 1: the splits run one after another, the later ones
+                                       // into xh's memory (a set's size; read no more by then), and add up
     float* part_gu;
     int* cnt_gu;
     int P_gu, nblk_h;

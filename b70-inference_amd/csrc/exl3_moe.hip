@@ -1160,12 +1160,11 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     Workspace ws;
     const size_t n_gu = (size_t)max_items * nbI, n_d = (size_t)max_items * nbH;
     const bool use_mfma = a.max_blocks > 0;
-    const bool xy = use_mfma && a.Kg > 0 && a.Kd > 0;           // xh and y share their memory
     size_t y_elems = (size_t)npairs * a.H;
     const auto scratch = [&] {
         return carve_size(1, 4) + carve_size(max_items, sizeof(ItemDesc)) +
                    carve_size(a.max_blocks, sizeof(ItemDesc)) +
-                   (use_mfma ? (xy ? 0 : carve_size(npairs * 2 * a.H, 2)) + carve_size(npairs * 2 * (a.H / 128), 4) +
+                   (use_mfma ? carve_size(npairs * 2 * a.H, 2) + carve_size(npairs * 2 * (a.H / 128), 4) +
                                    carve_size(npairs, 4) +
                                    carve_size(npairs * (a.I / 128), 4) + carve_size(kRowClasses * ((size_t)a.max_blocks + 1), 4)
                              : 0) +
@@ -1175,13 +1174,13 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
                    carve_size(n_gu * a.P_gu * 2 * MR * 128, 4) + carve_size(n_d * a.P_d * MR * 128, 4);
     };
     if (a.dense_P > 0) {
-        // Under stream capture a workspace without room for all splits' partials holds two sets, and the splits run one after
-        // another: the same sums, in the scratch of an unsplit call (whose transformed inputs and outputs take two sets).
+        // Under stream capture a workspace without room for all splits' partials holds one set, and the splits run one after
+        // another through the memory of the transformed inputs: the same sums, in the scratch of an unsplit call.
         a.dense_sets = a.dense_P;
         y_elems = (size_t)a.dense_sets * npairs * a.H;
-        if (a.dense_P > 2 && scratch() > workspace_room(st)) {
-            a.dense_sets = 2;
-            y_elems = (size_t)2 * npairs * a.H;
+        if (a.dense_P > 1 && scratch() > workspace_room(st)) {
+            a.dense_sets = 1;
+            y_elems = (size_t)npairs * a.H;
         }
     }
     const size_t bytes = scratch();
@@ -1194,7 +1193,7 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.items = items;
     ItemDesc* blocks = a.max_blocks ? c.take<ItemDesc>(a.max_blocks) : nullptr;
     a.blocks = blocks;
-    a.xh = use_mfma && !xy ? c.take<_Float16>(npairs * 2 * a.H) : nullptr;
+    a.xh = use_mfma ? c.take<_Float16>(npairs * 2 * a.H) : nullptr;
     a.xsum = use_mfma ? c.take<float>(npairs * 2 * (a.H / 128)) : nullptr;
     a.asum = use_mfma ? c.take<float>(npairs * (a.I / 128)) : nullptr;
     a.pair_e = use_mfma ? c.take<int>(npairs) : nullptr;
@@ -1208,7 +1207,6 @@ int moe_decode_path(MoeArgs a, int64_t npairs, hipStream_t st) {
     a.tok_nvalid = c.take<int>(a.M);
     a.abuf = c.take<uint16_t>(npairs * a.I);
     a.y = c.take<float>(y_elems);
-    if (xy) a.xh = reinterpret_cast<_Float16*>(a.y);
     a.part_gu = c.take<float>(n_gu * a.P_gu * 2 * MR * 128);
     a.part_d = c.take<float>(n_d * a.P_d * MR * 128);
     if (!a.part_d) return fail(EXL3_ERR_INVALID, "moe: workspace carve failed");

@@ -166,8 +166,8 @@ def test_no_spilling_row_block(lib, K, rg):
 
 @pytest.mark.parametrize("M,H,I", [(40, 8192, 2048), (300, 1024, 2048)])
 def test_dense_mlp_capture_shapes_have_many_splits(lib, M, H, I):
-    """The shapes of test_dense_mlp_captured_in_the_scratch_of_an_unsplit_call run their splits one after another: more of them
-    than the two sets of partials that the workspace holds."""
+    """The shapes of test_dense_mlp_captured_in_the_scratch_of_an_unsplit_call have several splits, more than the one set of
+    partials that its workspace holds."""
     rows = lib.moe_rows(M, 1, M, H, I, 3, 3, 0)
     assert plan(lib, M, H, I, 3, rows // 32, 8)[1] > 2
 

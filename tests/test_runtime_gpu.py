@@ -251,7 +251,7 @@ def test_few_rows_captured_in_the_gemv_scratch(exl3, oracle, fresh, k, n, M):
 @pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
 @pytest.mark.parametrize("M,H,I", [(40, 8192, 2048), (300, 1024, 2048)])
 def test_dense_mlp_captured_in_the_scratch_of_an_unsplit_call(exl3, oracle, fresh, monkeypatch, M, H, I):
-    """A dense MLP's k-split down projection captured where the workspace holds two sets of partials only (a set is more than
+    """A dense MLP's k-split down projection captured where the workspace holds one set of partials only (a set is more than
     the MiB to spare): the splits run one after another and give the eager call's bits."""
     lib = fresh
     tables, orc = make_experts(exl3, oracle, 1, H, I, 3, 3, 4400)
