@@ -1393,6 +1393,8 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
         moe_expected_items(a, 64) >= 48.0)
         mfma = true;
     if (env_int("EXL3MI_MOE_MFMA", 0)) mfma = true;
+    const bool wide = a.Kg > 0 && a.Kd > 0;
+    if (wide && !a_span_ok(npairs < 32 ? npairs : 32, a.H > a.I ? a.H : a.I)) mfma = false;   // no block's A would fit
     a.MR = mfma ? 0 : M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : kMoeSmallRows;
     // rows per GEMV item: one for sparse routing (pairs <= E / 2; experts of 2048 -> 512, 8 tokens, against eight rows
     // per item: 512 experts top-17 170.6 -> 86.6 us), two up to 1.5 pairs per expert (128 experts top-17 78.7 against
@@ -1421,7 +1423,6 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     int64_t mi = mfma ? 0 : E + npairs / a.MR;
     if (mi > npairs) mi = npairs;
     a.max_items = (int)mi;
-    const bool wide = a.Kg > 0 && a.Kd > 0;
     a.block_rows = wide ? moe_wide_rows(M, E, npairs, a.H, a.I, a.Kg, a.Kd, env_int("EXL3MI_MOE_BLOCK", 0)) : kMfmaRows;
     if (mfma && wide && E == 1 && a.topk == 0 && a.shared == 0) {          // a dense MLP: its down projection as a dense linear
         const int rc = dense_down_splits(M, a.H, a.I, a.Kd, a.block_rows, 8, &a.dense_P);
@@ -1431,8 +1432,6 @@ static int moe_run(MoeArgs& a, hipStream_t st) {
     EXL3_CHECK_ARG((int64_t)a.max_items * (a.H / 128) < 0x7FFFFFFF && a.max_blocks <= (wide ? 1 << 21 : 65535) &&
                        (int64_t)(a.max_blocks + 8) * (a.I > a.H ? a.I / 128 : a.H / 128) < 0x7FFFFFFF,
                    "exl3_moe_forward: grid too large");
-    EXL3_CHECK_ARG(!mfma || !wide || a_span_ok(npairs < a.block_rows ? npairs : a.block_rows, a.H > a.I ? a.H : a.I),
-                   "exl3_moe_forward: H=%d or I=%d too large", a.H, a.I);
     return moe_decode_path(a, npairs, st);
 }
 
